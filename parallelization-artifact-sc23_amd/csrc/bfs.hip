@@ -95,7 +95,8 @@ IG_DEV void top_down(const BfsArgs& a, int L, const FrontierCounters& ic, const 
   };
   expand_huge(in, huge_count(ic.hpack), huge_chunks(ic.hpack), a.nindex, visit);
   expand_mid(in, ic.nm, a.nindex, visit);
-  expand_small(in.q, ic.n, a.nindex, visit);
+  const unsigned avg = ic.nm == 0 && ic.hpack == 0 ? static_cast<unsigned>(ic.m / ic.n) : 16u;
+  expand_small(in.q, ic.n, a.nindex, visit, small_share(ic.n, avg));
 }
 
 IG_DEV void bottom_up(const BfsArgs& a, int L, unsigned heavy_mid, unsigned heavy_huge, const FrontierQueues& out,
@@ -294,7 +295,7 @@ IG_DEV int small_phase(const BfsArgs& a, int L, unsigned n, BfsControl* ctl, lon
   return L;
 }
 
-__global__ __launch_bounds__(kBfsBlock) void bfs_kernel(BfsArgs a)
+__global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void bfs_kernel(BfsArgs a)
 {
   // the set-up's heavy-list collection needs a larger mid buffer than the
   // level emitter (no spills to the global counter); they share the LDS

@@ -254,31 +254,58 @@ IG_DEV void expand_huge(const FrontierQueues& in, unsigned nh, unsigned nch, con
   }
 }
 
-// Mid lists: one wave per vertex.
+// Mid lists: one wave each, or, while there are few of them, k waves each (k
+// up to 16, while 2 * k waves per list still fit the grid), wave j of a list
+// taking its windows j, j + k, ...  Each window is a chain of device-scope
+// round trips (the neighbour's check, its claim or atomicMin, its degree), so a
+// 4000-entry list walked by one wave set a level's length: BFS's level of 997
+// lists and 3.6M entries on R-MAT 22 took 198 us (calls 0.65 -> 0.53 ms).
 template <typename F>
 IG_DEV void expand_mid(const FrontierQueues& in, unsigned nm, const int* __restrict__ nindex, F&& f)
 {
   const int lane = lane_id();
-  const int wpb = blockDim.x / kWave;
-  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nm; i += gridDim.x * wpb) {
-    const int v = ld_relaxed(&in.mq[i]);
+  const unsigned wpb = blockDim.x / kWave;
+  const unsigned nwaves = gridDim.x * wpb;
+  unsigned k = 1;
+  while (k < 16 && static_cast<unsigned long long>(nm) * k * 2 <= nwaves) k *= 2;
+  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nm * k; i += nwaves) {
+    const int v = ld_relaxed(&in.mq[i / k]);
     const int beg = nindex[v], end = nindex[v + 1];
-    for (int base = beg; base < end; base += kWave) {
+    for (int base = beg + static_cast<int>(i % k) * kWave; base < end; base += static_cast<int>(k) * kWave) {
       const int e = base + lane;
       f(v, e, e < end);
     }
   }
 }
 
-// Small lists: 64 vertices per wave, 64 CSR entries per step.
-template <typename F>
-IG_DEV void expand_small(const int* __restrict__ q, unsigned n, const int* __restrict__ nindex, F&& f)
+// Vertices per wave of an expand_small pass over n small-queue vertices of
+// average list length `avg`: 64 when they fill the grid's waves, else fewer,
+// down to about one 64-entry window per wave.  A wave's windows are serial
+// chains of round trips (2 to 3 us each), so 64 vertices of 16 entries on one
+// wave made a narrow level 30 to 50 us long while most waves had nothing to
+// do; below one window per wave, more workgroups only means more
+// same-address appends at the flush.  SSSP calls on R-MAT 12 and 16 0.65 and
+// 0.87 -> 0.29 and 0.70 ms, random 2^20 (degree 16) 2.28 -> 1.27, 1024^2 and
+// 2048^2 roads 29.8 and 74.2 -> 20.7 and 48.6; BFS on the 2048^2 road 40.3 ->
+// 28.4 ms, random 2^20 0.36 -> 0.28.
+IG_DEV unsigned small_share(unsigned n, unsigned avg)
 {
-  const int lane = lane_id();
-  const int wpb = blockDim.x / kWave;
-  for (unsigned c = blockIdx.x * wpb + threadIdx.x / kWave; c * kWave < n; c += gridDim.x * wpb) {
-    const unsigned idx = c * kWave + lane;
-    const bool valid = idx < n;
+  const unsigned nwaves = gridDim.x * (blockDim.x / kWave);
+  unsigned per = kWave;
+  while (per > 1 && per * avg > kWave && (n + per / 2 - 1) / (per / 2) <= nwaves) per /= 2;
+  return per;
+}
+
+// Small lists: `per` (at most 64) vertices per wave, 64 CSR entries per step.
+template <typename F>
+IG_DEV void expand_small(const int* __restrict__ q, unsigned n, const int* __restrict__ nindex, F&& f,
+                         unsigned per = kWave)
+{
+  const unsigned lane = lane_id();
+  const unsigned wpb = blockDim.x / kWave;
+  for (unsigned c = blockIdx.x * wpb + threadIdx.x / kWave; c * per < n; c += gridDim.x * wpb) {
+    const unsigned idx = c * per + lane;
+    const bool valid = lane < per && idx < n;
     const int v = valid ? ld_relaxed(&q[idx]) : 0;
     const int beg = valid ? nindex[v] : 0;
     const int deg = valid ? nindex[v + 1] - beg : 0;

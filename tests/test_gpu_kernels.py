@@ -78,6 +78,28 @@ def test_sssp_few_mid_lists(ig, orc, ctx):
     assert np.array_equal(ctx.bfs(dg, 0), orc.bfs(g, 0))
 
 
+@pytest.mark.parametrize("leaves", [0, 1, 3, 15, 16, 62])
+@pytest.mark.parametrize("mids", [1, 63, 64, 65, 767, 6145])
+def test_short_list_levels(ig, orc, ctx, mids, leaves):
+    """A source joined to `mids` vertices of `leaves` leaves each (lists of up
+    to 63 entries): levels of few or many short lists, which a grid pass
+    hands out 1 to 64 to a wave.  The one-workgroup phase is off, so that
+    every level is a grid pass."""
+    n = 1 + mids * (1 + leaves)
+    m = np.arange(1, 1 + mids)
+    src = np.concatenate([np.zeros(mids, np.int64), np.repeat(m, leaves)])
+    dst = np.concatenate([m, np.arange(1 + mids, n)])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32), wseed=9, wmin=1, wmax=300)
+    dg = ig.DeviceGraph(g)
+    ctx.set_hint(ig._lib.HINT_SMALL_FRONTIER, 1)
+    try:
+        for s in (0, n - 1):
+            assert np.array_equal(ctx.bfs(dg, s), orc.bfs(g, s)), s
+            assert np.array_equal(ctx.sssp(dg, s), orc.sssp(g, s)), s
+    finally:
+        ctx.set_hint(ig._lib.HINT_SMALL_FRONTIER, 0)
+
+
 def test_cc_catalog(ig, orc, ctx):
     for g in catalog(ig):
         assert np.array_equal(ctx.cc(ig.DeviceGraph(g)), orc.cc(g)), g.name
