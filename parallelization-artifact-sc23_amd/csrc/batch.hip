@@ -10,7 +10,8 @@
 // Gangs.  A task runs on a gang of k workgroups, k = the task's CSR entries
 // / 2^18 rounded up to a power of two: small graphs take one workgroup and
 // synchronise with __syncthreads only, large ones a gang with its own bounded
-// barrier.  The cap depends on how much work a barrier separates: 256 for
+// barrier.  Where that leaves workgroups of the grid without a task, the tasks
+// that would finish last take them (widen_gangs).  The cap depends on how much work a barrier separates: 256 for
 // the dense sweeps of PR, CC and MIS, 128 for BFS, 64 for SSSP's many short
 // rounds, and 16 for BFS on deep sparse graphs (average degree below 6),
 // whose thousands of levels are bound by barrier latency.  A free workgroup joins the first task in queue
@@ -74,6 +75,8 @@
 #include <algorithm>
 #include <climits>
 #include <cstring>
+#include <queue>
+#include <utility>
 #include <vector>
 
 #include "csum.hpp"
@@ -87,6 +90,7 @@ constexpr int kBatchBlock = 512;
 constexpr int kBatchWaves = kBatchBlock / kWave;
 constexpr int kMaxGang = INDIGO_MAX_GANG;
 constexpr int kGangShift = 18;   // CSR entries per gang member
+constexpr int kWidenEntries = 4096;  // CSR entries per member of a widened gang (widen_floor)
 constexpr int kHeavyDeg = 1024;  // lists this long are split into items
 constexpr int kItem = 1024;      // entries per item
 constexpr int kCcSample = 2;      // CC: neighbours linked per vertex before the giant root is chosen
@@ -911,15 +915,19 @@ size_t scratch_bytes(int alg, int nodes, int edges)
 
 }  // namespace
 
+// Largest gang of an algorithm: how much work one of its barriers separates.
+static int gang_cap(int alg, int nodes, int edges)
+{
+  if (alg == INDIGO_QUERY_SSSP) return 64;
+  if (alg != INDIGO_QUERY_BFS) return kMaxGang;
+  return static_cast<long long>(edges) < 6LL * nodes ? 16 : 128;
+}
+
 int batch_gang(int alg, int nodes, int edges)
 {
   if (alg < INDIGO_QUERY_BFS || alg > INDIGO_QUERY_PR || nodes < 0 || edges < 0) return 0;
   const long long entries = static_cast<long long>(edges) + nodes;
-  int cap = kMaxGang;
-  if (alg == INDIGO_QUERY_BFS || alg == INDIGO_QUERY_SSSP) {
-    cap = alg == INDIGO_QUERY_BFS ? 128 : 64;
-    if (alg == INDIGO_QUERY_BFS && static_cast<long long>(edges) < 6LL * nodes) cap = 16;
-  }
+  const int cap = gang_cap(alg, nodes, edges);
   int k = 1;
   while (k < cap && (static_cast<long long>(k) << kGangShift) < entries) k <<= 1;
   return k;
@@ -928,6 +936,68 @@ int batch_gang(int alg, int nodes, int edges)
 namespace {
 
 int gang_for(int alg, int nodes, int edges, int grid) { return std::min(batch_gang(alg, nodes, edges), std::max(1, grid)); }
+
+// Estimated nanoseconds of one query on one workgroup, fitted to batches of
+// one query on graphs of 2^10 to 2^18 entries.
+double query_cost(const indigo_query& Q, const indigo_graph_ref& G)
+{
+  const double entries = static_cast<double>(G.edges) + G.nodes;
+  switch (Q.alg) {
+    case INDIGO_QUERY_BFS: return entries * 16;
+    case INDIGO_QUERY_SSSP: return entries * 7 * Q.nsrc;
+    case INDIGO_QUERY_PR: return entries * 35;
+    case INDIGO_QUERY_MIS: return entries * 9;
+    default: return entries * 5;
+  }
+}
+
+// Fewest CSR entries per member of a widened gang.  On sparse graphs a BFS or
+// SSSP of few sources has levels too narrow to pay a gang barrier for (one BFS
+// on a 64^2 grid 0.74 ms on one workgroup, 0.90 on four; 64 at once 4.5 and
+// 1.9): the floor is 16 / nsrc times as high for BFS below 16 sources, four
+// times for SSSP below 4.
+long long widen_floor(const indigo_query& Q, const indigo_graph_ref& G)
+{
+  if (G.edges < 6LL * G.nodes) {
+    if (Q.alg == INDIGO_QUERY_BFS && Q.nsrc < 16) return kWidenEntries * 16 / Q.nsrc;
+    if (Q.alg == INDIGO_QUERY_SSSP && Q.nsrc < 4) return kWidenEntries * 4;
+  }
+  return kWidenEntries;
+}
+
+// A batch whose gangs leave workgroups of the grid without a task: the task
+// that would finish last (largest cost per member) doubles its gang, while
+// the free workgroups last and its members keep widen_floor entries each
+// (and the algorithm's bound on gangs holds).  Gangs that a caller chose stay.
+// With gangs of 2^18 entries per member alone, a batch was as long as its
+// largest task on a workgroup or two (SSSP of 16 sources on 10^5 vertices: 20
+// to 30 ms) while most of the grid idled.  Batches of 24, 12, 6 and 2 graphs of
+// 2^10 to 2^17 vertices, five algorithms each: 52.6, 69.5, 27.6 and 22.9 ->
+// 15.2, 11.8, 10.8 and 5.0 ms; floors of 1024 and 2048 entries per member
+// measured the same within 12%, 16384 up to 23% slower.
+void widen_gangs(std::vector<int>& gang, const indigo_graph_ref* graphs, const indigo_query* queries, int grid)
+{
+  long long used = 0;
+  for (int k : gang) used += k;
+  if (used >= grid) return;
+  using Entry = std::pair<double, int>;  // cost per member, query
+  std::priority_queue<Entry> heap;
+  for (size_t q = 0; q < gang.size(); q++)
+    if (queries[q].gang == 0) heap.push({query_cost(queries[q], graphs[queries[q].graph]) / gang[q], static_cast<int>(q)});
+  while (!heap.empty()) {
+    const Entry top = heap.top();
+    heap.pop();
+    const int q = top.second;
+    const indigo_graph_ref& G = graphs[queries[q].graph];
+    const long long entries = static_cast<long long>(G.edges) + G.nodes;
+    const int k = gang[q];
+    if (2 * k > gang_cap(queries[q].alg, G.nodes, G.edges) || entries / (2 * k) < widen_floor(queries[q], G)) continue;
+    if (used + k > grid) continue;
+    gang[q] = 2 * k;
+    used += k;
+    heap.push({top.first / 2, q});
+  }
+}
 
 }  // namespace
 
@@ -1016,6 +1086,13 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
     work[q] = static_cast<long long>(G.edges) + G.nodes;
   }
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work[a] > work[b]; });
+  std::vector<int> gang(static_cast<size_t>(nqueries));
+  for (int q = 0; q < nqueries; q++) {
+    const indigo_graph_ref& G = graphs[queries[q].graph];
+    gang[q] = queries[q].gang > 0 ? std::min(queries[q].gang, grid_cap)
+                                  : gang_for(queries[q].alg, G.nodes, G.edges, grid_cap);
+  }
+  widen_gangs(gang, graphs, queries, grid_cap);
   size_t scratch_total = 0;
   for (int q = 0; q < nqueries; q++)
     scratch_total += scratch_bytes(queries[q].alg, graphs[queries[q].graph].nodes, graphs[queries[q].graph].edges);
@@ -1037,7 +1114,7 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
     BatchTask& T = h_tasks[i];
     std::memset(&T, 0, sizeof(T));
     T.alg = Q.alg;
-    T.gang = Q.gang > 0 ? std::min(Q.gang, grid_cap) : gang_for(Q.alg, G.nodes, G.edges, grid_cap);
+    T.gang = gang[order[i]];
     T.nodes = G.nodes;
     T.edges = G.edges;
     T.nindex = G.d_nindex;

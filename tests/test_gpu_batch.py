@@ -93,6 +93,30 @@ def test_batch_capped_grid(ig, ctx, cap):
     _check_against_plain(ctx, gs, dgs, qs)
 
 
+@pytest.mark.parametrize("nodes", [1364, 1366, 5461, 5464, 43691])
+@pytest.mark.parametrize("cap", [0, 5, 64])
+def test_batch_idle_grid(ig, orc, ctx, nodes, cap):
+    """A batch of one small graph (just below and above 8192 and 32768
+    entries and vertices, and a larger one) leaves most of the grid without a
+    task: gangs of 2 to 64 where 2^18 entries per member would take one."""
+    from test_gpu_kernels import _pr_check
+
+    g = ig.erdos_renyi(nodes, nodes * 5 // 2, seed=nodes, wmin=1, wmax=255)
+    dg = ig.DeviceGraph(g)
+    rng = np.random.default_rng(nodes)
+    qs = [ig.Query("bfs", 0, dg, rng.integers(0, nodes, 17)), ig.Query("bfs", 0, dg, [1]),
+          ig.Query("sssp", 0, dg, rng.integers(0, nodes, 4)), ig.Query("sssp", 0, dg, [2]),
+          ig.Query("cc", 0, dg), ig.Query("mis", 0, dg)]
+    pr = ig.Query("pr", 0, dg)
+    for some in ([q] for q in qs):
+        ctx.batch([dg], some, max_workgroups=cap)
+    ctx.batch([dg], [pr], max_workgroups=cap)
+    _check_against_plain(ctx, [g], [dg], qs)
+    _pr_check(ig, orc, g, *pr.result())
+    ctx.batch([dg], qs, max_workgroups=cap)
+    _check_against_plain(ctx, [g], [dg], qs)
+
+
 def test_batch_rejects_bad_queries(ig, ctx):
     g = ig.grid(4, 4)
     dg = ig.DeviceGraph(g)
