@@ -134,16 +134,18 @@ IG_DEV void relax(const SsspArgs& a, int dv, int e, bool active, int T, int it_s
     // device-scope read: a plain load may see a stale L2 copy of a distance
     // another XCD has lowered, and let a useless atomic through
     if (nd < ld_relaxed(&a.dist[u])) {
-      const int old = atomic_min_relaxed(&a.dist[u], nd);
-      if (nd < old) {
-        udeg = degree_of(a.nindex, u);
-        if (udeg > 0) {
-          if (nd < T)
-            near = __hip_atomic_exchange(&a.stamp[u], it_stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != it_stamp;
-          else
-            park = __hip_atomic_exchange(&a.farstamp[u], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch;
-        }
-      }
+      // the minimum, the dedup exchange and the degree leave together: a
+      // lane whose check passed may join u whether or not its own atomicMin
+      // was the one that lowered dist[u] - someone did, in this iteration
+      const bool below = nd < T;
+      atomic_min_relaxed(&a.dist[u], nd);
+      int* mark = below ? &a.stamp[u] : &a.farstamp[u];
+      const int tag = below ? it_stamp : epoch;
+      const int seen = __hip_atomic_exchange(mark, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      udeg = degree_of(a.nindex, u);
+      const bool join = seen != tag && udeg > 0;
+      near = join && below;
+      park = join && !below;
     }
   }
   frontier_emit_block(S.near, near, u, udeg, out, oc);
