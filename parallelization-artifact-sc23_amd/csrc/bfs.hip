@@ -99,8 +99,8 @@ IG_DEV void top_down(const BfsArgs& a, int L, const FrontierCounters& ic, const 
   expand_small(in.q, ic.n, a.nindex, visit, small_share(ic.n, avg));
 }
 
-IG_DEV void bottom_up(const BfsArgs& a, int L, unsigned heavy_mid, unsigned heavy_huge, const FrontierQueues& out,
-                      FrontierCounters* oc, FrontierEmitter& E)
+IG_DEV void bottom_up(const BfsArgs& a, int L, unsigned nheavy, const FrontierQueues& out, FrontierCounters* oc,
+                      FrontierEmitter& E)
 {
   const int next = L + 1;
   const int lane = lane_id();
@@ -127,9 +127,8 @@ IG_DEV void bottom_up(const BfsArgs& a, int L, unsigned heavy_mid, unsigned heav
   }
   // long lists: one wave per vertex, 64 entries per ballot
   const int wpb = blockDim.x / kWave;
-  const unsigned total = heavy_mid + heavy_huge;
-  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < total; i += gridDim.x * wpb) {
-    const int v = i < heavy_mid ? ld_relaxed(&a.heavy.mq[i]) : ld_relaxed(&a.heavy.hq[i - heavy_mid]);
+  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nheavy; i += gridDim.x * wpb) {
+    const int v = ld_relaxed(&a.heavy.mq[i]);
     if (ld_relaxed(&a.dist[v]) != kInf) continue;
     const int beg = a.nindex[v], end = a.nindex[v + 1];
     bool found = false;
@@ -312,7 +311,7 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
   const int stride = gridDim.x * blockDim.x;
   if (tid == 0) ctl->trace.start = now_ticks();
   for (int i = tid; i < a.nodes; i += stride) st_relaxed(&a.dist[i], (i == a.src) ? 0 : kInf);
-  if (a.allow_bu) collect_heavy(s_lds.collect, a.nodes, a.nindex, a.heavy, &ctl->heavy);
+  if (a.allow_bu) collect_heavy<kMidDeg, INT_MAX, kHugeChunk>(s_lds.collect, a.nodes, a.nindex, a.heavy, &ctl->heavy);
   if (blockIdx.x == 0 && threadIdx.x < kWave) {
     const int deg = degree_of(a.nindex, a.src);
     frontier_emit(threadIdx.x == 0 && deg > 0, a.src, deg, a.fq[0], &ctl->cnt[0]);
@@ -321,8 +320,7 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
     if (tid == 0) ctl->status = 1;
     return;
   }
-  const unsigned heavy_mid = ld_relaxed(&ctl->heavy.nm);
-  const unsigned heavy_huge = huge_count(ld_relaxed(&ctl->heavy.hpack));
+  const unsigned nheavy = ld_relaxed(&ctl->heavy.nm);
   bool bu = false;
   unsigned long long seen_edges = 0;
   int bu_levels = 0;
@@ -375,7 +373,7 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
     FrontierCounters* oc = &ctl->cnt[(L + 1) % 3];
     fe_reset(s_emit);
     if (bu) {
-      bottom_up(a, L, heavy_mid, heavy_huge, out, oc, s_emit);
+      bottom_up(a, L, nheavy, out, oc, s_emit);
       bu_levels++;
     } else {
       top_down(a, L, ic, in, out, oc, s_emit);

@@ -8,13 +8,17 @@
 //   * small: length < kMidDeg.  Expanded 64 vertices per wave with an in-wave
 //     load balancer (prefix sum of lengths + owner search), so a wave always
 //     handles 64 consecutive CSR entries and never more than 64 * 63 in all;
-//   * mid:   kMidDeg <= length < kHugeDeg.  One wave per vertex, lanes
-//     striding its list (coalesced);
-//   * huge:  length >= kHugeDeg.  Split into kHugeChunk-entry work items
-//     spread over all workgroups.  Its counter packs (chunk count << 32 |
-//     vertex count) so one 64-bit atomic allocates both the slot and the
-//     vertex's first chunk index; hoff[] is therefore sorted by slot and a
-//     chunk's owner is found by binary search.
+//   * mid:   kMidDeg <= length < kHugeDeg.  One wave per vertex (several
+//     while there are few), lanes striding its list (coalesced);
+//   * huge:  length >= kHugeDeg.  Split into kHugeChunk-entry work items, one
+//     wave each.  Its counter packs (chunk count << 32 | vertex count) so one
+//     64-bit atomic allocates both the slots and the vertices' first chunk
+//     indices; hoff[] is therefore sorted by slot and a wave finds a chunk's
+//     owner by a 64-way search.
+// kHugeDeg bounds a wave's serial chain to 8 windows of about 3 us.  With lists
+// of up to 4095 entries on one wave (and longer ones in 2048-entry workgroup
+// items), the longest list set an iteration: SSSP on R-MAT 22, 20, 18 and 16
+// took 4.95, 2.11, 0.91 and 0.66 ms, now 4.09, 1.43, 0.76 and 0.50.
 // Appends are wave-aggregated (ballot + mbcnt prefix, one atomic per wave and
 // queue).  Counters are triple-buffered across levels so that the set written
 // in level L, read in L+1 and cleared in L+2 never has two roles at once.
@@ -30,8 +34,8 @@
 namespace indigo {
 
 constexpr int kMidDeg = 64;
-constexpr int kHugeDeg = 4096;
-constexpr int kHugeChunk = 2048;
+constexpr int kHugeDeg = 512;
+constexpr int kHugeChunk = 512;
 
 struct alignas(128) FrontierCounters {
   unsigned int n;            // small queue length
@@ -98,100 +102,144 @@ IG_DEV FrontierCounters counters_load(const FrontierCounters* c)
   return r;
 }
 
+// First chunk indices of a wave's huge vertices, appended straight to the global
+// queue with one atomic (all lanes converged).
+template <int kChunk>
+IG_DEV void huge_append(bool huge, int u, int deg, const FrontierQueues& fq, FrontierCounters* c)
+{
+  const unsigned long long hm = __ballot(huge);
+  if (hm == 0) return;
+  const int chunks = huge ? (deg + kChunk - 1) / kChunk : 0;
+  const int incl = wave_inclusive_scan(chunks);
+  const int total = wave_shfl(incl, kWave - 1);
+  const int leader = __ffsll(static_cast<long long>(hm)) - 1;
+  unsigned long long old = 0;
+  if (lane_id() == leader)
+    old = atomic_add_relaxed(&c->hpack, (static_cast<unsigned long long>(total) << 32) | __popcll(hm));
+  old = wave_shfl(old, leader);
+  if (huge) {
+    const unsigned slot = static_cast<unsigned>(old & 0xffffffffull) + lanes_below(hm);
+    st_relaxed(&fq.hq[slot], u);
+    st_relaxed(&fq.hoff[slot], static_cast<unsigned>(old >> 32) + static_cast<unsigned>(incl - chunks));
+  }
+}
+
 // Wave-collective: every active lane with `pred` appends vertex u (whose list
 // has deg entries) to the frontier `fq`/`c`.  All 64 lanes must be converged.
-// kMid is the list length from which a vertex goes to the mid queue.
-template <int kMid = kMidDeg>
 IG_DEV void frontier_emit(bool pred, int u, int deg, const FrontierQueues& fq, FrontierCounters* c)
 {
   const bool huge = pred && deg >= kHugeDeg;
-  const bool mid = pred && deg >= kMid && !huge;
-  const bool small = pred && deg < kMid;
+  const bool mid = pred && deg >= kMidDeg && !huge;
+  const bool small = pred && deg < kMidDeg;
   const unsigned long long dsum = wave_sum(static_cast<unsigned long long>(pred ? deg : 0));
   if (lane_id() == 0 && dsum != 0) atomic_add_relaxed(&c->m, dsum);
   wave_append(small, u, fq.q, &c->n);
   wave_append(mid, u, fq.mq, &c->nm);
-  const unsigned long long hm = __ballot(huge);
-  if (hm != 0) {
-    const int chunks = huge ? (deg + kHugeChunk - 1) / kHugeChunk : 0;
-    const int incl = wave_inclusive_scan(chunks);
-    const int total = wave_shfl(incl, kWave - 1);
-    const int leader = __ffsll(static_cast<long long>(hm)) - 1;
-    unsigned long long old = 0;
-    if (lane_id() == leader)
-      old = atomic_add_relaxed(&c->hpack, (static_cast<unsigned long long>(total) << 32) | __popcll(hm));
-    old = wave_shfl(old, leader);
-    if (huge) {
-      const unsigned slot = static_cast<unsigned>(old & 0xffffffffull) + lanes_below(hm);
-      st_relaxed(&fq.hq[slot], u);
-      st_relaxed(&fq.hoff[slot], static_cast<unsigned>(old >> 32) + static_cast<unsigned>(incl - chunks));
-    }
-  }
+  huge_append<kHugeChunk>(huge, u, deg, fq, c);
 }
 
-// Workgroup-aggregated version of frontier_emit (see emit.hpp): small and mid
-// appends and the degree sum are buffered in LDS and flushed with one atomic
-// per queue by fe_flush; huge entries (rare) still go straight to global.
+// Workgroup-aggregated version of frontier_emit (see emit.hpp): appends and the
+// degree sum are buffered in LDS and flushed with one atomic per queue by
+// fe_flush.  A huge entry takes its slot and its first chunk index from one
+// 64-bit LDS atomic, so both stay sorted; entries beyond kHugeCap go straight to
+// the global queue.
 constexpr int kEmitSmallCap = 4096;
 constexpr int kEmitMidCap = 512;
+constexpr int kEmitHugeCap = 256;
 
-template <int kSmallCap, int kMidCap>
+template <int kSmallCap, int kMidCap, int kHugeCap>
 struct FrontierEmitterT {
   BlockQueue<kSmallCap> small;
   BlockQueue<kMidCap> mid;
   BlockSum m;
+  unsigned long long hpack;  // (chunks << 32) | buffered huge entries
+  unsigned long long hbase;  // the same of the global queue before this workgroup's
+  int hu[kHugeCap];
+  unsigned hchunk[kHugeCap];
 };
-using FrontierEmitter = FrontierEmitterT<kEmitSmallCap, kEmitMidCap>;
+using FrontierEmitter = FrontierEmitterT<kEmitSmallCap, kEmitMidCap, kEmitHugeCap>;
 // For collect_heavy over a whole graph with a low threshold: no small queue,
 // room for a workgroup's whole share of mid lists (an append beyond the
 // buffer costs a same-address global atomic, about 10 ns each, serialised).
-using HeavyCollector = FrontierEmitterT<64, 2048>;
+using HeavyCollector = FrontierEmitterT<64, 2048, 64>;
 
 // Workgroup-collective.
-template <int S, int M>
-IG_DEV void fe_reset(FrontierEmitterT<S, M>& E)
+template <int S, int M, int H>
+IG_DEV void fe_reset(FrontierEmitterT<S, M, H>& E)
 {
   if (threadIdx.x == 0) {
     E.small.count = 0;
     E.mid.count = 0;
     E.m.v = 0ull;
+    E.hpack = 0ull;
   }
   __syncthreads();
 }
 
-// Wave-collective.
-template <int kMid = kMidDeg, int S, int M>
-IG_DEV void frontier_emit_block(FrontierEmitterT<S, M>& E, bool pred, int u, int deg, const FrontierQueues& fq,
+// Wave-collective.  kMid and kHuge are the list lengths from which a vertex
+// goes to the mid and the huge queue, kChunk the entries per huge chunk.
+template <int kMid = kMidDeg, int kHuge = kHugeDeg, int kChunk = kHugeChunk, int S, int M, int H>
+IG_DEV void frontier_emit_block(FrontierEmitterT<S, M, H>& E, bool pred, int u, int deg, const FrontierQueues& fq,
                                 FrontierCounters* c)
 {
-  const bool huge = pred && deg >= kHugeDeg;
+  if (__ballot(pred) == 0ull) return;
+  const bool huge = pred && deg >= kHuge;
   const bool mid = pred && deg >= kMid && !huge;
   const bool small = pred && deg < kMid;
   bs_add(E.m, static_cast<unsigned long long>(pred ? deg : 0));
   bq_append(E.small, small, u, fq.q, &c->n);
   bq_append(E.mid, mid, u, fq.mq, &c->nm);
   const unsigned long long hm = __ballot(huge);
-  if (hm != 0) {
-    const int chunks = huge ? (deg + kHugeChunk - 1) / kHugeChunk : 0;
-    const int incl = wave_inclusive_scan(chunks);
-    const int total = wave_shfl(incl, kWave - 1);
-    const int leader = __ffsll(static_cast<long long>(hm)) - 1;
-    unsigned long long old = 0;
-    if (lane_id() == leader)
-      old = atomic_add_relaxed(&c->hpack, (static_cast<unsigned long long>(total) << 32) | __popcll(hm));
-    old = wave_shfl(old, leader);
-    if (huge) {
-      const unsigned slot = static_cast<unsigned>(old & 0xffffffffull) + lanes_below(hm);
-      st_relaxed(&fq.hq[slot], u);
-      st_relaxed(&fq.hoff[slot], static_cast<unsigned>(old >> 32) + static_cast<unsigned>(incl - chunks));
+  if (hm == 0) return;
+  const int chunks = huge ? (deg + kChunk - 1) / kChunk : 0;
+  const int incl = wave_inclusive_scan(chunks);
+  const int total = wave_bcast(incl, kWave - 1);
+  const int pop = __popcll(hm);
+  const int leader = __ffsll(static_cast<long long>(hm)) - 1;
+  unsigned long long old = 0;
+  int room = 0;
+  if (lane_id() == leader) {
+    // taken only while the whole batch fits, so that the buffered entries
+    // are a gapless prefix
+    old = E.hpack;
+    for (;;) {
+      room = static_cast<int>(old & 0xffffffffull) + pop <= H;
+      if (!room) break;
+      const unsigned long long got =
+          atomicCAS(&E.hpack, old, old + ((static_cast<unsigned long long>(total) << 32) | static_cast<unsigned>(pop)));
+      if (got == old) break;
+      old = got;
     }
+  }
+  room = wave_shfl(room, leader);
+  if (room == 0) {
+    huge_append<kChunk>(huge, u, deg, fq, c);
+    return;
+  }
+  old = wave_shfl(old, leader);
+  if (huge) {
+    const int slot = static_cast<int>(old & 0xffffffffull) + lanes_below(hm);
+    E.hu[slot] = u;
+    E.hchunk[slot] = static_cast<unsigned>(old >> 32) + static_cast<unsigned>(incl - chunks);
   }
 }
 
 // Workgroup-collective.
-template <int S, int M>
-IG_DEV void fe_flush(FrontierEmitterT<S, M>& E, const FrontierQueues& fq, FrontierCounters* c)
+template <int S, int M, int H>
+IG_DEV void fe_flush(FrontierEmitterT<S, M, H>& E, const FrontierQueues& fq, FrontierCounters* c)
 {
+  __syncthreads();
+  const int nh = static_cast<int>(E.hpack & 0xffffffffull);
+  if (nh > 0) {
+    if (threadIdx.x == 0) E.hbase = atomic_add_relaxed(&c->hpack, E.hpack);
+    __syncthreads();
+    const unsigned slot0 = static_cast<unsigned>(E.hbase & 0xffffffffull);
+    const unsigned chunk0 = static_cast<unsigned>(E.hbase >> 32);
+    for (int i = threadIdx.x; i < nh; i += blockDim.x) {
+      st_relaxed(&fq.hq[slot0 + i], E.hu[i]);
+      st_relaxed(&fq.hoff[slot0 + i], chunk0 + E.hchunk[i]);
+    }
+  }
   bq_flush(E.small, fq.q, &c->n);
   bq_flush(E.mid, fq.mq, &c->nm);
   if (threadIdx.x == 0 && E.m.v != 0ull) atomic_add_relaxed(&c->m, E.m.v);
@@ -210,11 +258,29 @@ IG_DEV int huge_owner(const unsigned* hoff, int nh, unsigned item)
   return lo;
 }
 
+// The same, by a whole wave (all lanes converged): 64 probes a step, so two
+// dependent loads for up to 4096 huge entries.
+IG_DEV int huge_owner_wave(const unsigned* hoff, int nh, unsigned item)
+{
+  int lo = 0, n = nh;  // the answer is in [lo, lo + n)
+  while (n > 1) {
+    const int step = (n + kWave - 1) / kWave;
+    const int at = lane_id() * step;
+    // lane 0's probe holds (its entry starts at or before item), the others
+    // hold up to the answer's own block
+    const unsigned long long le = __ballot(at < n && (at == 0 || ld_relaxed(&hoff[lo + at]) <= item));
+    const int block = __popcll(le) - 1;
+    lo += block * step;
+    n = min(step, n - block * step);
+  }
+  return lo;
+}
+
 // Workgroup-collective grid-stride pass over vertices 0..nodes-1 (64 per
 // wave) that appends every vertex with a list of >= kMid entries to the mid /
 // huge queues, aggregated per workgroup.
-template <int kMid = kMidDeg, int S, int M>
-IG_DEV void collect_heavy(FrontierEmitterT<S, M>& E, int nodes, const int* __restrict__ nindex,
+template <int kMid, int kHuge, int kChunk, int S, int M, int H>
+IG_DEV void collect_heavy(FrontierEmitterT<S, M, H>& E, int nodes, const int* __restrict__ nindex,
                           const FrontierQueues& fq, FrontierCounters* c)
 {
   const int lane = lane_id();
@@ -224,7 +290,7 @@ IG_DEV void collect_heavy(FrontierEmitterT<S, M>& E, int nodes, const int* __res
   for (int w = blockIdx.x * wpb + threadIdx.x / kWave; w < nw; w += gridDim.x * wpb) {
     const int v = w * kWave + lane;
     const int deg = v < nodes ? nindex[v + 1] - nindex[v] : 0;
-    frontier_emit_block<kMid>(E, deg >= kMid, v, deg, fq, c);
+    frontier_emit_block<kMid, kHuge, kChunk>(E, deg >= kMid, v, deg, fq, c);
   }
   fe_flush(E, fq, c);
 }
@@ -234,29 +300,40 @@ IG_DEV void collect_heavy(FrontierEmitterT<S, M>& E, int nodes, const int* __res
 // workgroup) converged; `active` says whether (v, e) is a real CSR entry of a
 // frontier vertex v.  f may use wave-collective operations.
 
-// Huge lists: one workgroup per kHugeChunk-entry item.
+// Waves per item of a pass over n items on the grid's waves: the largest
+// power of two up to `most` that leaves no wave with two items.
+IG_DEV unsigned waves_per_item(unsigned n, unsigned most)
+{
+  const unsigned nwaves = gridDim.x * (blockDim.x / kWave);
+  unsigned k = 1;
+  while (k < most && static_cast<unsigned long long>(n) * k * 2 <= nwaves) k *= 2;
+  return k;
+}
+
+// Huge lists: one wave per kHugeChunk-entry item, or, while there are few items,
+// k waves each (k up to one per window), wave j taking windows j, j + k, ...
 template <typename F>
 IG_DEV void expand_huge(const FrontierQueues& in, unsigned nh, unsigned nch, const int* __restrict__ nindex, F&& f)
 {
-  __shared__ int s_owner;
-  for (unsigned item = blockIdx.x; item < nch; item += gridDim.x) {
-    if (threadIdx.x == 0) s_owner = huge_owner(in.hoff, static_cast<int>(nh), item);
-    __syncthreads();
-    const int j = s_owner;
-    __syncthreads();
+  const int lane = lane_id();
+  const unsigned wpb = blockDim.x / kWave;
+  const unsigned k = waves_per_item(nch, kHugeChunk / kWave);
+  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nch * k; i += gridDim.x * wpb) {
+    const unsigned item = i / k;
+    const int j = huge_owner_wave(in.hoff, static_cast<int>(nh), item);
     const int v = ld_relaxed(&in.hq[j]);
     const int beg = nindex[v] + static_cast<int>(item - ld_relaxed(&in.hoff[j])) * kHugeChunk;
     const int end = min(nindex[v + 1], beg + kHugeChunk);
-    for (int base = beg; base < end; base += blockDim.x) {
-      const int e = base + static_cast<int>(threadIdx.x);
+    for (int base = beg + static_cast<int>(i % k) * kWave; base < end; base += static_cast<int>(k) * kWave) {
+      const int e = base + lane;
       f(v, e, e < end);
     }
   }
 }
 
 // Mid lists: one wave each, or, while there are few of them, k waves each (k
-// up to 16, while 2 * k waves per list still fit the grid), wave j of a list
-// taking its windows j, j + k, ...  Each window is a chain of device-scope
+// up to one per window), wave j of a list taking its windows j, j + k, ...
+// Each window is a chain of device-scope
 // round trips (the neighbour's check, its claim or atomicMin, its degree), so a
 // 4000-entry list walked by one wave set a level's length: BFS's level of 997
 // lists and 3.6M entries on R-MAT 22 took 198 us (calls 0.65 -> 0.53 ms).
@@ -265,10 +342,8 @@ IG_DEV void expand_mid(const FrontierQueues& in, unsigned nm, const int* __restr
 {
   const int lane = lane_id();
   const unsigned wpb = blockDim.x / kWave;
-  const unsigned nwaves = gridDim.x * wpb;
-  unsigned k = 1;
-  while (k < 16 && static_cast<unsigned long long>(nm) * k * 2 <= nwaves) k *= 2;
-  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nm * k; i += nwaves) {
+  const unsigned k = waves_per_item(nm, kHugeDeg / kWave);
+  for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nm * k; i += gridDim.x * wpb) {
     const int v = ld_relaxed(&in.mq[i / k]);
     const int beg = nindex[v], end = nindex[v + 1];
     for (int base = beg + static_cast<int>(i % k) * kWave; base < end; base += static_cast<int>(k) * kWave) {

@@ -10,7 +10,7 @@
 //   every vertex with a short list (< kPrWaveDeg entries) is summed by one
 //   lane in vertex order (coalesced score / contrib / index traffic);
 //   longer lists, collected once into a static list, one wave each; lists of
-//   kHugeDeg or more in kHugeChunk-entry items, one workgroup each, whose
+//   kPrHugeDeg or more in kPrHugeChunk-entry items, one workgroup each, whose
 //   partial sums go to a per-item slot; the workgroup that finishes a huge
 //   vertex's last item (a counter per vertex) combines its item partials in
 //   item order, so no second barrier is needed;
@@ -43,6 +43,8 @@ namespace {
 
 constexpr int kPrBlock = 512;
 constexpr int kPrWaveDeg = 16;
+constexpr int kPrHugeDeg = 4096;   // lists split into items
+constexpr int kPrHugeChunk = 2048;  // entries per item, one workgroup each
 constexpr float kDamp = 0.85f;
 
 constexpr int kPrMaxGrid = 4096;
@@ -72,9 +74,9 @@ struct PrArgs {
   const int* __restrict__ degree;  // optional caller-provided degrees (PR_GPU contract)
   float* scores;
   float* contrib[2];
-  FrontierQueues heavy;  // lists of >= kPrWaveDeg entries (mid) and >= kHugeDeg (huge)
+  FrontierQueues heavy;  // lists of >= kPrWaveDeg entries (mid) and >= kPrHugeDeg (huge)
   float2* hpart;         // per huge item: compensated partial (sum, error)
-  int hcap;              // huge vertices at most: edges / kHugeDeg + 1
+  int hcap;              // huge vertices at most: edges / kPrHugeDeg + 1
   unsigned* hdone;       // per huge vertex: items finished this sweep
   double* hres;          // per huge vertex: |s' - s| of this sweep
   double* partial;       // [2][2 * kPrMaxGrid] per-workgroup residuals (phase A, phase B)
@@ -194,7 +196,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
   }
   for (int j = tid; j < a.hcap; j += stride) st_relaxed(&a.hdone[j], 0u);
   trace_level(&ctl->trace, 0, 0u, 0ull, 0);
-  collect_heavy<kPrWaveDeg>(s_emit, a.nodes, a.nindex, a.heavy, &ctl->heavy);
+  collect_heavy<kPrWaveDeg, kPrHugeDeg, kPrHugeChunk>(s_emit, a.nodes, a.nindex, a.heavy, &ctl->heavy);
   trace_level(&ctl->trace, 1, 0u, 0ull, 1);
   if (!grid_barrier(&ctl->bar, deadline)) {
     if (tid == 0) ctl->status = 1;
@@ -223,10 +225,10 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
       const int j = s_owner;
       const int v = a.heavy.hq[j];
       const int len = a.nindex[v + 1] - a.nindex[v];
-      const int items = (len + kHugeChunk - 1) / kHugeChunk;
+      const int items = (len + kPrHugeChunk - 1) / kPrHugeChunk;
       const unsigned first = a.heavy.hoff[j];
-      const int beg = a.nindex[v] + static_cast<int>(item - first) * kHugeChunk;
-      const int end = min(a.nindex[v + 1], beg + kHugeChunk);
+      const int beg = a.nindex[v] + static_cast<int>(item - first) * kPrHugeChunk;
+      const int end = min(a.nindex[v + 1], beg + kPrHugeChunk);
       CSum acc;
       gather<kPrBlock>(acc, cin, a.nlist, beg, end, static_cast<int>(threadIdx.x));
       const CSum blk = block_merge(acc, s_ps, s_pc);
@@ -310,17 +312,17 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
 }  // namespace
 
 // Upper bound on the number of huge items: every huge list has at least
-// kHugeDeg entries, so items <= edges / kHugeChunk + edges / kHugeDeg.
+// kPrHugeDeg entries, so items <= edges / kPrHugeChunk + edges / kPrHugeDeg.
 static size_t pr_max_chunks(int edges)
 {
-  return static_cast<size_t>(edges) / kHugeChunk + static_cast<size_t>(edges) / kHugeDeg + 2;
+  return static_cast<size_t>(edges) / kPrHugeChunk + static_cast<size_t>(edges) / kPrHugeDeg + 2;
 }
 
 size_t pr_workspace_bytes(int nodes, int edges)
 {
   const size_t v = static_cast<size_t>(nodes);
   return Carver::round(sizeof(PrControl)) + 6 * Carver::round(v * 4) + Carver::round(pr_max_chunks(edges) * 8) +
-         Carver::round((static_cast<size_t>(edges) / kHugeDeg + 1) * 12) + 256 +
+         Carver::round((static_cast<size_t>(edges) / kPrHugeDeg + 1) * 12) + 256 +
          Carver::round(4 * kPrMaxGrid * 8) + Carver::round(kPrMaxGrid * 4) + Carver::round(kPrMaxGrid * 8) + 4096;
 }
 
@@ -351,7 +353,7 @@ int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   a.heavy.hq = cv.take<int>(nodes);
   a.heavy.hoff = cv.take<unsigned>(nodes);
   a.hpart = cv.take<float2>(pr_max_chunks(edges));
-  a.hcap = edges / kHugeDeg + 1;  // every huge list holds kHugeDeg entries or more
+  a.hcap = edges / kPrHugeDeg + 1;  // every huge list holds kPrHugeDeg entries or more
   a.hdone = cv.take<unsigned>(static_cast<size_t>(a.hcap));
   a.hres = cv.take<double>(static_cast<size_t>(a.hcap));
   a.partial = cv.take<double>(4 * kPrMaxGrid);

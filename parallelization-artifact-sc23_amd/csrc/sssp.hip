@@ -109,6 +109,7 @@ IG_DEV void se_reset(SsspEmit& S)
 
 IG_DEV void se_park(SsspEmit& S, bool park, int u, int d, int* far, unsigned* far_cnt)
 {
+  if (__ballot(park) == 0ull) return;
   bq_append(S.far, park, u, far, far_cnt);
   const int m = wave_min(park ? d : kInf);
   if (lane_id() == 0 && m != kInf) atomicMin(&S.far_min, static_cast<unsigned>(m));

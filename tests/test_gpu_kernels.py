@@ -100,6 +100,32 @@ def test_short_list_levels(ig, orc, ctx, mids, leaves):
         ctx.set_hint(ig._lib.HINT_SMALL_FRONTIER, 0)
 
 
+@pytest.mark.parametrize("hubs, leaves", [(3, 62), (3, 63), (3, 510), (3, 511), (3, 512), (3, 1023), (3, 1024),
+                                          (1, 2050), (65, 700), (4100, 511), (3000, 600)])
+def test_long_list_levels(ig, orc, ctx, hubs, leaves):
+    """A source joined to `hubs` vertices that share `leaves` leaves: lists of
+    leaves + 1 entries around the bin edges (64, 512) and the 512-entry
+    chunks, from few lists (several waves each) to more than a workgroup
+    buffers, by the grid only."""
+    n = 1 + hubs + leaves
+    h = np.arange(1, 1 + hubs)
+    src = np.concatenate([np.zeros(hubs, np.int64), np.repeat(h, leaves)])
+    dst = np.concatenate([h, np.tile(np.arange(1 + hubs, n), hubs)])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32), wseed=4, wmin=1, wmax=200)
+    dg = ig.DeviceGraph(g)
+    assert np.array_equal(ctx.cc(dg), orc.cc(g))
+    for direction in (0, 1):
+        ctx.set_hint(ig._lib.HINT_SMALL_FRONTIER, 1)
+        ctx.set_hint(ig._lib.HINT_BFS_DIRECTION, direction)
+        try:
+            for s in (0, n - 1):
+                assert np.array_equal(ctx.bfs(dg, s), orc.bfs(g, s)), (s, direction)
+                assert np.array_equal(ctx.sssp(dg, s), orc.sssp(g, s)), s
+        finally:
+            ctx.set_hint(ig._lib.HINT_SMALL_FRONTIER, 0)
+            ctx.set_hint(ig._lib.HINT_BFS_DIRECTION, 0)
+
+
 def test_cc_catalog(ig, orc, ctx):
     for g in catalog(ig):
         assert np.array_equal(ctx.cc(ig.DeviceGraph(g)), orc.cc(g)), g.name
