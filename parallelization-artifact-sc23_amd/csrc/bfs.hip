@@ -24,12 +24,13 @@
 //     start) one wave each with a ballot per 64 entries.
 // The direction follows Beamer's heuristic (m_f > m_u / 14 -> bottom-up,
 // n_f < V / 24 -> top-down), evaluated identically by every workgroup.
-// Small frontiers (high-diameter graphs) are advanced by workgroup 0 alone
-// with LDS queues and workgroup barriers only (small_phase).  Vertices without
+// Narrow frontiers (high-diameter graphs) are advanced by one workgroup or a
+// team of them, with LDS queues and no grid barriers (team_phase).  Vertices without
 // neighbours get their level but never enter a frontier.
 #include "bfs.hpp"
 
 #include "frontier.hpp"
+#include "team.hpp"
 #include "trace.hpp"
 
 namespace indigo {
@@ -37,21 +38,34 @@ namespace indigo {
 namespace {
 
 constexpr int kBfsBlock = 512;
-// One-workgroup phase: LDS queue capacity; the phase runs while the frontier's
-// degree sum (an upper bound on the next frontier) fits.
-constexpr int kSmallCap = 4096;
+// Team phase: LDS capacity of a member's share, in vertices and in the degree
+// sum (an upper bound on its next share).
+constexpr int kSmallCap = 2048;
+// Degree sums up to which a frontier is one workgroup's, and a member's average
+// share of a team's.  (One workgroup for up to 2047 entries made a 300 x 411 road
+// 2.11 ms instead of 1.58; shares of 512 measured the same as 1024.)  A team also
+// takes only a frontier at most twice as large as the one before: on a graph
+// whose levels explode, it would have to hand the next one back at once.
+constexpr unsigned kSoloEntries = 1024;
+constexpr unsigned kShareEntries = 1024;
+
+// Largest share with which a team goes on: one workgroup hands over to the
+// grid (and a team) above kSoloEntries, a team when a member's LDS may not hold
+// the next share.
+IG_DEV unsigned team_share(int size) { return size == 1 ? kSoloEntries : static_cast<unsigned>(kSmallCap); }
 
 struct BfsControl {
   GridBarrier bar;
-  PaddedU32 small_ack;  // workgroups that have read the counters before a one-workgroup phase
+  TeamSlots team;
   FrontierCounters cnt[3];
   FrontierCounters heavy;  // static lists of >= kMidDeg entries (bottom-up)
   int levels;
   int bottom_up_levels;
   int small_levels;
   int status;
-  int level_base;  // level at which the grid resumes after a one-workgroup phase
-  int pad[27];
+  int level_base;   // level at which the grid resumes after a team phase
+  unsigned last_m;  // degree sum of the level before it
+  int pad[26];
   LevelTrace trace;
 };
 
@@ -144,152 +158,102 @@ IG_DEV void bottom_up(const BfsArgs& a, int L, unsigned nheavy, const FrontierQu
   }
 }
 
-// LDS of the one-workgroup phase (shares the kernel's LDS with the level
-// emitter, which is idle meanwhile).
+// LDS of the team phase (shares the kernel's LDS with the level emitter, which
+// is idle meanwhile).
 struct SmallLds {
-  int q[kSmallCap];      // frontier of the current level, refilled with the next one
-  int incl[kSmallCap];   // inclusive prefix of the current frontier's degrees
-  int shift[kSmallCap];  // nindex[v] - exclusive prefix: entry k of frontier slot j is nlist[shift[j] + k]
-  int wsum[kBfsBlock / kWave];
-  int cnt;
-  int total;
+  TeamShare<kSmallCap> share;
   int abort_flag;
 };
 
-// Workgroup 0 advances levels alone while the frontier's degree sum fits the
-// LDS arrays, paying workgroup barriers only.  Entered at level L with the
-// frontier in the small global queue (n entries, degree sum <= kSmallCap);
-// on leaving (frontier empty, or its degree sum too large) it re-emits the
-// frontier of the level it reached into that level's global queues and
-// counters, cleared first.  The counters may only be touched once every other
-// workgroup has read level L's counters: each of them bumps small_ack
-// (release) after deciding on this phase, and workgroup 0 waits for all of
-// them (bounded) before the hand-back.  Returns the level reached.
+// A team of workgroups (one, or up to kTeamMax) advances levels alone while
+// the frontier's lists are short and few: team.hpp has the scheme.  To the grid
+// the phase is one pass like any other: entered at level L with the frontier in
+// `in` (n vertices of the small queue), it leaves the frontier of the level that
+// it reached (empty, or too large for the members) in `out` / `oc`, so the
+// workgroups outside the team go straight to the barrier.  A team whose members'
+// shares do not all fit the LDS changes nothing and returns L.  Returns the
+// level reached; *last gets the degree sum of the level before it.
 //
-// A level is three dependent rounds of global accesses: the frontier's
-// index pairs (all at once, one run of slots per thread), then after a
-// workgroup prefix sum the list entries spread evenly over all 512 threads,
-// then one CAS per entry (INT_MAX -> L + 1, so each vertex is claimed once).
+// A level is two dependent rounds of global accesses: the list entries, and
+// then, together, each entry's claim (a CAS INT_MAX -> L + 1, so each vertex is
+// claimed once) and its neighbour's index pair, which the next level finds in
+// LDS.  A slot's list is walked by g lanes, g the power of two that spreads
+// the share over the workgroup (64 at most), 4 entries in flight
+// per lane; a share averages kSmallCap / slots entries a slot at most, so
+// no lane walks long.  (A workgroup prefix sum and a binary search in LDS for each
+// entry's owner, on one workgroup, had made a level 10 us on the 1024^2 grid; wider
+// frontiers ran on the grid, 8 to 15 us a level.)  1024^2 grid 16.4 -> 6.3 ms a call,
+// roads of 1024^2, 2048^2 and 4096^2 28, 40 and 110 -> 5.8, 10.0 and 29.6 ms.
 // Claimed vertices join the next frontier whatever their degree; those
 // without neighbours contribute no entries and are not handed back.
-IG_DEV int small_phase(const BfsArgs& a, int L, unsigned n, BfsControl* ctl, long long deadline, bool* aborted,
-                       SmallLds& S)
+IG_DEV int team_phase(const BfsArgs& a, int L, unsigned n, const Team& tm, const FrontierQueues& in,
+                      const FrontierQueues& out, FrontierCounters* oc, BfsControl* ctl, long long deadline,
+                      bool* aborted, unsigned* last, SmallLds& S)
 {
-  constexpr int kPer = kSmallCap / kBfsBlock;  // frontier slots per thread
-  const int lane = lane_id();
-  const int wid = threadIdx.x / kWave;
-  const int* gin = a.fq[L & 1].q;
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) S.q[i] = ld_relaxed(&gin[i]);
-  if (threadIdx.x == 0) {
-    S.cnt = static_cast<int>(n);
-    S.abort_flag = 0;
-  }
-  __syncthreads();
-  *aborted = false;
-  int cn = S.cnt;
+  constexpr int kFly = 4;  // entries in flight per lane
+  const int t = static_cast<int>(threadIdx.x);
+  TeamShare<kSmallCap>& F = S.share;
+  if (t == 0) S.abort_flag = 0;
+  unsigned entries = 0;
+  int cn = share_load(F, L & 1, tm, static_cast<int>(n), a.nindex, [&](int i) { return ld_relaxed(&in.q[i]); }, &entries);
+  TeamSum sum;
+  *aborted = !team_exchange(&ctl->team, kSlotEntry, tm, static_cast<unsigned>(L) + 1u, entries, 0u, &ctl->bar,
+                            deadline, F, sum);
+  // (a share of more vertices than the LDS holds has more entries, too: the
+  // queue's lists are not empty)
+  if (*aborted || sum.most > static_cast<unsigned>(kSmallCap)) return L;
   for (;;) {
-    if (cn == 0) break;
-    if ((L & 63) == 0 && threadIdx.x == 0) S.abort_flag = kernel_aborted(&ctl->bar, deadline) ? 1 : 0;
-    // round 1: index pairs of this thread's run of frontier slots
-    const int i0 = min(cn, static_cast<int>(threadIdx.x) * kPer);
-    const int i1 = min(cn, i0 + kPer);
-    int beg[kPer], deg[kPer];
-    int mine = 0;
+    if ((L & 63) == 0 && t == 0) S.abort_flag = kernel_aborted(&ctl->bar, deadline) ? 1 : 0;
+    int shift = 0;  // g = 1 << shift lanes per slot
+    while (shift < 6 && (cn << (shift + 1)) <= kBfsBlock) shift++;
+    const int sub = t & ((1 << shift) - 1);
+    const int now = L & 1, next = L + 1;
+    if (t == 0) F.cnt[(L + 2) % 3] = 0ull;
+    for (int i0 = 0; i0 < cn; i0 += kBfsBlock >> shift) {
+      const int i = i0 + (t >> shift);
+      const int beg = i < cn ? F.beg[now][i] : 0;
+      const int end = i < cn ? beg + F.deg[now][i] : 0;
+      for (int e0 = beg + sub; __ballot(e0 < end) != 0ull; e0 += kFly << shift) {
+        int u[kFly];
+        IndexPair ip[kFly];
+        bool act[kFly];
 #pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const bool ok = i0 + j < i1;
-      const int v = ok ? S.q[i0 + j] : 0;
-      beg[j] = ok ? a.nindex[v] : 0;
-      deg[j] = ok ? a.nindex[v + 1] - beg[j] : 0;
-      mine += deg[j];
+        for (int q = 0; q < kFly; q++) {
+          const int e = e0 + (q << shift);
+          act[q] = e < end;
+          u[q] = act[q] ? a.nlist[e] : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < kFly; q++) {
+          if (act[q]) ip[q] = index_pair(a.nindex, u[q]);
+          act[q] = act[q] && cas_relaxed(&a.dist[u[q]], kInf, next);
+        }
+        // (at most as many claims as the share has entries)
+        share_append(F, next, act, u, ip);
+      }
     }
-    const int winc = wave_inclusive_scan(mine);
-    if (lane == kWave - 1) S.wsum[wid] = winc;
     __syncthreads();
     if (S.abort_flag) {
       *aborted = true;
       return L;
     }
-    int before = 0, total = 0;
-    for (int w = 0; w < kBfsBlock / kWave; w++) {
-      before += w < wid ? S.wsum[w] : 0;
-      total += S.wsum[w];
-    }
-    if (total > kSmallCap) break;  // S.q still holds level L's frontier
-    int run = before + winc - mine;
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      if (i0 + j < i1) {
-        S.incl[i0 + j] = run + deg[j];
-        S.shift[i0 + j] = beg[j] - run;
-        run += deg[j];
-      }
-    }
-    if (threadIdx.x == 0) S.cnt = 0;
-    __syncthreads();
-    // rounds 2 and 3: list entries, then claims; the next frontier refills S.q
-    const int next = L + 1;
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const int k = j * kBfsBlock + static_cast<int>(threadIdx.x);
-      const bool act = k < total;
-      int u = 0;
-      if (act) {
-        int lo = 0, hi = cn - 1;  // owner: the first slot with incl > k
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (S.incl[mid] > k) hi = mid;
-          else lo = mid + 1;
-        }
-        u = a.nlist[S.shift[lo] + k];
-      }
-      beg[j] = u;  // reuse: the entry's neighbour
-      deg[j] = act ? 1 : 0;
-    }
-#pragma unroll
-    for (int j = 0; j < kPer; j++) deg[j] = deg[j] && cas_relaxed(&a.dist[beg[j]], kInf, next);
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const unsigned long long m = __ballot(deg[j] != 0);
-      if (m != 0) {
-        const int leader = __ffsll(static_cast<long long>(m)) - 1;
-        int b = 0;
-        if (lane == leader) b = atomicAdd(&S.cnt, __popcll(m));
-        b = wave_shfl(b, leader);
-        // at most `total` <= kSmallCap claims in all
-        if (deg[j]) S.q[b + lanes_below(m)] = beg[j];
-      }
-    }
-    __syncthreads();
-    cn = S.cnt;
     L = next;
-    __syncthreads();
-  }
-  // hand the level-L frontier back to the grid, once all others have read
-  // the entry level's counters
-  if (threadIdx.x == 0) {
-    const unsigned others = gridDim.x - 1u;
-    while (__hip_atomic_load(&ctl->small_ack.v, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < others) {
-      if (kernel_aborted(&ctl->bar, deadline)) {
-        S.abort_flag = 1;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
+    *last = sum.total;
+    const unsigned long long c = F.cnt[L % 3];
+    cn = static_cast<int>(c & 0xffffffffull);
+    if (!team_exchange(&ctl->team, kSlotLevel + (L & 1), tm, static_cast<unsigned>(L), static_cast<unsigned>(c >> 32),
+                       static_cast<unsigned>(cn), &ctl->bar, deadline, F, sum) ||
+        (share_uneven(tm, sum) &&
+         !share_deal(&ctl->team, L & 1, tm, static_cast<unsigned>(L), out.mq, a.nindex, &ctl->bar, deadline, F, cn, sum))) {
+      *aborted = true;
+      return L;
     }
-    __hip_atomic_store(&ctl->small_ack.v, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (!S.abort_flag)
-      for (int k = 0; k < 3; k++) counters_clear(&ctl->cnt[k]);
-  }
-  __syncthreads();
-  if (S.abort_flag) {
-    *aborted = true;
-    return L;
+    if (sum.total == 0u || sum.most > team_share(tm.size)) break;
   }
   for (int base = 0; base < cn; base += blockDim.x) {
-    const int i = base + static_cast<int>(threadIdx.x);
-    const int v = i < cn ? S.q[i] : 0;
-    const int d = i < cn ? degree_of(a.nindex, v) : 0;
-    frontier_emit(d > 0, v, d, a.fq[L & 1], &ctl->cnt[L % 3]);
+    const int i = base + t;
+    const int d = i < cn ? F.deg[L & 1][i] : 0;
+    frontier_emit(d > 0, i < cn ? F.v[L & 1][i] : 0, d, out, oc);
   }
   return L;
 }
@@ -325,11 +289,14 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
   unsigned long long seen_edges = 0;
   int bu_levels = 0;
   int L = 0;
+  int R = 0;              // pass: counters rotate and queues alternate by it
+  int declined = -1;      // level that a team has left to the grid
+  unsigned long long prev = 0;  // degree sum of the level before L
   for (;;) {
-    const FrontierCounters ic = counters_load(&ctl->cnt[L % 3]);
+    const FrontierCounters ic = counters_load(&ctl->cnt[R % 3]);
     const unsigned long long nf = static_cast<unsigned long long>(ic.n) + ic.nm + huge_count(ic.hpack);
     if (nf == 0) break;
-    seen_edges += ic.m;
+    if (declined != L) seen_edges += ic.m;
     if (a.allow_bu) {
       const unsigned long long e = static_cast<unsigned long long>(a.edges);
       const unsigned long long mu = e > seen_edges ? e - seen_edges : 0ull;
@@ -339,19 +306,29 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
         bu = false;
       }
     }
-    const bool small = !bu && a.allow_small && ic.nm == 0 && ic.hpack == 0 &&
-                       ic.m <= static_cast<unsigned long long>(kSmallCap);
-    trace_level(&ctl->trace, L, static_cast<unsigned>(nf), ic.m, small ? 2 : (bu ? 1 : 0));
-    if (small) {
-      // one-workgroup phase; the other workgroups acknowledge that they have
-      // read this level's counters and wait at the next barrier
-      if (blockIdx.x != 0 && threadIdx.x == 0)
-        __hip_atomic_fetch_add(&ctl->small_ack.v, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-      if (blockIdx.x == 0) {
+    int team = 0;  // workgroups of a team phase, 0: a grid level
+    if (!bu && a.allow_small && declined != L && ic.nm == 0 && ic.hpack == 0) {
+      const int limit = team_limit();
+      if (ic.m <= kSoloEntries) team = 1;
+      else if (limit > 1 && ic.m <= static_cast<unsigned long long>(limit) * kShareEntries && ic.m <= 2ull * prev)
+        team = limit;
+    }
+    prev = ic.m;
+    trace_level(&ctl->trace, L, static_cast<unsigned>(nf), ic.m, team != 0 ? 2 : (bu ? 1 : 0));
+    if (tid == 0) counters_clear(&ctl->cnt[(R + 2) % 3]);
+    const FrontierQueues& in = a.fq[R & 1];
+    const FrontierQueues& out = a.fq[(R + 1) & 1];
+    FrontierCounters* oc = &ctl->cnt[(R + 1) % 3];
+    if (team != 0) {
+      // the workgroups outside the team wait at the next barrier
+      const Team tm = make_team(team);
+      if (tm.rank >= 0) {
         bool aborted = false;
-        const int L2 = small_phase(a, L, ic.n, ctl, deadline, &aborted, s_lds.small);
-        if (threadIdx.x == 0) {
+        unsigned last = 0;
+        const int L2 = team_phase(a, L, ic.n, tm, in, out, oc, ctl, deadline, &aborted, &last, s_lds.small);
+        if (tm.rank == 0 && threadIdx.x == 0) {
           st_relaxed(&ctl->level_base, L2);
+          st_relaxed(&ctl->last_m, last);
           ctl->small_levels += L2 - L;
         }
       }
@@ -360,17 +337,15 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
         return;
       }
       const int L2 = ld_relaxed(&ctl->level_base);
-      if (L2 == L) {  // cannot happen: the phase always advances at least one level
-        if (tid == 0) ctl->status = 2;
-        return;
+      if (L2 == L) {  // an uneven frontier: this level goes to the grid
+        declined = L;
+        continue;
       }
+      prev = ld_relaxed(&ctl->last_m);
       L = L2;
+      R++;
       continue;
     }
-    if (tid == 0) counters_clear(&ctl->cnt[(L + 2) % 3]);
-    const FrontierQueues& in = a.fq[L & 1];
-    const FrontierQueues& out = a.fq[(L + 1) & 1];
-    FrontierCounters* oc = &ctl->cnt[(L + 1) % 3];
     fe_reset(s_emit);
     if (bu) {
       bottom_up(a, L, nheavy, out, oc, s_emit);
@@ -384,6 +359,7 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
       return;
     }
     L++;
+    R++;
   }
   if (tid == 0) {
     ctl->levels = L;

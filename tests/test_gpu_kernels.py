@@ -126,6 +126,66 @@ def test_long_list_levels(ig, orc, ctx, hubs, leaves):
             ctx.set_hint(ig._lib.HINT_BFS_DIRECTION, 0)
 
 
+@pytest.mark.parametrize("workgroups", [0, 1, 9, 17, 100])
+@pytest.mark.parametrize("delta", [0, 40, 100000])
+def test_team_levels(ig, orc, ctx, workgroups, delta):
+    """Graphs with levels of 1 to 10000 entries: one workgroup, teams of 2 (17
+    workgroups), 12 (100) and 32 members, and the grid in turn; delta 40 makes
+    SSSP split its far pile all the time."""
+    ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, workgroups)
+    ctx.set_hint(ig._lib.HINT_SSSP_DELTA, delta)
+    try:
+        for g in (weighted(ig, ig.grid(700, 501), seed=2, wmax=100), ig.road(600, 511, seed=3, wmin=1, wmax=1000)):
+            dg = ig.DeviceGraph(g)
+            for src in (0, (g.nodes + 500) // 2):
+                assert np.array_equal(ctx.bfs(dg, src), orc.bfs(g, src)), (g.name, src)
+                assert np.array_equal(ctx.sssp(dg, src), orc.sssp(g, src)), (g.name, src)
+    finally:
+        ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, 0)
+        ctx.set_hint(ig._lib.HINT_SSSP_DELTA, 0)
+
+
+@pytest.mark.parametrize("leaves", [1023, 1024, 1025, 2047, 2048, 2049])
+def test_sssp_split_fills_share(ig, orc, ctx, leaves):
+    """All leaves of a star are parked at once and fall below the next split
+    together, more than a member's share (1024) or far pile (2048) holds; each
+    has one vertex behind it."""
+    n = 1 + 2 * leaves
+    m = np.arange(1, 1 + leaves)
+    src = np.concatenate([np.zeros(leaves, np.int64), m])
+    dst = np.concatenate([m, m + leaves])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32), wseed=3, wmin=900, wmax=1000)
+    dg = ig.DeviceGraph(g)
+    ctx.set_hint(ig._lib.HINT_SSSP_DELTA, 200)
+    try:
+        for s in (0, 1, n - 1):
+            assert np.array_equal(ctx.sssp(dg, s), orc.sssp(g, s)), s
+    finally:
+        ctx.set_hint(ig._lib.HINT_SSSP_DELTA, 0)
+
+
+def test_sssp_far_pile_spills(ig, orc, ctx):
+    """A path of weight-1 links whose vertices have 40 leaves of weight 1000 each:
+    one near vertex at a time, whose leaves are parked beyond the 2048 that a
+    member's pile holds."""
+    path, fan = 200, 40
+    n = path * (1 + fan)
+    leaf = np.arange(path, n)
+    src = np.concatenate([np.arange(path - 1), np.repeat(np.arange(path), fan)])
+    dst = np.concatenate([np.arange(1, path), leaf])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32))
+    sp = g.sp()
+    g = g.with_weights(np.where((sp < path) & (g.nlist < path), 1, 1000 + np.maximum(sp, g.nlist) % 7))
+    dg = ig.DeviceGraph(g)
+    for delta in (0, 50, 100000):
+        ctx.set_hint(ig._lib.HINT_SSSP_DELTA, delta)
+        try:
+            for s in (0, path // 2, n - 1):
+                assert np.array_equal(ctx.sssp(dg, s), orc.sssp(g, s)), (delta, s)
+        finally:
+            ctx.set_hint(ig._lib.HINT_SSSP_DELTA, 0)
+
+
 def test_cc_catalog(ig, orc, ctx):
     for g in catalog(ig):
         assert np.array_equal(ctx.cc(ig.DeviceGraph(g)), orc.cc(g)), g.name
