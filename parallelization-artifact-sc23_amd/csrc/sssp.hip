@@ -27,19 +27,17 @@
 //     the rest stay parked;
 //   * vertices are expanded with their current distance (re-read at
 //     expansion), so stale duplicates only cost work, never correctness;
-//   * while the near frontier is small (only short lists, degree sum <=
-//     kSsspSmallCap), workgroup 0 runs the near iterations alone with the
-//     frontier in LDS and workgroup barriers only (small_near), parking
-//     entries at or above the split in the far pile as the grid does, and
-//     also the splits while the far pile has at most kSsspSmallCap entries;
-//     it hands the frontier back when it outgrows the LDS, or when the
-//     frontier empties with a larger (or no) far pile.  Deep sparse graphs spend thousands of iterations on
-//     frontiers of tens of vertices, where the grid barrier was most of an
-//     iteration's cost.
+//   * while the near frontier is narrow (only short lists, few entries), one
+//     workgroup or a team of them runs the near iterations and the splits
+//     alone, with the frontier and the newly parked vertices in LDS and no grid
+//     barriers (team_near); it hands both back to the grid when they outgrow
+//     the LDS.  Deep sparse graphs spend thousands of iterations on frontiers
+//     of tens to thousands of vertices.
 // delta defaults to a sampled mean weight x 32 / mean degree (at least 1).
 #include "sssp.hpp"
 
 #include "frontier.hpp"
+#include "team.hpp"
 #include "trace.hpp"
 
 namespace indigo {
@@ -47,11 +45,17 @@ namespace indigo {
 namespace {
 
 constexpr int kSsspBlock = 512;
-constexpr int kSsspSmallCap = 2048;  // list entries of a one-workgroup iteration
+// Team phase: LDS capacity of a member's near share, in vertices and in entries,
+// and of its far pile; degree sums up to which a near frontier is one
+// workgroup's, and a member's average share of a team's.
+constexpr int kShareCap = 1024;
+constexpr int kFarCap = 2048;
+constexpr unsigned kSoloEntries = 1024;
+constexpr unsigned kShareEntries = 512;
 
 struct SsspControl {
   GridBarrier bar;
-  PaddedU32 small_ack;  // workgroups that have read the counters before a one-workgroup phase
+  TeamSlots team;
   FrontierCounters cnt[3];
   PaddedU32 far_cnt[3];
   PaddedU32 far_min[3];
@@ -59,11 +63,13 @@ struct SsspControl {
   int epochs;
   int status;
   int delta;
-  int small_iters;  // iterations (near and split) run by workgroup 0 alone
-  int level_base;   // counter rotation index at which the grid resumes after a one-workgroup phase
-  int it_base;      // iteration (stamp) count at which it resumes
-  int split_base;   // split T at which it resumes
-  int epoch_base;   // far-pile epoch at which it resumes
+  int small_iters;  // iterations (near and split) run by teams
+  // where the grid resumes after a team phase: iteration (stamp) count, split
+  // T, far-pile epoch, degree sum of the frontier before the one handed over
+  int it_base;
+  int split_base;
+  int epoch_base;
+  unsigned last_m;
   int pad[23];
   LevelTrace trace;
 };
@@ -153,243 +159,219 @@ IG_DEV void relax(const SsspArgs& a, int dv, int e, bool active, int T, int it_s
   se_park(S, park, u, nd, far, far_cnt);
 }
 
-// LDS of the one-workgroup phase (shares the kernel's LDS with the emitter,
-// which is idle meanwhile).
-struct SsspSmallLds {
-  int q[kSsspSmallCap];      // near frontier of the current iteration, refilled with the next one
-  int incl[kSsspSmallCap];   // inclusive prefix of the frontier's degrees
-  int shift[kSsspSmallCap];  // nindex[v] - exclusive prefix: entry k of slot j is nlist[shift[j] + k]
-  int dv[kSsspSmallCap];     // distance of slot j's vertex at expansion
-  int wsum[kSsspBlock / kWave];
-  int cnt;
+// LDS of the team phase (shares the kernel's LDS with the emitter, which is idle
+// meanwhile): the member's near share, and its own far pile by epoch parity.
+struct SsspTeamLds {
+  TeamShare<kShareCap> share;
+  int far[2][kFarCap];
+  int nfar[2];
+  unsigned far_min[2];
   int abort_flag;
-  unsigned far_min;
 };
 
-// Workgroup 0 runs near iterations alone while the frontier's degree sum
-// fits the LDS arrays.  Entered at rotation index L with the near frontier in
-// the small global queue (n entries); each iteration relaxes every entry as
-// relax() does (distance check, atomicMin, then the stamp for an improvement
-// below T, which joins the next frontier in LDS, or the far-pile stamp for
-// one at or above T, parked in the current epoch's global pile).  When the
-// frontier empties and the far pile holds at most kSsspSmallCap entries, it
-// also splits as the grid does: T moves to max(T, far minimum) + delta, the
-// pile is re-filed (below the new T into the frontier, still above it into
-// the next epoch's pile, settled entries dropped) and the piles rotate.  On
-// leaving (frontier too large, or empty with a larger or no far pile) it
-// re-emits the frontier into the global queues and counters of the rotation
-// index reached, cleared first, once every other workgroup has acknowledged
-// reading the entry counters (small_ack, as in the BFS kernel's
-// one-workgroup phase).  L and it advance by one per iteration and split, as
-// in the grid; T and epoch are updated in place.
-IG_DEV void small_near(const SsspArgs& a, int& L, int& it, unsigned n, int& T, int& epoch, int delta,
-                       SsspControl* ctl, long long deadline, bool* aborted, SsspSmallLds& S)
+// Wave-collective: parks each lane's vertices u[q] (distance d[q]) with `park` in
+// the member's far pile of `epoch`, past its capacity in the global one.
+template <int kFly>
+IG_DEV void team_park(const SsspArgs& a, SsspControl* ctl, SsspTeamLds& S, const bool (&park)[kFly],
+                      const int (&u)[kFly], const int (&d)[kFly], int epoch)
 {
-  constexpr int kPer = kSsspSmallCap / kSsspBlock;  // frontier slots per thread
-  const int lane = lane_id();
-  const int wid = threadIdx.x / kWave;
-  int* far = a.far[epoch % 3];
-  unsigned* far_cnt = &ctl->far_cnt[epoch % 3].v;
-  const int* gin = a.fq[L & 1].q;
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) S.q[i] = ld_relaxed(&gin[i]);
-  if (threadIdx.x == 0) {
-    S.cnt = static_cast<int>(n);
-    S.abort_flag = 0;
-    S.far_min = static_cast<unsigned>(kInf);
+  int mine = 0, least = kInf;
+#pragma unroll
+  for (int q = 0; q < kFly; q++) {
+    if (park[q]) {
+      mine++;
+      least = min(least, d[q]);
+    }
   }
-  __syncthreads();
-  *aborted = false;
-  int cn = S.cnt;
+  const int incl = wave_inclusive_scan(mine);
+  const int all = wave_bcast(incl, kWave - 1);
+  if (all == 0) return;
+  const int p = epoch & 1;
+  int slot = 0;
+  if (lane_id() == 0) slot = atomicAdd(&S.nfar[p], all);
+  slot = wave_bcast(slot, 0) + incl - mine;
+#pragma unroll
+  for (int q = 0; q < kFly; q++) {
+    if (park[q]) {
+      if (slot < kFarCap) S.far[p][slot] = u[q];
+      else st_relaxed(&a.far[epoch % 3][atomic_add_relaxed(&ctl->far_cnt[epoch % 3].v, 1u)], u[q]);
+      slot++;
+    }
+  }
+  if (mine != 0) atomicMin(&S.far_min[p], static_cast<unsigned>(least));
+}
+
+// A team of workgroups (one, or up to kTeamMax) runs near iterations and
+// splits alone while the near frontier's lists are short and few: team.hpp has
+// the scheme.  To the grid the phase is one pass: entered with the near frontier
+// in `in` (n vertices of the small queue, perhaps none), it leaves the frontier it
+// reached (empty, or too large for the members) in `out` / `oc`, and everything
+// parked in the global pile of the epoch it reached.  it, T and epoch are updated
+// in place; they stay as they are where the members' shares do not all fit.
+// *last gets the degree sum of the frontier before the one left.
+//
+// A near iteration is three dependent rounds of global accesses: the list
+// entries, their weights and the vertices' own distances; the distance checks;
+// and for those that pass, together, the minimum, the dedup exchange and the
+// index pair (relax() has the reason).  Lists are walked as in the BFS kernel's
+// team phase.  A split is one round and one more exchange: the members agree on
+// the smallest parked distance, then each re-files its own pile (and its part of
+// the global one); a pile holds a vertex once (farstamp), so marks are
+// plain stores.  Roads of 1024^2, 2048^2 and 4096^2: 20.5, 49.5 and 215 -> 8.9,
+// 24.9 and 65 ms a call (one workgroup took six dependent rounds and a binary
+// search an iteration; wider frontiers and piles ran on the grid).
+IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, int& T, int& epoch, int delta,
+                      const FrontierQueues& in, const FrontierQueues& out, FrontierCounters* oc, SsspControl* ctl,
+                      long long deadline, unsigned* last, SsspTeamLds& S)
+{
+  constexpr int kFly = 2;  // entries in flight per lane (3 and 4 spilled: 1024^2 road 8.9 ms a call, 9.3 and 11.9)
+  const int t = static_cast<int>(threadIdx.x);
+  TeamShare<kShareCap>& F = S.share;
+  if (t == 0) {
+    S.abort_flag = 0;
+    for (int p = 0; p < 2; p++) {
+      S.nfar[p] = 0;
+      S.far_min[p] = static_cast<unsigned>(kInf);
+    }
+  }
+  unsigned entries = 0;
+  int cn = share_load(F, it & 1, tm, static_cast<int>(n), a.nindex, [&](int i) { return ld_relaxed(&in.q[i]); },
+                      &entries);
+  TeamSum sum;
+  if (!team_exchange(&ctl->team, kSlotEntry, tm, static_cast<unsigned>(it) + 1u, entries, 0u, &ctl->bar, deadline, F,
+                     sum))
+    return false;
+  // (a share of more vertices than the LDS holds has more entries, too)
+  if (sum.most > static_cast<unsigned>(kShareCap)) return true;
   for (;;) {
-    if ((it & 63) == 0 && threadIdx.x == 0) S.abort_flag = kernel_aborted(&ctl->bar, deadline) ? 1 : 0;
-    if (cn == 0) {
-      // near frontier empty: split here while the far pile is small
-      const unsigned nf = ld_relaxed(far_cnt);
-      if (nf == 0 || nf > static_cast<unsigned>(kSsspSmallCap)) break;
-      const unsigned fm = min(ld_relaxed(&ctl->far_min[epoch % 3].v), S.far_min);
-      const int fmin = static_cast<int>(fm);
-      trace_level(&ctl->trace, L, nf, 0ull, 3);
-      __syncthreads();  // every thread has read S.far_min and the abort flag
-      if (S.abort_flag) {
-        *aborted = true;
-        return;
-      }
+    if ((it & 63) == 0 && t == 0) S.abort_flag = kernel_aborted(&ctl->bar, deadline) ? 1 : 0;
+    *last = sum.total;
+    if (sum.total == 0u) {
+      // near frontier empty: move the split and re-file the far piles
+      const int p = epoch & 1;
+      const int* gfar = a.far[epoch % 3];
+      const unsigned ng = ld_relaxed(&ctl->far_cnt[epoch % 3].v);
+      unsigned least = min(S.far_min[p], ld_relaxed(&ctl->far_min[epoch % 3].v));
+      if (!team_min(&ctl->team, tm, static_cast<unsigned>(it) + 1u, least, &ctl->bar, deadline, F, &least)) return false;
+      if (least >= static_cast<unsigned>(kInf) || ng > static_cast<unsigned>(tm.size * kFarCap)) break;
+      trace_level(&ctl->trace, it, ng + S.nfar[p], 0ull, 3);
+      const int fmin = static_cast<int>(least);
       const int T_old = T;
       const long long Tn = static_cast<long long>(T > fmin ? T : fmin) + delta;
       T = Tn > kInf ? kInf : static_cast<int>(Tn);
       it++;
-      const int nepoch = epoch + 1;
-      int* nfar = a.far[nepoch % 3];
-      unsigned* nfar_cnt = &ctl->far_cnt[nepoch % 3].v;
-      if (threadIdx.x == 0) {
-        // pile (epoch + 2) % 3 was consumed by the previous split
-        st_relaxed(&ctl->far_cnt[(epoch + 2) % 3].v, 0u);
-        st_relaxed(&ctl->far_min[(epoch + 2) % 3].v, static_cast<unsigned>(kInf));
-        S.far_min = static_cast<unsigned>(kInf);
-        S.cnt = 0;
-        ctl->epochs++;
+      epoch++;
+      if (t == 0) {
+        F.cnt[(it + 1) % 3] = 0ull;
+        S.nfar[p ^ 1] = 0;
+        S.far_min[p ^ 1] = static_cast<unsigned>(kInf);
+        if (tm.rank == 0) {
+          // the pile two epochs on was consumed by the previous split
+          st_relaxed(&ctl->far_cnt[(epoch + 1) % 3].v, 0u);
+          st_relaxed(&ctl->far_min[(epoch + 1) % 3].v, static_cast<unsigned>(kInf));
+          ctl->epochs++;
+        }
       }
       __syncthreads();
-      for (unsigned base = 0; base < nf; base += blockDim.x) {
-        const unsigned i = base + threadIdx.x;
-        bool to_near = false, keep = false;
-        int u = 0, du = 0;
-        if (i < nf) {
-          u = ld_relaxed(&far[i]);
-          du = ld_relaxed(&a.dist[u]);
-          if (du >= T_old) {
-            if (du < T)
-              to_near = __hip_atomic_exchange(&a.stamp[u], it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != it;
-            else
-              keep = __hip_atomic_exchange(&a.farstamp[u], nepoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
-                     nepoch;
+      const int own = min(S.nfar[p], kFarCap);
+      const int part = (static_cast<int>(ng) - tm.rank + tm.size - 1) / tm.size;
+      for (int base = 0; base < own + part; base += kSsspBlock) {
+        const int i = base + t;
+        bool near[1] = {false}, keep[1] = {false};
+        int u[1] = {0}, du[1] = {0};
+        IndexPair ip[1];
+        if (i < own + part) {
+          u[0] = i < own ? S.far[p][i] : ld_relaxed(&gfar[(i - own) * tm.size + tm.rank]);
+          du[0] = ld_relaxed(&a.dist[u[0]]);
+          ip[0] = index_pair(a.nindex, u[0]);
+          near[0] = du[0] >= T_old && du[0] < T;
+          keep[0] = du[0] >= T;
+          if (near[0]) st_relaxed(&a.stamp[u[0]], it);
+          if (keep[0]) st_relaxed(&a.farstamp[u[0]], epoch);
+        }
+        // what a full share cannot hold goes to the grid at once (and ends the phase)
+        const bool over = share_append(F, it, near, u, ip);
+        if (__ballot(over) != 0ull) frontier_emit(over, u[0], ip[0].end - ip[0].beg, out, oc);
+        team_park(a, ctl, S, keep, u, du, epoch);
+      }
+    } else {
+      trace_level(&ctl->trace, it, static_cast<unsigned>(cn), sum.total, 2);
+      const int now = it & 1;
+      it++;
+      if (t == 0) F.cnt[(it + 1) % 3] = 0ull;
+      int shift = 0;  // g = 1 << shift lanes per slot
+      while (shift < 6 && (cn << (shift + 1)) <= kSsspBlock) shift++;
+      const int sub = t & ((1 << shift) - 1);
+      for (int i0 = 0; i0 < cn; i0 += kSsspBlock >> shift) {
+        const int i = i0 + (t >> shift);
+        const int beg = i < cn ? F.beg[now][i] : 0;
+        const int end = i < cn ? beg + F.deg[now][i] : 0;
+        const int dv = i < cn ? ld_relaxed(&a.dist[F.v[now][i]]) : 0;
+        for (int e0 = beg + sub; __ballot(e0 < end) != 0ull; e0 += kFly << shift) {
+          int u[kFly], nd[kFly];
+          IndexPair ip[kFly];
+          bool near[kFly], park[kFly];
+#pragma unroll
+          for (int q = 0; q < kFly; q++) {
+            const int e = e0 + (q << shift);
+            near[q] = e < end;
+            u[q] = near[q] ? a.nlist[e] : 0;
+            nd[q] = near[q] ? a.eweight[e] : 0;
           }
+#pragma unroll
+          for (int q = 0; q < kFly; q++) nd[q] += dv;
+#pragma unroll
+          for (int q = 0; q < kFly; q++) near[q] = near[q] && nd[q] < ld_relaxed(&a.dist[u[q]]);
+#pragma unroll
+          for (int q = 0; q < kFly; q++) {
+            park[q] = false;
+            if (near[q]) {
+              const bool below = nd[q] < T;
+              const int tag = below ? it : epoch;
+              atomic_min_relaxed(&a.dist[u[q]], nd[q]);
+              const int seen = __hip_atomic_exchange(below ? &a.stamp[u[q]] : &a.farstamp[u[q]], tag, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+              ip[q] = index_pair(a.nindex, u[q]);
+              const bool join = seen != tag && ip[q].end > ip[q].beg;
+              near[q] = join && below;
+              park[q] = join && !below;
+            }
+          }
+          share_append(F, it, near, u, ip);
+          team_park(a, ctl, S, park, u, nd, epoch);
         }
-        const unsigned long long m = __ballot(to_near);
-        if (m != 0) {
-          const int leader = __ffsll(static_cast<long long>(m)) - 1;
-          int b = 0;
-          if (lane == leader) b = atomicAdd(&S.cnt, __popcll(m));
-          b = wave_shfl(b, leader);
-          // at most nf <= kSsspSmallCap entries in all
-          if (to_near) S.q[b + lanes_below(m)] = u;
-        }
-        wave_append(keep, u, nfar, nfar_cnt);
-        const int km = wave_min(keep ? du : kInf);
-        if (lane == 0 && km != kInf) atomicMin(&S.far_min, static_cast<unsigned>(km));
-      }
-      epoch = nepoch;
-      far = nfar;
-      far_cnt = nfar_cnt;
-      __syncthreads();
-      cn = S.cnt;
-      L++;
-      __syncthreads();
-      continue;
-    }
-    // round 1: index pairs and distances of this thread's run of slots
-    const int i0 = min(cn, static_cast<int>(threadIdx.x) * kPer);
-    const int i1 = min(cn, i0 + kPer);
-    int beg[kPer], deg[kPer], dvs[kPer];
-    int mine = 0;
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const bool ok = i0 + j < i1;
-      const int v = ok ? S.q[i0 + j] : 0;
-      beg[j] = ok ? a.nindex[v] : 0;
-      deg[j] = ok ? a.nindex[v + 1] - beg[j] : 0;
-      dvs[j] = ok ? ld_relaxed(&a.dist[v]) : 0;
-      mine += deg[j];
-    }
-    const int winc = wave_inclusive_scan(mine);
-    if (lane == kWave - 1) S.wsum[wid] = winc;
-    __syncthreads();
-    if (S.abort_flag) {
-      *aborted = true;
-      return;
-    }
-    int before = 0, total = 0;
-    for (int w = 0; w < kSsspBlock / kWave; w++) {
-      before += w < wid ? S.wsum[w] : 0;
-      total += S.wsum[w];
-    }
-    if (total > kSsspSmallCap) break;  // S.q still holds this iteration's frontier
-    trace_level(&ctl->trace, L, static_cast<unsigned>(cn), static_cast<unsigned long long>(total), 2);
-    int run = before + winc - mine;
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      if (i0 + j < i1) {
-        S.incl[i0 + j] = run + deg[j];
-        S.shift[i0 + j] = beg[j] - run;
-        S.dv[i0 + j] = dvs[j];
-        run += deg[j];
       }
     }
-    if (threadIdx.x == 0) S.cnt = 0;
     __syncthreads();
-    it++;
-    // round 2: the list entries, spread evenly over the workgroup
-    int u[kPer], nd[kPer];
-    bool act[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const int k = j * kSsspBlock + static_cast<int>(threadIdx.x);
-      act[j] = k < total;
-      u[j] = 0;
-      nd[j] = kInf;
-      if (act[j]) {
-        int lo = 0, hi = cn - 1;  // owner: the first slot with incl > k
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (S.incl[mid] > k) hi = mid;
-          else lo = mid + 1;
-        }
-        const int e = S.shift[lo] + k;
-        u[j] = a.nlist[e];
-        nd[j] = S.dv[lo] + a.eweight[e];
-      }
-    }
-    // round 3: relaxations (device-scope reads, as relax())
-    bool imp[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; j++) imp[j] = act[j] && nd[j] < ld_relaxed(&a.dist[u[j]]);
-#pragma unroll
-    for (int j = 0; j < kPer; j++) imp[j] = imp[j] && nd[j] < atomic_min_relaxed(&a.dist[u[j]], nd[j]);
-    bool near[kPer], park[kPer];
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      near[j] = imp[j] && nd[j] < T &&
-                __hip_atomic_exchange(&a.stamp[u[j]], it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != it;
-      park[j] = imp[j] && nd[j] >= T &&
-                __hip_atomic_exchange(&a.farstamp[u[j]], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch;
-    }
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      const unsigned long long m = __ballot(near[j]);
-      if (m != 0) {
-        const int leader = __ffsll(static_cast<long long>(m)) - 1;
-        int b = 0;
-        if (lane == leader) b = atomicAdd(&S.cnt, __popcll(m));
-        b = wave_shfl(b, leader);
-        // stamps admit each vertex once per iteration: at most total <= kSsspSmallCap
-        if (near[j]) S.q[b + lanes_below(m)] = u[j];
-      }
-      wave_append(park[j], u[j], far, far_cnt);
-      const int pm = wave_min(park[j] ? nd[j] : kInf);
-      if (lane == 0 && pm != kInf) atomicMin(&S.far_min, static_cast<unsigned>(pm));
-    }
-    __syncthreads();
-    cn = S.cnt;
-    L++;
-    __syncthreads();
+    if (S.abort_flag) return false;
+    const unsigned long long c = F.cnt[it % 3];
+    const bool full = (c & 0xffffffffull) > static_cast<unsigned long long>(kShareCap);
+    cn = full ? kShareCap : static_cast<int>(c & 0xffffffffull);
+    if (!team_exchange(&ctl->team, kSlotLevel + (it & 1), tm, static_cast<unsigned>(it),
+                       full ? 0xffffu : static_cast<unsigned>(c >> 32), static_cast<unsigned>(cn), &ctl->bar, deadline,
+                       F, sum))
+      return false;
+    if (sum.most == 0xffffu) break;
+    if (share_uneven(tm, sum) && !share_deal(&ctl->team, it & 1, tm, static_cast<unsigned>(it), out.mq, a.nindex,
+                                             &ctl->bar, deadline, F, cn, sum))
+      return false;
+    if (sum.most > (tm.size == 1 ? kSoloEntries : static_cast<unsigned>(kShareCap))) break;
   }
-  // hand the frontier back to the grid, once all others have read the entry
-  // iteration's counters
-  if (threadIdx.x == 0) {
-    if (S.far_min != static_cast<unsigned>(kInf)) atomic_min_relaxed(&ctl->far_min[epoch % 3].v, S.far_min);
-    const unsigned others = gridDim.x - 1u;
-    while (__hip_atomic_load(&ctl->small_ack.v, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < others) {
-      if (kernel_aborted(&ctl->bar, deadline)) {
-        S.abort_flag = 1;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    __hip_atomic_store(&ctl->small_ack.v, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (!S.abort_flag)
-      for (int k = 0; k < 3; k++) counters_clear(&ctl->cnt[k]);
+  // the rest of the frontier and the member's pile go to the grid
+  const int own = min(S.nfar[epoch & 1], kFarCap);
+  __syncthreads();
+  if (t == 0 && own > 0) {
+    S.nfar[0] = static_cast<int>(atomic_add_relaxed(&ctl->far_cnt[epoch % 3].v, static_cast<unsigned>(own)));
+    atomic_min_relaxed(&ctl->far_min[epoch % 3].v, S.far_min[epoch & 1]);
   }
   __syncthreads();
-  if (S.abort_flag) {
-    *aborted = true;
-    return;
+  for (int i = t; i < own; i += kSsspBlock) st_relaxed(&a.far[epoch % 3][S.nfar[0] + i], S.far[epoch & 1][i]);
+  for (int base = 0; base < cn; base += kSsspBlock) {
+    const int i = base + t;
+    const int d = i < cn ? F.deg[it & 1][i] : 0;
+    frontier_emit(d > 0, i < cn ? F.v[it & 1][i] : 0, d, out, oc);
   }
-  for (int base = 0; base < cn; base += blockDim.x) {
-    const int i = base + static_cast<int>(threadIdx.x);
-    const int v = i < cn ? S.q[i] : 0;
-    const int d = i < cn ? degree_of(a.nindex, v) : 0;
-    frontier_emit(d > 0, v, d, a.fq[L & 1], &ctl->cnt[L % 3]);
-  }
+  return true;
 }
 
 // 6 waves per SIMD: three 512-thread workgroups per CU, the persistent grid's
@@ -398,7 +380,7 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
 {
   __shared__ union {
     SsspEmit emit;
-    SsspSmallLds small;
+    SsspTeamLds small;
   } s_lds;
   SsspEmit& s_emit = s_lds.emit;
   SsspControl* ctl = a.ctl;
@@ -464,63 +446,71 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
   const int delta = ld_relaxed(&ctl->delta);
   int T = delta;  // split: near holds distances < T
   int epoch = 1;  // far pile generation (farstamp value); far[epoch % 3] is current
-  int it = 0;     // near iterations (stamp values start at 1)
-  int L = 0;      // counter rotation index
+  int it = 0;     // near iterations and splits (stamp values start at 1)
+  int R = 0;      // pass: counters rotate and queues alternate by it
+  int declined = -1;           // iteration that a team has left to the grid
+  unsigned long long prev = 0;  // degree sum of the frontier before
   for (;;) {
-    FrontierCounters* ic = &ctl->cnt[L % 3];
+    FrontierCounters* ic = &ctl->cnt[R % 3];
     const unsigned n = ld_relaxed(&ic->n);
     const unsigned nm = ld_relaxed(&ic->nm);
     const unsigned long long hp = ld_relaxed(&ic->hpack);
     const unsigned nh = huge_count(hp), nch = huge_chunks(hp);
-    FrontierCounters* oc = &ctl->cnt[(L + 1) % 3];
-    const FrontierQueues& in = a.fq[L & 1];
-    const FrontierQueues& out = a.fq[(L + 1) & 1];
-    if (tid == 0) counters_clear(&ctl->cnt[(L + 2) % 3]);
+    FrontierCounters* oc = &ctl->cnt[(R + 1) % 3];
+    const FrontierQueues& in = a.fq[R & 1];
+    const FrontierQueues& out = a.fq[(R + 1) & 1];
+    if (tid == 0) counters_clear(&ctl->cnt[(R + 2) % 3]);
     int* far = a.far[epoch % 3];
     unsigned* far_cnt = &ctl->far_cnt[epoch % 3].v;
     unsigned* far_min = &ctl->far_min[epoch % 3].v;
     const bool split = static_cast<unsigned long long>(n) + nm + nh == 0;
     const unsigned long long m = ld_relaxed(&ic->m);
-    const bool small =
-        a.allow_small && !split && nm == 0 && nh == 0 && m <= static_cast<unsigned long long>(kSsspSmallCap);
-    trace_level(&ctl->trace, L, split ? ld_relaxed(far_cnt) : n + nm + nh, split ? 0ull : m,
-                split ? 3 : (small ? 2 : 0));
-    if (small) {
-      // one-workgroup phase; the other workgroups acknowledge that they have
-      // read this iteration's counters and wait at the next barrier
-      if (blockIdx.x != 0 && threadIdx.x == 0)
-        __hip_atomic_fetch_add(&ctl->small_ack.v, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-      if (blockIdx.x == 0) {
-        bool aborted = false;
-        int L2 = L, it2 = it, T2 = T, epoch2 = epoch;
-        small_near(a, L2, it2, n, T2, epoch2, delta, ctl, deadline, &aborted, s_lds.small);
-        if (threadIdx.x == 0) {
-          st_relaxed(&ctl->level_base, L2);
+    const unsigned nfar = split ? ld_relaxed(far_cnt) : 0u;
+    if (split && nfar == 0) break;
+    int team = 0;  // workgroups of a team phase, 0: a grid pass
+    if (a.allow_small && declined != it && nm == 0 && nh == 0) {
+      const int limit = team_limit();
+      if (split) team = nfar <= static_cast<unsigned>(kFarCap) ? 1 : 0;
+      else if (m <= kSoloEntries) team = 1;
+      else if (m <= static_cast<unsigned long long>(limit) * kShareEntries && m <= 2ull * prev) team = limit;
+    }
+    prev = m;
+    trace_level(&ctl->trace, it, split ? nfar : n + nm + nh, split ? 0ull : m, split ? 3 : (team != 0 ? 2 : 0));
+    if (team != 0) {
+      // the workgroups outside the team wait at the next barrier
+      const Team tm = make_team(team);
+      if (tm.rank >= 0) {
+        int it2 = it, T2 = T, epoch2 = epoch;
+        unsigned last = 0;
+        const bool ok =
+            team_near(a, it2, n, tm, T2, epoch2, delta, in, out, oc, ctl, deadline, &last, s_lds.small);
+        if (ok && tm.rank == 0 && threadIdx.x == 0) {
           st_relaxed(&ctl->it_base, it2);
           st_relaxed(&ctl->split_base, T2);
           st_relaxed(&ctl->epoch_base, epoch2);
-          ctl->small_iters += L2 - L;
+          st_relaxed(&ctl->last_m, last);
+          ctl->small_iters += it2 - it;
         }
       }
       if (!grid_barrier<true>(&ctl->bar, deadline)) {
         if (tid == 0) ctl->status = 1;
         return;
       }
-      const int L2 = ld_relaxed(&ctl->level_base);
-      if (L2 == L) {  // cannot happen: the phase always runs at least one iteration
-        if (tid == 0) ctl->status = 2;
-        return;
+      const int it2 = ld_relaxed(&ctl->it_base);
+      if (it2 == it) {  // an uneven frontier: this pass goes to the grid
+        declined = it;
+        continue;
       }
-      L = L2;
-      it = ld_relaxed(&ctl->it_base);
+      it = it2;
       T = ld_relaxed(&ctl->split_base);
       epoch = ld_relaxed(&ctl->epoch_base);
+      prev = ld_relaxed(&ctl->last_m);
+      R++;
       continue;
     }
     if (split) {
       // near frontier empty: move the split and re-file the far pile
-      const unsigned nf = ld_relaxed(far_cnt);
-      if (nf == 0) break;
+      const unsigned nf = nfar;
       const int fmin = static_cast<int>(ld_relaxed(far_min));
       const int T_old = T;
       const long long Tn = static_cast<long long>(T > fmin ? T : fmin) + delta;
@@ -575,7 +565,7 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
       if (tid == 0) ctl->status = 1;
       return;
     }
-    L++;
+    R++;
   }
   if (tid == 0) ctl->iterations = it;
 }
