@@ -7,8 +7,9 @@
 // L1 change of the iteration is > 1e-4 and fewer than 100 iterations ran.
 //
 // Design: one persistent kernel; per iteration
-//   every vertex with a short list (< kPrWaveDeg entries) is summed by one
-//   lane in vertex order (coalesced score / contrib / index traffic);
+//   vertices with short lists (< kPrWaveDeg entries) are taken 64 to a wave in
+//   vertex order (coalesced score / contrib / index traffic), one lane or one
+//   group of lanes to a list;
 //   longer lists, collected once into a static list, one wave each; lists of
 //   kPrHugeDeg or more in kPrHugeChunk-entry items, one workgroup each, whose
 //   partial sums go to a per-item slot; the workgroup that finishes a huge
@@ -42,7 +43,9 @@ namespace indigo {
 namespace {
 
 constexpr int kPrBlock = 512;
-constexpr int kPrWaveDeg = 16;
+constexpr int kPrLaneDeg = 8;    // shorter lists: one lane each (twice as long where no list of the wave is longer)
+constexpr int kPrWaveDeg = 64;   // longer lists up to this: one group of lanes each
+constexpr int kPrGroup = 8;      // lanes of a group
 constexpr int kPrHugeDeg = 4096;   // lists split into items
 constexpr int kPrHugeChunk = 2048;  // entries per item, one workgroup each
 constexpr float kDamp = 0.85f;
@@ -95,30 +98,78 @@ IG_DEV int deg_of(const PrArgs& a, int v)
 // acc += cin[nlist[e]] for e = beg + first, beg + first + step, ... < end,
 // in that order, with kPrUnroll independent loads in flight per lane: the
 // gathers are latency-bound chains (index, then contribution), so a plain
-// loop would wait out one round trip per window.
+// loop would wait out one round trip per window.  Past the end a lane adds 0.
 template <int kStep>
 IG_DEV void gather(CSum& acc, const float* __restrict__ cin, const int* __restrict__ nlist, int beg, int end,
                    int first)
 {
-  int e = beg + first;
-  for (; e + (kPrUnroll - 1) * kStep < end; e += kPrUnroll * kStep) {
+  for (int e = beg + first; e < end; e += kPrUnroll * kStep) {
     int u[kPrUnroll];
 #pragma unroll
-    for (int q = 0; q < kPrUnroll; q++) u[q] = nlist[e + q * kStep];
+    for (int q = 0; q < kPrUnroll; q++) u[q] = e + q * kStep < end ? nlist[e + q * kStep] : -1;
     float c[kPrUnroll];
 #pragma unroll
-    for (int q = 0; q < kPrUnroll; q++) c[q] = cin[u[q]];
+    for (int q = 0; q < kPrUnroll; q++) c[q] = u[q] >= 0 ? cin[u[q]] : 0.f;
 #pragma unroll
     for (int q = 0; q < kPrUnroll; q++) acc.add(c[q]);
   }
-  for (; e < end; e += kStep) acc.add(cin[nlist[e]]);
 }
 
-// New score of v from its gathered sum; writes score and next contrib and
-// returns |s' - s| in FP64.
-IG_DEV double finish_vertex(const PrArgs& a, int v, float total, float base, float* cout)
+// Sum over the kPrGroup lanes of a group, in each of them.
+IG_DEV CSum group_merge(CSum a)
 {
-  const float old = a.scores[v];
+#pragma unroll
+  for (int d = kPrGroup / 2; d > 0; d >>= 1) {
+    const float s2 = __shfl_xor(a.s, d, kWave);
+    const float c2 = __shfl_xor(a.c, d, kWave);
+    a.merge(s2, c2);
+  }
+  return a;
+}
+
+// Wave-collective: the gathered sum of each lane's list [beg, end) where it has
+// fewer than kPrWaveDeg entries (0 elsewhere).  Lists of fewer than kPrLaneDeg
+// entries are summed by their own lane; the others go kPrGroup lanes to a list,
+// kWave / kPrGroup lists at a time, instead of a wave to a list of 16 to 63
+// (random graph of 2^20 vertices and degree 16: 2.06 -> 1.11 ms a call).  A wave
+// without lists of 2 * kPrLaneDeg entries leaves all to their lanes: on degree 4
+// the few longer ones' extra step cost 5%.
+// few: the wave has at most kWave / kPrGroup lists, all of them grouped.
+IG_DEV float short_sums(const float* __restrict__ cin, const int* __restrict__ nlist, int beg, int end, bool few)
+{
+  const int lane = lane_id();
+  const int deg = end - beg;
+  const bool any = few || __ballot(deg >= 2 * kPrLaneDeg && deg < kPrWaveDeg) != 0ull;
+  const int limit = few ? 1 : (any ? kPrLaneDeg : 2 * kPrLaneDeg);
+  CSum own;
+  if (deg < limit) gather<1>(own, cin, nlist, beg, end, 0);
+  float sum = own.value();
+  if (!any) return sum;
+  const bool grouped = deg >= limit && deg < kPrWaveDeg;
+  const unsigned long long m = __ballot(grouped);
+  const int rows = __popcll(m);
+  const int rank = lanes_below(m);
+  // lane r gets the lane of the r-th grouped list (others push past the rows)
+  const int rest = lane - rank + rows;  // lanes without a grouped list, in order, behind them
+  const int at = __builtin_amdgcn_ds_permute((grouped ? rank : rest) << 2, lane);
+  constexpr int kPer = kWave / kPrGroup;
+  for (int r0 = 0; r0 < rows; r0 += kPer) {
+    const int r = r0 + lane / kPrGroup;
+    const int from = wave_shfl(at, r < kWave ? r : kWave - 1);
+    const int b = wave_shfl(beg, from), e = wave_shfl(end, from);
+    CSum acc;
+    if (r < rows) gather<kPrGroup>(acc, cin, nlist, b, e, lane % kPrGroup);
+    acc = group_merge(acc);
+    const float v = wave_shfl(acc.value(), ((rank - r0) & (kPer - 1)) * kPrGroup);
+    if (grouped && rank >= r0 && rank < r0 + kPer) sum = v;
+  }
+  return sum;
+}
+
+// New score of v from its gathered sum and its old score; writes score and next
+// contrib and returns |s' - s| in FP64.
+IG_DEV double finish_vertex(const PrArgs& a, int v, float old, float total, float base, float* cout)
+{
   const float s = base + kDamp * total;
   a.scores[v] = s;
   cout[v] = s / static_cast<float>(deg_of(a, v));
@@ -208,6 +259,23 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
   const unsigned long long hp = ld_relaxed(&ctl->heavy.hpack);
   const unsigned nh = huge_count(hp), nch = huge_chunks(hp);
 
+  // short lists: vertices per wave and turn (fewer while waves are free,
+  // where lists average enough entries for the groups)
+  const int wave = static_cast<int>(blockIdx.x) * wpb + static_cast<int>(threadIdx.x) / kWave;
+  const int nwaves = static_cast<int>(gridDim.x) * wpb;
+  int per = kWave;
+  const bool dense = a.nindex[a.nodes] >= kPrLaneDeg * static_cast<long long>(a.nodes);
+  const int least = dense ? kWave / kPrGroup : kWave;
+  while (per > least && (a.nodes + per / 2 - 1) / (per / 2) <= nwaves) per /= 2;
+  const int chunks = (a.nodes + per - 1) / per;
+  const bool few = per <= kWave / kPrGroup;
+  // A wave's place among the waves moves on by about 4/9 of them a turn.  On R-MAT
+  // graphs a list's length goes with the set bits of its vertex id, so a wave that
+  // kept its place, a multiple of 2^11 vertices apart, met the same kind of
+  // lists every turn (R-MAT 22: 7.06 ms a call, 6.6 with the moves).
+  const int move = (nwaves * 4 / 9) & ~(wpb - 1);
+  auto next_turn = [&](int at) { return at + move < nwaves ? at + move : at + move - nwaves; };
+
   int it = 0;
   for (;;) {
     it++;
@@ -251,7 +319,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
         }
         tot = wave_merge(tot);
         if (lane == 0) {
-          st_relaxed(&a.hres[j], finish_vertex(a, v, tot.value(), base, cout));
+          st_relaxed(&a.hres[j], finish_vertex(a, v, a.scores[v], tot.value(), base, cout));
           st_relaxed(&a.hdone[j], 0u);  // every item of this sweep has counted
         }
       }
@@ -259,22 +327,27 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
     }
     trace_level(&ctl->trace, tl + 1, static_cast<unsigned>(it), 0ull, 1);
     // phase A: mid lists, one wave each
-    for (unsigned i = blockIdx.x * wpb + threadIdx.x / kWave; i < nm; i += gridDim.x * wpb) {
+    for (unsigned i0 = 0, at = wave; i0 < nm; i0 += nwaves, at = next_turn(at)) {
+      const unsigned i = i0 + at;
+      if (i >= nm) continue;
       const int v = a.heavy.mq[i];
       const int beg = a.nindex[v], end = a.nindex[v + 1];
+      const float old = a.scores[v];
       CSum acc;
       gather<kWave>(acc, cin, a.nlist, beg, end, lane);
       acc = wave_merge(acc);
-      if (lane == 0) d += finish_vertex(a, v, acc.value(), base, cout);
+      if (lane == 0) d += finish_vertex(a, v, old, acc.value(), base, cout);
     }
     trace_level(&ctl->trace, tl + 2, static_cast<unsigned>(it), 0ull, 2);
-    // phase A: short lists, one lane each, vertex order
-    for (int v = tid; v < a.nodes; v += stride) {
-      const int beg = a.nindex[v], end = a.nindex[v + 1];
-      if (end - beg >= kPrWaveDeg) continue;
-      CSum acc;
-      gather<1>(acc, cin, a.nlist, beg, end, 0);
-      d += finish_vertex(a, v, acc.value(), base, cout);
+    // phase A: short lists, 64 vertices a wave, vertex order
+    for (int c0 = 0, at = wave; c0 < chunks; c0 += nwaves, at = next_turn(at)) {
+      const int c = c0 + at;
+      const int v = c * per + lane;
+      const bool mine = lane < per && c < chunks && v < a.nodes;
+      const int beg = mine ? a.nindex[v] : 0, end = mine ? a.nindex[v + 1] : 0;
+      const float old = mine ? a.scores[v] : 0.f;  // (in flight beside the gathers)
+      const float sum = short_sums(cin, a.nlist, beg, end, few);
+      if (mine && end - beg < kPrWaveDeg) d += finish_vertex(a, v, old, sum, base, cout);
     }
     d = block_sum_f64(d, s_red);
     if (threadIdx.x == 0) slots[2 * blockIdx.x] = d;

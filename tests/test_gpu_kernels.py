@@ -233,6 +233,22 @@ def _pr_check(ig, orc, g, scores, iters):
     assert err.sum() <= PR_L1, (g.name, err.sum())
 
 
+@pytest.mark.parametrize("copies", [1, 3, 40, 700])
+def test_pagerank_list_lengths(ig, orc, ctx, copies):
+    """Stars of 1 to 130 leaves, around the lengths at which a list goes from a
+    lane to a group of lanes (8, 16) and to a wave (64), joined in a ring by
+    their centres; from fewer vertices than the grid has waves to several
+    turns of all of them."""
+    sizes = np.tile([1, 5, 6, 7, 13, 14, 15, 61, 62, 63, 130], copies)
+    k = len(sizes)
+    leaf = np.arange(k, k + sizes.sum())
+    src = np.concatenate([np.arange(k), np.repeat(np.arange(k), sizes)])
+    dst = np.concatenate([(np.arange(k) + 1) % k, leaf])
+    g = ig.from_edges(k + int(sizes.sum()), src.astype(np.int32), dst.astype(np.int32))
+    scores, iters = ctx.pagerank(ig.DeviceGraph(g))
+    _pr_check(ig, orc, g, scores, iters)
+
+
 def test_pagerank_catalog(ig, orc, ctx):
     for g in catalog(ig):
         scores, iters = ctx.pagerank(ig.DeviceGraph(g))
