@@ -81,6 +81,7 @@
 
 #include "csum.hpp"
 #include "device_common.hpp"
+#include "unionfind.hpp"
 
 namespace indigo {
 
@@ -517,44 +518,14 @@ IG_DEV bool run_sssp(const BatchTask& T, const Team& tm)
 }
 
 // ---- CC ------------------------------------------------------------------------
-IG_DEV int find_root(int* parent, int x)
-{
-  int p = ld_relaxed(&parent[x]);
-  while (p != x) {
-    const int gp = ld_relaxed(&parent[p]);
-    if (gp == p) return p;
-    st_relaxed(&parent[x], gp);  // path halving: gp is an ancestor of x
-    x = gp;
-    p = ld_relaxed(&parent[x]);
-  }
-  return x;
-}
-
-// Root of x without path halving.  The final flatten writes roots into the
-// same array the finds walk: a halving store that read parent[x] before it
-// was flattened could put an intermediate ancestor back over the root, so
-// that pass stores roots only.
+// Root of x without find_root's store.  The final flatten writes roots into the
+// same array the finds walk: a store of what was the root when the walk read it
+// could land over the flattened entry, so that pass stores final roots only.
 IG_DEV int root_of(const int* parent, int x)
 {
   int p;
   while ((p = ld_relaxed(&parent[x])) != x) x = p;
   return x;
-}
-
-IG_DEV void link(int* parent, int a, int b)
-{
-  int ra = find_root(parent, a);
-  int rb = find_root(parent, b);
-  while (ra != rb) {
-    const int hi = ra > rb ? ra : rb;
-    const int lo = ra > rb ? rb : ra;
-    int expected = hi;
-    if (__hip_atomic_compare_exchange_strong(&parent[hi], &expected, lo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT))
-      return;
-    ra = find_root(parent, ra == hi ? expected : ra);
-    rb = find_root(parent, rb == hi ? expected : rb);
-  }
 }
 
 // Workgroup-collective: the most frequent root among kCcSamples vertices

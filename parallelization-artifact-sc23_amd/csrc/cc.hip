@@ -30,8 +30,6 @@
 // unless b was too - and then both are in c's component already.  On R-MAT
 // graphs the giant component holds nearly every vertex with edges, so step
 // 5 reads only a few lists.
-// Finds use path halving with relaxed stores: every store replaces a parent
-// by one of its ancestors, so concurrent finds and links stay valid.
 #include "cc.hpp"
 
 #include <climits>
@@ -86,35 +84,44 @@ __global__ __launch_bounds__(kCcBlock) void cc_compress(int nodes, int* parent)
 }
 
 // One workgroup: the most frequent root among kGiantSamples vertices spread
-// over the id range (ties to the smaller root).
+// over the id range (ties to the smaller root), counted in a hash table in LDS
+// (open addressing, at most half full).  Comparing all pairs of samples took
+// 71 us, a quarter of a call on R-MAT 22; the table 6.6.
 __global__ __launch_bounds__(kCcBlock) void cc_giant(int nodes, int* parent, CcControl* ctl)
 {
-  __shared__ int s_root[kGiantSamples];
-  __shared__ int s_best[kCcBlock], s_cnt[kCcBlock];
+  constexpr int kSlots = 2 * kGiantSamples;
+  __shared__ int s_root[kSlots];
+  __shared__ unsigned s_cnt[kSlots];
+  __shared__ unsigned long long s_best[kCcBlock / kWave];
+  for (int i = threadIdx.x; i < kSlots; i += blockDim.x) {
+    s_root[i] = -1;
+    s_cnt[i] = 0u;
+  }
+  __syncthreads();
   for (int i = threadIdx.x; i < kGiantSamples; i += blockDim.x) {
     const int v = static_cast<int>((static_cast<unsigned long long>(i) * 2654435761ull) % static_cast<unsigned>(nodes));
-    s_root[i] = find_root(parent, v);
+    const int r = find_root(parent, v);
+    int k = static_cast<int>((static_cast<unsigned>(r) * 2654435769u) % kSlots);
+    for (;;) {
+      const int old = atomicCAS(&s_root[k], -1, r);
+      if (old == -1 || old == r) break;
+      k = (k + 1) % kSlots;
+    }
+    atomicAdd(&s_cnt[k], 1u);
   }
   __syncthreads();
-  int best = INT_MAX, bcnt = 0;
-  for (int i = threadIdx.x; i < kGiantSamples; i += blockDim.x) {
-    int c = 0;
-    for (int j = 0; j < kGiantSamples; j++) c += s_root[j] == s_root[i];
-    if (c > bcnt || (c == bcnt && s_root[i] < best)) {
-      bcnt = c;
-      best = s_root[i];
-    }
+  unsigned long long best = 0;  // (count << 32) | ~root
+  for (int i = threadIdx.x; i < kSlots; i += blockDim.x) {
+    const unsigned long long key =
+        s_root[i] < 0 ? 0ull : (static_cast<unsigned long long>(s_cnt[i]) << 32) | ~static_cast<unsigned>(s_root[i]);
+    best = key > best ? key : best;
   }
-  s_best[threadIdx.x] = best;
-  s_cnt[threadIdx.x] = bcnt;
+  best = wave_max(best);
+  if (lane_id() == 0) s_best[threadIdx.x / kWave] = best;
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int t = 1; t < static_cast<int>(blockDim.x); t++)
-      if (s_cnt[t] > bcnt || (s_cnt[t] == bcnt && s_best[t] < best)) {
-        bcnt = s_cnt[t];
-        best = s_best[t];
-      }
-    st_relaxed(&ctl->giant, best);
+    for (int w = 1; w < kCcBlock / kWave; w++) best = s_best[w] > best ? s_best[w] : best;
+    st_relaxed(&ctl->giant, static_cast<int>(~static_cast<unsigned>(best & 0xffffffffull)));
   }
 }
 

@@ -186,6 +186,24 @@ def test_sssp_far_pile_spills(ig, orc, ctx):
             ctx.set_hint(ig._lib.HINT_SSSP_DELTA, 0)
 
 
+@pytest.mark.parametrize("degree", [1, 2, 4, 8, 16])
+def test_cc_large_trees_meet(ig, orc, ctx, degree):
+    """Random graphs whose lanes all join the same few roots: below and above
+    the average degree of the Afforest order, the edge form and a batch."""
+    g = ig.erdos_renyi(100003, 100003 * degree // 2, seed=degree)
+    dg = ig.DeviceGraph(g)
+    want = orc.cc(g)
+    for variant in (ig._lib.VARIANT_VERTEX, ig._lib.VARIANT_EDGE):
+        ctx.set_hint(ig._lib.HINT_VARIANT, variant)
+        try:
+            assert np.array_equal(ctx.cc(dg), want), variant
+        finally:
+            ctx.set_hint(ig._lib.HINT_VARIANT, 0)
+    q = ig.Query("cc", 0, dg)
+    ctx.batch([dg], [q])
+    assert np.array_equal(q.result(), want)
+
+
 def test_cc_catalog(ig, orc, ctx):
     for g in catalog(ig):
         assert np.array_equal(ctx.cc(ig.DeviceGraph(g)), orc.cc(g)), g.name
