@@ -42,7 +42,7 @@
 //                  one pass;
 //   1. out-select : N+ lists, order-preserving; lists < kMidDeg by the
 //                  in-wave balancer, longer ones binned into mid (one wave
-//                  each) and huge (kHugeChunk-entry items, one workgroup
+//                  each) and huge (kTcHugeChunk-entry items, one workgroup
 //                  each, compacted per item); also flags unsorted lists and
 //                  self loops; records (|N+|, hub number) per vertex and,
 //                  per CSR entry, one byte: does the neighbour outrank the
@@ -90,7 +90,15 @@ constexpr int kMidSlots = 8192;
 constexpr int kBigBlock = 1024;
 constexpr int kBigSlots = 32768;
 static_assert(kMidBlock == 512 && kMidSlots == 8192, "the main-kernel name below spells these out");
-static_assert(kHugeChunk % kTcBlock == 0, "tc_pack_huge moves whole items");
+// The selections' own bins: lists of kTcHugeDeg entries and more go in
+// kTcHugeChunk-entry items, one workgroup each, shorter ones one wave each.  The
+// frontier passes' 512-entry bins cost more packing than they balance (R-MAT 22
+// 10.40 ms a call); items from 4096 entries on left long lists to single waves:
+// R-MAT 22 / 20 / 18 / 14 9.97 / 2.49 / 0.82 / 0.283 ms, from 1024 on 9.85 / 2.35 /
+// 0.79 / 0.257 (1024-entry items: 9.96 / 2.38 / 0.79 / 0.247).
+constexpr int kTcHugeDeg = 1024;
+constexpr int kTcHugeChunk = 2048;
+static_assert(kTcHugeChunk % kTcBlock == 0, "tc_pack_huge moves whole items");
 // Probe bound of a wave-pass task: 2^13 below 2^24 CSR entries, else 2^14.
 // The workgroup passes take the rest; on small graphs their parallelism
 // beats the wave pass's per-task round trips (R-MAT 14-18: 0.38 -> 0.25,
@@ -338,7 +346,7 @@ __global__ __launch_bounds__(kTcBlock) IG_SGPR_CAP void tc_select(int nodes, con
     const int beg = valid ? nindex[v] : 0;
     const int dv = valid ? nindex[v + 1] - beg : 0;
     const bool long_list = dv >= kMidDeg;
-    if (kOut) frontier_emit_block(s_emit, long_list, v, dv, heavy, &ctl->heavy);
+    if (kOut) frontier_emit_block<kMidDeg, kTcHugeDeg, kTcHugeChunk>(s_emit, long_list, v, dv, heavy, &ctl->heavy);
     const bool mine = valid && !long_list;
     const int odv = mine ? sel.own_odeg(v) : 0;
     const int nar = mine && sel.narrow(v) ? 1 : 0;
@@ -386,7 +394,7 @@ __global__ __launch_bounds__(kTcBlock) IG_SGPR_CAP void tc_select(int nodes, con
 
 // Selection over the binned long lists.  Mid lists: one wave each, in order,
 // written at the list's own position and recorded.  Huge lists: one
-// workgroup per kHugeChunk-entry item, compacted in order at the item's own
+// workgroup per kTcHugeChunk-entry item, compacted in order at the item's own
 // position with the item's count in hcnt; tc_pack_huge then closes the gaps.
 template <bool kOut, typename Sel, typename Rec>
 __global__ __launch_bounds__(kTcBlock) IG_SGPR_CAP void tc_select_heavy(const int* __restrict__ nindex,
@@ -409,9 +417,9 @@ __global__ __launch_bounds__(kTcBlock) IG_SGPR_CAP void tc_select_heavy(const in
     const int dv = ve - vb;
     const int odv = sel.own_odeg(v);
     const bool nar = sel.narrow(v);
-    const int off = static_cast<int>(item - heavy.hoff[j]) * kHugeChunk;  // the item's first entry in the row
+    const int off = static_cast<int>(item - heavy.hoff[j]) * kTcHugeChunk;  // the item's first entry in the row
     const int beg = vb + off;
-    const int end = min(ve, beg + kHugeChunk);
+    const int end = min(ve, beg + kTcHugeChunk);
     int run = 0;
     for (int base = beg; base < end; base += kTcBlock) {
       const int e = base + static_cast<int>(threadIdx.x);
@@ -482,14 +490,14 @@ __global__ __launch_bounds__(kTcBlock) void tc_pack_huge(const int* __restrict__
                                                          FrontierQueues heavy, const int* __restrict__ hcnt, Sel sel,
                                                          Rec rec, const TcControl* ctl)
 {
-  constexpr int kPer = kHugeChunk / kTcBlock;
+  constexpr int kPer = kTcHugeChunk / kTcBlock;
   const unsigned nh = huge_count(ctl->heavy.hpack);
   for (unsigned j = blockIdx.x; j < nh; j += gridDim.x) {
     const int v = heavy.hq[j];
     const int vb = nindex[v], dv = nindex[v + 1] - vb;
     const bool nar = sel.narrow(v);
     const unsigned c0 = heavy.hoff[j];
-    const int nc = (dv + kHugeChunk - 1) / kHugeChunk;
+    const int nc = (dv + kTcHugeChunk - 1) / kTcHugeChunk;
     int run = 0;
     for (int c = 0; c < nc; c++) {
       const int k = hcnt[c0 + c];
@@ -497,10 +505,10 @@ __global__ __launch_bounds__(kTcBlock) void tc_pack_huge(const int* __restrict__
 #pragma unroll
       for (int q = 0; q < kPer; q++) {
         const int i = q * kTcBlock + static_cast<int>(threadIdx.x);
-        buf[q] = i < k ? row_get(list, vb, c * kHugeChunk + i, nar) : 0;
+        buf[q] = i < k ? row_get(list, vb, c * kTcHugeChunk + i, nar) : 0;
       }
       __syncthreads();
-      if (run != c * kHugeChunk) {
+      if (run != c * kTcHugeChunk) {
 #pragma unroll
         for (int q = 0; q < kPer; q++) {
           const int i = q * kTcBlock + static_cast<int>(threadIdx.x);
@@ -1137,7 +1145,7 @@ size_t part_words(int nodes, int edges)
 size_t hcnt_words(int edges)
 {
   const size_t e = static_cast<size_t>(edges);
-  return e / kHugeChunk + e / kHugeDeg + 2;
+  return e / kTcHugeChunk + e / kTcHugeDeg + 2;
 }
 
 }  // namespace
