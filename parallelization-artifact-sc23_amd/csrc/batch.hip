@@ -11,10 +11,11 @@
 // / 2^18 rounded up to a power of two: small graphs take one workgroup and
 // synchronise with __syncthreads only, large ones a gang with its own bounded
 // barrier.  Where that leaves workgroups of the grid without a task, the tasks
-// that would finish last take them (widen_gangs).  The cap depends on how much work a barrier separates: 256 for
-// the dense sweeps of PR, CC and MIS, 128 for BFS, 64 for SSSP's many short
-// rounds, and 16 for BFS on deep sparse graphs (average degree below 6),
-// whose thousands of levels are bound by barrier latency.  A free workgroup joins the first task in queue
+// that would finish last take them (widen_gangs).  The cap depends on how much
+// work a barrier separates: 256 for the dense sweeps of PR, CC and MIS, 128 for
+// BFS, 64 for SSSP's many short rounds (256 of idle workgroups), and 16 for BFS
+// on deep sparse graphs (average degree below 6), whose thousands of levels are
+// bound by barrier latency.  A free workgroup joins the first task in queue
 // order that still has a free slot (one atomic on the task's `joined`
 // counter); the gang starts when all k members have arrived.  Because every
 // workgroup is resident and gangs are filled strictly in queue order, a gang
@@ -48,10 +49,9 @@
 //         turns the next masks into the new frontier and writes the level
 //         into the slab rows of the new bits.  Deep graphs (grids, roads)
 //         cost their edge work plus two barriers per level.
-//   SSSP: Bellman-Ford driven by a queue of active vertices over a
-//         per-source distance slab, with per-vertex 32-bit active masks;
-//         relaxations by atomicMin, a vertex is queued for the next round
-//         when its distance for some source drops.
+//   SSSP: Bellman-Ford driven by a queue of active vertices over vertex-major
+//         rows of distances; relaxations by atomicMin, a vertex is queued for
+//         the next round when its distance for some source drops.
 //   CC  : union-find hooking the larger root under the smaller (labels =
 //         component minima), then flattening; graphs of average degree 8 or
 //         more link in Afforest order and skip the giant component's lists.
@@ -81,6 +81,7 @@
 
 #include "csum.hpp"
 #include "device_common.hpp"
+#include "emit.hpp"
 #include "unionfind.hpp"
 
 namespace indigo {
@@ -97,6 +98,7 @@ constexpr int kItem = 1024;      // entries per item
 constexpr int kCcSample = 2;      // CC: neighbours linked per vertex before the giant root is chosen
 constexpr int kCcSamples = 256;   // CC: vertices sampled to choose it
 constexpr int kCcAfforestMin = 4096;  // CC: smallest graph that takes the Afforest order
+constexpr int kSsspQueue = 1024;  // SSSP: appends that a workgroup buffers per round
 constexpr int kPrWaveList = 32;  // PR: lists walked by a whole wave
 constexpr float kDamp = 0.85f;
 
@@ -120,6 +122,7 @@ struct BatchTask {
   int* out;
   void* scratch;  // per algorithm, see scratch_bytes
   int2* items;    // heavy-list items (vertex, first entry)
+  int item;       // lists of this many entries or more are split into items of as many
   int nsrc;
   int src[INDIGO_MAX_BFS_SOURCES];
 };
@@ -199,6 +202,14 @@ IG_DEV void wave_lds_sync()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// SSSP: log2 of a vertex's distances in the vertex-major rows.
+__host__ __device__ inline int sssp_row_shift(int nsrc)
+{
+  int s = 0;
+  while ((1 << s) < nsrc) s++;
+  return s;
+}
+
 IG_DEV bool heavy(int deg) { return deg >= kHeavyDeg; }
 
 // Wave-collective: walks the CSR entries of the vertex `v` of each lane with
@@ -254,7 +265,7 @@ IG_DEV bool build_items(const BatchTask& T, const Team& tm, int* nitems)
     const int v = c * kWave + lane;
     const int b = v < T.nodes ? T.nindex[v] : 0;
     const int deg = v < T.nodes ? T.nindex[v + 1] - b : 0;
-    const int n = heavy(deg) ? (deg + kItem - 1) / kItem : 0;
+    const int n = deg >= T.item ? (deg + T.item - 1) / T.item : 0;
     const int incl = wave_inclusive_scan(n);
     const int total = wave_bcast(incl, kWave - 1);
     if (total == 0) continue;
@@ -264,7 +275,7 @@ IG_DEV bool build_items(const BatchTask& T, const Team& tm, int* nitems)
     for (int j = 0; j < n; j++) {
       const unsigned slot = base + static_cast<unsigned>(incl - n + j);
       st_relaxed(&T.items[slot].x, v);
-      st_relaxed(&T.items[slot].y, b + j * kItem);
+      st_relaxed(&T.items[slot].y, b + j * T.item);
     }
   }
   if (!team_sync(tm)) return false;
@@ -432,24 +443,139 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
 }
 
 // ---- multi-source SSSP -------------------------------------------------------
-IG_DEV bool run_sssp(const BatchTask& T, const Team& tm)
+// The distances live vertex-major, row[v * G + i] for source i (G = nsrc rounded up
+// to a power of two), beside the distances at which they were last expanded
+// (done): a queued vertex expands the sources whose distance is below that.  A
+// wave takes the (list entry, source) pairs of its vertices one per lane, all
+// sources of an entry in neighbouring lanes, so only active pairs cost anything
+// and an entry's distances are runs of consecutive words.  With a lane per entry
+// that walked its sources over source-major rows, every distance was a line of
+// its own and each source a chain of three round trips.  Batches of 512 and 24
+// graphs (16 sources each): 805 and 61 -> 376 and 5.7 ms; R-MAT 18 and 14 alone 12.0
+// and 9.1 -> 3.8 and 1.5.  (Deferring distances above a threshold that grows by
+// twice the mean weight over the degree a round saved relaxations but no time.)
+// Vertices with split lists (heavy; for SSSP the lists are split into short items,
+// each entry being nsrc pairs) have their active sources in masks instead, which
+// their items read.  The rows are turned into the output's source-major slab at
+// the end.
+
+// The n-th (from 0) set bit of m.
+IG_DEV int nth_bit(unsigned m, int n)
+{
+  int pos = 0;
+#pragma unroll
+  for (int half = 16; half > 0; half >>= 1) {
+    const int low = __popc(m & ((1u << half) - 1u));
+    if (n >= low) {
+      n -= low;
+      m >>= half;
+      pos += half;
+    }
+  }
+  return pos;
+}
+
+struct SsspRows {
+  int* row;         // [V << shift]
+  int* done;        // [V << shift]
+  unsigned* stamp;  // [V] last round for which the vertex was queued
+  unsigned* mask;   // heavy vertices: sources active in the next round
+  int shift;
+  unsigned round;  // the next round
+  int* qnext;
+  unsigned* ncount;
+};
+
+// Wave-collective: relaxes the pairs of each lane's list [beg, beg + len) of vertex v
+// and the sources in m.
+IG_DEV void relax_pairs(const BatchTask& T, const SsspRows& R, int v, int beg, int len, unsigned m,
+                        BlockQueue<kSsspQueue>& s_next)
+{
+  constexpr int kFly = 2;  // pairs in flight per lane
+  const int lane = lane_id();
+  const int pairs = len * __popc(m);  // (below 1024 * 32)
+  const int incl = wave_inclusive_scan(pairs);
+  const int total = wave_bcast(incl, kWave - 1);
+  for (int base = 0; base < total; base += kFly * kWave) {
+    int u[kFly], nd[kFly], start[kFly];
+    size_t at[kFly];
+    bool on[kFly];
+    unsigned bit[kFly];
+#pragma unroll
+    for (int q = 0; q < kFly; q++) {
+      const int k = base + q * kWave + lane;
+      on[q] = k < total;
+      const int o = min(wave_owner(incl, k), kWave - 1);
+      const unsigned om = static_cast<unsigned>(wave_shfl(static_cast<int>(m), o));
+      const int ov = wave_shfl(v, o), ob = wave_shfl(beg, o);
+      const unsigned rem = static_cast<unsigned>(k - wave_shfl(incl - pairs, o));
+      const unsigned pop = __popc(om);
+      const unsigned entry = on[q] ? rem / pop : 0u;
+      const int rank = static_cast<int>(rem - entry * pop);
+      const int i = nth_bit(om, rank);
+      const int e = on[q] ? ob + static_cast<int>(entry) : 0;
+      start[q] = lane - rank;  // (the lane of the entry's first pair, below 0 in the step before)
+      bit[q] = 1u << i;
+      at[q] = static_cast<size_t>(i);
+      u[q] = on[q] ? T.nlist[e] : 0;
+      nd[q] = on[q] ? T.eweight[e] + ld_relaxed(&R.row[(static_cast<size_t>(ov) << R.shift) + i]) : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < kFly; q++) {
+      at[q] += static_cast<size_t>(u[q]) << R.shift;
+      on[q] = on[q] && nd[q] < ld_relaxed(&R.row[at[q]]);
+    }
+#pragma unroll
+    for (int q = 0; q < kFly; q++) {
+      const unsigned long long all = __ballot(on[q]);
+      if (all == 0ull) continue;
+      bool first = false;
+      if (on[q]) {
+        // (whether or not this lane's minimum is the one that lowers the
+        // distance: one of this round does)
+        atomic_min_relaxed(&R.row[at[q]], nd[q]);
+        const unsigned queued = ld_relaxed(&R.stamp[u[q]]);
+        if (T.nindex[u[q] + 1] - T.nindex[u[q]] >= T.item)
+          __hip_atomic_fetch_or(&R.mask[u[q]], bit[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the first improving lane of the entry queues u
+        const unsigned long long run = all & ((1ull << lane) - 1ull) & (~0ull << max(start[q], 0));
+        first = run == 0ull && queued != R.round &&
+                __hip_atomic_exchange(&R.stamp[u[q]], R.round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != R.round;
+      }
+      bq_append(s_next, first, u[q], R.qnext, R.ncount);
+    }
+  }
+}
+
+IG_DEV bool run_sssp(const BatchTask& T, const Team& tm, BlockQueue<kSsspQueue>& s_next)
 {
   const int V = T.nodes;
   const int lane = lane_id();
   const size_t Vs = static_cast<size_t>(V);
   unsigned* base = static_cast<unsigned*>(T.scratch);
-  unsigned* act[3] = {base, base + Vs, base + 2 * Vs};  // active masks by round mod 3
+  unsigned* act[3] = {base, base + Vs, base + 2 * Vs};  // heavy vertices' masks by round mod 3
   int* queue[3] = {reinterpret_cast<int*>(base + 3 * Vs), reinterpret_cast<int*>(base + 4 * Vs),
                    reinterpret_cast<int*>(base + 5 * Vs)};
+  SsspRows R;
+  R.shift = sssp_row_shift(T.nsrc);
+  R.stamp = base + 6 * Vs;
+  R.row = reinterpret_cast<int*>(base + 7 * Vs);
+  R.done = R.row + (Vs << R.shift);
   unsigned* qn = tm.gs->qn;
   const Chunks ch = team_chunks(tm, V);
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
-    if (v >= V) continue;
-    st_relaxed(&act[0][v], 0u);
-    st_relaxed(&act[1][v], 0u);
-    st_relaxed(&act[2][v], 0u);
-    for (int i = 0; i < T.nsrc; i++) st_relaxed(&T.out[static_cast<size_t>(i) * V + v], INT_MAX);
+    if (v < V) {
+      st_relaxed(&act[0][v], 0u);
+      st_relaxed(&act[1][v], 0u);
+      st_relaxed(&act[2][v], 0u);
+      st_relaxed(&R.stamp[v], 0u);
+    }
+    const size_t end = min(Vs, static_cast<size_t>(c + 1) * kWave) << R.shift;
+    for (size_t k = (static_cast<size_t>(c) * kWave << R.shift) + lane; k < end; k += kWave) {
+      st_relaxed(&R.row[k], INT_MAX);
+      st_relaxed(&R.done[k], INT_MAX);
+    }
   }
   int nitems = 0;
   if (!build_items(T, tm, &nitems)) return false;
@@ -457,62 +583,82 @@ IG_DEV bool run_sssp(const BatchTask& T, const Team& tm)
     const bool has = lane < T.nsrc;
     const int i = lane;
     const int s = has ? T.src[i] : 0;
-    unsigned old = 0u;
+    unsigned old = 1u;
     if (has) {
-      st_relaxed(&T.out[static_cast<size_t>(i) * V + s], 0);
+      st_relaxed(&R.row[(static_cast<size_t>(s) << R.shift) + i], 0);
       old = __hip_atomic_fetch_or(&act[0][s], 1u << i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    wave_append(has && old == 0u, s, queue[0], &qn[0]);
+    wave_append(old == 0u, s, queue[0], &qn[0]);
   }
   if (!team_sync(tm)) return false;
+  const int G = 1 << R.shift;
+  const int eps = kWave >> R.shift;  // vertices per step of the mask pass
+  const unsigned group = G == 32 ? ~0u : (1u << G) - 1u;
   for (int r = 0;; r++) {
     const unsigned* cur = act[r % 3];
-    unsigned* nxt = act[(r + 1) % 3];
     unsigned* prev = act[(r + 2) % 3];  // round r-1's masks: cleared now
     const int* qcur = queue[r % 3];
-    int* qnext = queue[(r + 1) % 3];
     const int* qprev = queue[(r + 2) % 3];
-    unsigned* ncount = &qn[(r + 1) & 3];
+    R.mask = act[(r + 1) % 3];
+    R.qnext = queue[(r + 1) % 3];
+    R.ncount = &qn[(r + 1) & 3];
+    R.round = static_cast<unsigned>(r) + 1u;
     const int ncur = static_cast<int>(ld_relaxed(&qn[r & 3]));
-    const int nprev = r > 0 ? static_cast<int>(ld_relaxed(&qn[(r + 3) & 3])) : 0;
+    const int nprev = r > 0 && (nitems > 0 || r == 1) ? static_cast<int>(ld_relaxed(&qn[(r + 3) & 3])) : 0;
+    bq_reset(s_next);
     if (tm.rank == 0 && threadIdx.x == 0) st_relaxed(&qn[(r + 2) & 3], 0u);
     for (int k = tm.rank * kBatchBlock + static_cast<int>(threadIdx.x); k < nprev; k += tm.size * kBatchBlock)
       st_relaxed(&prev[ld_relaxed(&qprev[k])], 0u);
-    auto relax = [&](unsigned m, int v, int e, bool valid) {
-      bool first = false;
-      int u = 0;
-      if (valid) {
-        u = T.nlist[e];
-        const int w = T.eweight[e];
-        unsigned gained = 0u;
-        for (unsigned bits = m; bits != 0u; bits &= bits - 1u) {
-          const int i = __ffs(static_cast<int>(bits)) - 1;
-          const size_t row = static_cast<size_t>(i) * V;
-          const int nd = ld_relaxed(&T.out[row + v]) + w;
-          if (nd < ld_relaxed(&T.out[row + u]) && nd < atomic_min_relaxed(&T.out[row + u], nd)) gained |= 1u << i;
-        }
-        if (gained != 0u)
-          first = __hip_atomic_fetch_or(&nxt[u], gained, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u;
-      }
-      wave_append(first, u, qnext, ncount);
-    };
-    const int nq = (ncur + kWave - 1) / kWave;
-    for (int c = ch.first; c < nq; c += ch.step) {
-      const int k = c * kWave + lane;
-      const bool a = k < ncur;
+    // few queued vertices: fewer per wave
+    int per = kWave;
+    while (per > 4 && ncur <= per / 2 * ch.step) per /= 2;
+    for (int c = ch.first; c * per < ncur; c += ch.step) {
+      const int k = c * per + lane;
+      const bool a = lane < per && k < ncur;
       const int v = a ? ld_relaxed(&qcur[k]) : 0;
-      const unsigned m = a ? ld_relaxed(&cur[v]) : 0u;
-      wave_entries_of(v, a, T.nindex, [&](int o, int e, bool valid) {
-        relax(static_cast<unsigned>(__shfl(static_cast<int>(m), o, kWave)), __shfl(v, o, kWave), e, valid);
-      });
+      const int beg = a ? T.nindex[v] : 0;
+      const int deg = a ? T.nindex[v + 1] - beg : 0;
+      const int len = deg < T.item ? deg : 0;
+      // the sources whose distance fell since the vertex was last expanded
+      unsigned m = 0u;
+      for (int t = 0; t * eps < per; t++) {
+        const int from = t * eps + (lane >> R.shift);
+        const size_t x = (static_cast<size_t>(wave_shfl(v, from)) << R.shift) + (lane & (G - 1));
+        bool open = wave_shfl(len, from) > 0;
+        if (open) {
+          const int now = ld_relaxed(&R.row[x]);
+          open = now < ld_relaxed(&R.done[x]);
+          if (open) st_relaxed(&R.done[x], now);
+        }
+        const unsigned long long all = __ballot(open);
+        if (lane / eps == t) m = static_cast<unsigned>(all >> ((lane % eps) << R.shift)) & group;
+      }
+      relax_pairs(T, R, v, beg, len, m, s_next);
     }
-    for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
-      const unsigned m = ld_relaxed(&cur[v]);
-      if (m == 0u) return;
-      for (int e0 = eb; e0 < ee; e0 += kWave) relax(m, v, e0 + lane, e0 + lane < ee);
-    });
+    // items: 64 of the wave's checked at a time
+    const int run = T.item / kWave;  // entries per lane
+    for (int i0 = ch.first; i0 < nitems; i0 += kWave * ch.step) {
+      const int i = i0 + lane * ch.step;
+      const int v = i < nitems ? ld_relaxed(&T.items[i].x) : 0;
+      const int eb = i < nitems ? ld_relaxed(&T.items[i].y) : 0;
+      const unsigned m = i < nitems ? ld_relaxed(&cur[v]) : 0u;
+      for (unsigned long long left = __ballot(m != 0u); left != 0ull; left &= left - 1ull) {
+        const int from = __ffsll(static_cast<long long>(left)) - 1;
+        const int iv = wave_bcast(v, from), b = wave_bcast(eb, from) + lane * run;
+        const int end = min(wave_bcast(eb, from) + T.item, T.nindex[iv + 1]);
+        relax_pairs(T, R, iv, b, max(0, min(run, end - b)), static_cast<unsigned>(wave_bcast(static_cast<int>(m), from)),
+                    s_next);
+      }
+    }
+    bq_flush(s_next, R.qnext, R.ncount);
     if (!team_sync(tm)) return false;
-    if (ld_relaxed(ncount) == 0u) break;
+    if (ld_relaxed(R.ncount) == 0u) break;
+  }
+  for (int c = ch.first; c < ch.count; c += ch.step) {
+    const int v = c * kWave + lane;
+    if (v >= V) continue;
+    for (int i = 0; i < T.nsrc; i++)
+      T.out[static_cast<size_t>(i) * V + v] = ld_relaxed(&R.row[(static_cast<size_t>(v) << R.shift) + i]);
   }
   return true;
 }
@@ -820,7 +966,7 @@ IG_DEV bool run_pr(const BatchTask& T, const Team& tm, double* s_red)
   return true;
 }
 
-__global__ __launch_bounds__(kBatchBlock) IG_SGPR_CAP void batch_kernel(const BatchTask* __restrict__ tasks, int ntasks,
+__global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) IG_SGPR_CAP void batch_kernel(const BatchTask* __restrict__ tasks, int ntasks,
                                                             GangState* gangs, BatchControl* ctl, long long budget,
                                                             long long residency_ticks)
 {
@@ -828,6 +974,7 @@ __global__ __launch_bounds__(kBatchBlock) IG_SGPR_CAP void batch_kernel(const Ba
   __shared__ unsigned long long s_acc[kBatchWaves][kWave];
   __shared__ int s_flag[kBatchWaves][kWave];
   __shared__ double s_red[kBatchWaves];
+  __shared__ BlockQueue<kSsspQueue> s_next;
   if (!residency_barrier(&ctl->bar, residency_ticks)) return;
   const long long deadline = now_ticks() + budget;
   for (;;) {
@@ -857,7 +1004,7 @@ __global__ __launch_bounds__(kBatchBlock) IG_SGPR_CAP void batch_kernel(const Ba
     if (!team_sync(tm)) break;  // the gang assembles
     bool ok = true;
     if (T.alg == INDIGO_QUERY_BFS) ok = run_bfs(T, tm, s_acc);
-    else if (T.alg == INDIGO_QUERY_SSSP) ok = run_sssp(T, tm);
+    else if (T.alg == INDIGO_QUERY_SSSP) ok = run_sssp(T, tm, s_next);
     else if (T.alg == INDIGO_QUERY_CC) ok = run_cc(T, tm, s_acc);
     else if (T.alg == INDIGO_QUERY_PR) ok = run_pr(T, tm, s_red);
     else ok = run_mis(T, tm, s_flag);
@@ -865,31 +1012,40 @@ __global__ __launch_bounds__(kBatchBlock) IG_SGPR_CAP void batch_kernel(const Ba
   }
 }
 
-size_t items_cap(int edges) { return 2 * (static_cast<size_t>(edges) / kItem) + 2; }
+// Entries per item: lists that long tie a wave up.  An entry of a multi-source SSSP
+// is a pair per source, so its items hold about kItem pairs.
+int item_entries(int alg, int nsrc)
+{
+  return alg == INDIGO_QUERY_SSSP ? std::max(kWave, kItem >> sssp_row_shift(nsrc)) : kItem;
+}
+
+size_t items_cap(int edges, int item) { return 2 * (static_cast<size_t>(edges) / item) + 2; }
 
 // Per-task scratch: the algorithm's arrays (alg_bytes), then the heavy items.
-size_t alg_bytes(int alg, int nodes, int edges)
+size_t alg_bytes(int alg, int nodes, int edges, int nsrc)
 {
   const size_t v = static_cast<size_t>(nodes);
   size_t b = 0;
   if (alg == INDIGO_QUERY_BFS) b = 4 * v * 8 + 2 * v * 4;             // seen, 2 frontiers, next; 2 queues
-  else if (alg == INDIGO_QUERY_SSSP) b = 6 * v * 4;                  // 3 active masks, 3 queues
+  else if (alg == INDIGO_QUERY_SSSP) b = 7 * v * 4 + ((2 * v * 4) << sssp_row_shift(nsrc));  // 3 masks, 3 queues, stamps; rows
   else if (alg == INDIGO_QUERY_MIS) b = 2 * v * 4;                   // heavy-vertex flags
-  else if (alg == INDIGO_QUERY_PR) b = 2 * kMaxGang * 8 + 2 * v * 4 + items_cap(edges) * 8;  // slots, contrib, partials
+  else if (alg == INDIGO_QUERY_PR) b = 2 * kMaxGang * 8 + 2 * v * 4 + items_cap(edges, kItem) * 8;  // slots, contrib, partials
   return Carver::round(b);
 }
 
-size_t scratch_bytes(int alg, int nodes, int edges)
+size_t scratch_bytes(int alg, int nodes, int edges, int nsrc)
 {
-  return alg_bytes(alg, nodes, edges) + Carver::round(items_cap(edges) * sizeof(int2));
+  return alg_bytes(alg, nodes, edges, nsrc) + Carver::round(items_cap(edges, item_entries(alg, nsrc)) * sizeof(int2));
 }
 
 }  // namespace
 
-// Largest gang of an algorithm: how much work one of its barriers separates.
-static int gang_cap(int alg, int nodes, int edges)
+// Largest gang of an algorithm: how much work one of its barriers separates.  An
+// SSSP of many sources goes on gaining past 64 members, but only workgroups that
+// have nothing else to do take it there (widen_gangs).
+static int gang_cap(int alg, int nodes, int edges, bool widen)
 {
-  if (alg == INDIGO_QUERY_SSSP) return 64;
+  if (alg == INDIGO_QUERY_SSSP) return widen ? kMaxGang : 64;
   if (alg != INDIGO_QUERY_BFS) return kMaxGang;
   return static_cast<long long>(edges) < 6LL * nodes ? 16 : 128;
 }
@@ -898,7 +1054,7 @@ int batch_gang(int alg, int nodes, int edges)
 {
   if (alg < INDIGO_QUERY_BFS || alg > INDIGO_QUERY_PR || nodes < 0 || edges < 0) return 0;
   const long long entries = static_cast<long long>(edges) + nodes;
-  const int cap = gang_cap(alg, nodes, edges);
+  const int cap = gang_cap(alg, nodes, edges, false);
   int k = 1;
   while (k < cap && (static_cast<long long>(k) << kGangShift) < entries) k <<= 1;
   return k;
@@ -962,7 +1118,7 @@ void widen_gangs(std::vector<int>& gang, const indigo_graph_ref* graphs, const i
     const indigo_graph_ref& G = graphs[queries[q].graph];
     const long long entries = static_cast<long long>(G.edges) + G.nodes;
     const int k = gang[q];
-    if (2 * k > gang_cap(queries[q].alg, G.nodes, G.edges) || entries / (2 * k) < widen_floor(queries[q], G)) continue;
+    if (2 * k > gang_cap(queries[q].alg, G.nodes, G.edges, true) || entries / (2 * k) < widen_floor(queries[q], G)) continue;
     if (used + k > grid) continue;
     gang[q] = 2 * k;
     used += k;
@@ -1066,7 +1222,8 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
   widen_gangs(gang, graphs, queries, grid_cap);
   size_t scratch_total = 0;
   for (int q = 0; q < nqueries; q++)
-    scratch_total += scratch_bytes(queries[q].alg, graphs[queries[q].graph].nodes, graphs[queries[q].graph].edges);
+    scratch_total += scratch_bytes(queries[q].alg, graphs[queries[q].graph].nodes, graphs[queries[q].graph].edges,
+                                   queries[q].nsrc);
   const size_t n = static_cast<size_t>(nqueries);
   const size_t bytes = Carver::round(sizeof(BatchControl)) + Carver::round(n * sizeof(GangState)) +
                        Carver::round(n * sizeof(BatchTask)) + scratch_total + 4096;
@@ -1088,13 +1245,14 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
     T.gang = gang[order[i]];
     T.nodes = G.nodes;
     T.edges = G.edges;
+    T.item = item_entries(Q.alg, Q.nsrc);
     T.nindex = G.d_nindex;
     T.nlist = G.d_nlist;
     T.eweight = G.d_eweight;
     T.out = Q.d_out;
     T.scratch = scratch + off;
-    T.items = reinterpret_cast<int2*>(scratch + off + alg_bytes(Q.alg, G.nodes, G.edges));
-    off += scratch_bytes(Q.alg, G.nodes, G.edges);
+    T.items = reinterpret_cast<int2*>(scratch + off + alg_bytes(Q.alg, G.nodes, G.edges, Q.nsrc));
+    off += scratch_bytes(Q.alg, G.nodes, G.edges, Q.nsrc);
     T.nsrc = (Q.alg == INDIGO_QUERY_BFS || Q.alg == INDIGO_QUERY_SSSP) ? Q.nsrc : 0;
     for (int s = 0; s < T.nsrc; s++) T.src[s] = Q.src[s];
   }
@@ -1154,7 +1312,20 @@ int batch_wait(indigo_ctx* ctx)
 int batch_run(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, const indigo_query* queries,
               int nqueries, int max_workgroups)
 {
-  IG_TRY(batch_launch(ctx, graphs, ngraphs, queries, nqueries, max_workgroups));
+  const int rc = batch_launch(ctx, graphs, ngraphs, queries, nqueries, max_workgroups);
+  if (rc == INDIGO_ERR_OUT_OF_MEMORY && nqueries > 1) {
+    // the queries' scratch does not fit beside their outputs: half of them at a time
+    clear_error();
+    const int half = nqueries / 2;
+    IG_TRY(batch_run(ctx, graphs, ngraphs, queries, half, max_workgroups));
+    const float ms = ctx->last_ms;
+    IG_TRY(batch_run(ctx, graphs, ngraphs, queries + half, nqueries - half, max_workgroups));
+    ctx->last_ms += ms;
+    ctx->last_kernel_ms += ms;
+    ctx->last_iterations = nqueries;
+    return INDIGO_OK;
+  }
+  IG_TRY(rc);
   return batch_wait(ctx);
 }
 
