@@ -124,6 +124,17 @@ IG_DEV T wave_min(T x)
   return x;
 }
 
+// A worker's place in its next turn over vertices in id order, out of n workers
+// that each take one run of vertices a turn: it moves on by 4/9 of them.  On R-MAT
+// graphs a list's length goes with the set bits of its vertex id, so a worker
+// that kept its place, a multiple of a power of two vertices apart, would meet the
+// same kind of lists every turn.
+IG_DEV unsigned next_place(unsigned at, unsigned n)
+{
+  const unsigned move = n * 4u / 9u;
+  return at + move < n ? at + move : at + move - n;
+}
+
 // Appends `item` for every lane with `pred` to queue[] using one atomic per
 // wave on *counter; returns the slot (or -1).  Lanes that are inactive at the
 // call simply do not take part.

@@ -105,6 +105,54 @@ IG_DEV void exclude_neighbours_lane(const MisArgs& a, int v, int beg, int end)
   }
 }
 
+// The two together for a vertex per group of 1 << gs lanes (same v, beg, end in a
+// group; beg = end where there is none), four entries per lane in flight; all
+// lanes of the wave must be converged.  Returns the new state.
+IG_DEV int decide_group(const MisArgs& a, int v, int beg, int end, int gs)
+{
+  const unsigned long long kv = mis_key(v, a.flip);
+  const int lane = lane_id();
+  const int sub = lane & ((1 << gs) - 1);
+  const unsigned long long group = (gs == 6 ? ~0ull : (1ull << (1 << gs)) - 1ull) << (lane - sub);
+  int r = beg < end ? -1 : kIncluded;
+  for (int e0 = beg + sub; __ballot(r < 0) != 0ull; e0 += kMisLaneUnroll << gs) {
+    int su[kMisLaneUnroll];
+#pragma unroll
+    for (int q = 0; q < kMisLaneUnroll; q++) {
+      const int e = e0 + (q << gs);
+      const int u = r < 0 && e < end ? a.nlist[e] : v;
+      su[q] = u != v && mis_key(u, a.flip) > kv ? ld_relaxed(&a.status[u]) : kExcluded;
+    }
+    bool inc = false, hi = false;
+#pragma unroll
+    for (int q = 0; q < kMisLaneUnroll; q++) {
+      inc |= su[q] == kIncluded;
+      hi |= su[q] == kUndecided;
+    }
+    const unsigned long long incs = __ballot(inc) & group, his = __ballot(hi) & group;
+    if (r < 0) {
+      if (incs != 0ull) r = kExcluded;
+      else if (his != 0ull) r = kUndecided;
+      else if (e0 - sub + (kMisLaneUnroll << gs) >= end) r = kIncluded;
+    }
+  }
+  if (beg < end && r != kUndecided && sub == 0) st_relaxed(&a.status[v], r);
+  if (r == kIncluded) {
+    for (int e0 = beg + sub; e0 < end; e0 += kMisLaneUnroll << gs) {
+      int u[kMisLaneUnroll], su[kMisLaneUnroll];
+#pragma unroll
+      for (int q = 0; q < kMisLaneUnroll; q++) u[q] = e0 + (q << gs) < end ? a.nlist[e0 + (q << gs)] : v;
+#pragma unroll
+      for (int q = 0; q < kMisLaneUnroll; q++)
+        su[q] = u[q] != v && mis_key(u[q], a.flip) < kv ? ld_relaxed(&a.status[u[q]]) : kExcluded;
+#pragma unroll
+      for (int q = 0; q < kMisLaneUnroll; q++)
+        if (su[q] == kUndecided) st_relaxed(&a.status[u[q]], kExcluded);
+    }
+  }
+  return r;
+}
+
 // Whole wave decides vertex v (long list), 4 x 64 entries per step; all
 // lanes must be converged.
 IG_DEV int decide_wave(const MisArgs& a, int v, int beg, int end)
@@ -134,14 +182,20 @@ IG_DEV int decide_wave(const MisArgs& a, int v, int beg, int end)
 IG_DEV void exclude_neighbours_wave(const MisArgs& a, int v, int beg, int end)
 {
   const unsigned long long kv = mis_key(v, a.flip);
-  for (int e = beg + lane_id(); e < end; e += kWave) {
-    const int u = a.nlist[e];
-    if (u != v && mis_key(u, a.flip) < kv && ld_relaxed(&a.status[u]) == kUndecided)  // as exclude_neighbours_lane
-      st_relaxed(&a.status[u], kExcluded);
+  for (int base = beg + lane_id(); base < end; base += 4 * kWave) {
+    int u[4], su[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) u[q] = base + q * kWave < end ? a.nlist[base + q * kWave] : v;
+#pragma unroll
+    for (int q = 0; q < 4; q++)  // as exclude_neighbours_lane
+      su[q] = u[q] != v && mis_key(u[q], a.flip) < kv ? ld_relaxed(&a.status[u[q]]) : kExcluded;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (su[q] == kUndecided) st_relaxed(&a.status[u[q]], kExcluded);
   }
 }
 
-__global__ __launch_bounds__(kMisBlock) IG_SGPR_CAP void mis_kernel(MisArgs a)
+__global__ __launch_bounds__(kMisBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) IG_SGPR_CAP void mis_kernel(MisArgs a)
 {
   __shared__ BlockQueue<4096> s_wl;
   __shared__ BlockQueue<1024> s_hwl;
@@ -187,16 +241,25 @@ __global__ __launch_bounds__(kMisBlock) IG_SGPR_CAP void mis_kernel(MisArgs a)
     int* hout = a.hwl[(r + 1) & 1];
     bq_reset(s_wl);
     bq_reset(s_hwl);
-    // short lists: one lane each
-    for (unsigned base = blockIdx.x * blockDim.x; base < n; base += stride) {
-      const unsigned idx = base + threadIdx.x;
+    // short lists: one lane each, or, while there are fewer of them than lanes,
+    // a group of lanes each.  A lane alone takes up to 16 steps of two round
+    // trips to decide and 63 to exclude, which made every round 30 to 50 us long
+    // even for a dozen vertices (R-MAT 12 and 16 0.26 and 0.31 ms a call, now
+    // 0.11 and 0.17; a byte per state instead of a word, for the gathers' sake, was
+    // 10% slower: its lines are written more often).
+    int gs = 0;
+    while (gs < 6 && (static_cast<unsigned long long>(n) << (gs + 1)) <= static_cast<unsigned long long>(stride)) gs++;
+    for (unsigned base = 0, at = blockIdx.x; base < n; base += stride >> gs, at = next_place(at, gridDim.x)) {
+      const unsigned idx = base + ((at * blockDim.x + threadIdx.x) >> gs);
       bool keep = false;
-      int v = 0;
+      int v = 0, beg = 0, end = 0;
       if (idx < n) {
         v = (r == 0) ? static_cast<int>(idx) : ld_relaxed(&in[idx]);
         if (ld_relaxed(&a.status[v]) == kUndecided) {
-          const int beg = a.nindex[v], end = a.nindex[v + 1];
-          if (end - beg < kMidDeg) {
+          beg = a.nindex[v];
+          end = a.nindex[v + 1];
+          if (end - beg >= kMidDeg) end = beg = -1;
+          else if (beg == end || gs == 0) {
             const int st = decide_lane(a, v, beg, end);
             if (st == kIncluded) {
               st_relaxed(&a.status[v], kIncluded);
@@ -209,6 +272,7 @@ __global__ __launch_bounds__(kMisBlock) IG_SGPR_CAP void mis_kernel(MisArgs a)
           }
         }
       }
+      if (gs > 0) keep = decide_group(a, v, beg, end, gs) == kUndecided && (lane & ((1 << gs) - 1)) == 0;
       bq_append(s_wl, keep, v, out, &oc->n);
     }
     // long lists: one wave each

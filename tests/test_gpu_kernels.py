@@ -204,6 +204,21 @@ def test_cc_large_trees_meet(ig, orc, ctx, degree):
     assert np.array_equal(q.result(), want)
 
 
+@pytest.mark.parametrize("signed", [False, True])
+@pytest.mark.parametrize("workgroups", [0, 3, 40])
+@pytest.mark.parametrize("nodes", [2, 63, 1000, 20483, 70001])
+def test_mis_lane_groups(ig, orc, ctx, nodes, workgroups, signed):
+    """Worklists from a few vertices, 64 lanes each, to more vertices than the
+    grid has lanes (40 workgroups: 20480), on degrees around the group steps."""
+    ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, workgroups)
+    try:
+        for degree in (1, 6, 30, 63):
+            g = ig.erdos_renyi(nodes, nodes * degree // 2, seed=degree)
+            assert np.array_equal(ctx.mis(ig.DeviceGraph(g), signed), orc.mis(g, signed)), degree
+    finally:
+        ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, 0)
+
+
 def test_cc_catalog(ig, orc, ctx):
     for g in catalog(ig):
         assert np.array_equal(ctx.cc(ig.DeviceGraph(g)), orc.cc(g)), g.name
