@@ -174,7 +174,7 @@ int cc_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const in
   return INDIGO_OK;
 }
 
-int mis_device(indigo_ctx* ctx, int nodes, const int* nindex, const int* nlist, int signed_priority, int* status,
+int mis_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* nlist, int signed_priority, int* status,
                double* seconds)
 {
   IG_TRY(ensure_workspace(ctx, mis_workspace_bytes(nodes)));
@@ -184,7 +184,7 @@ int mis_device(indigo_ctx* ctx, int nodes, const int* nindex, const int* nlist, 
   int rounds = 0;
   for (;;) {
     IG_TRY(timing_begin(ctx));
-    IG_TRY(mis_run(ctx, nodes, nindex, nlist, signed_priority, status));
+    IG_TRY(mis_run(ctx, nodes, edges, nindex, nlist, signed_priority, status));
     IG_TRY(timing_end(ctx, 2, 0));
     const int rc = mis_collect(ctx, &rounds);
     if (rc != kNotResident) IG_TRY(rc);
@@ -396,7 +396,7 @@ int indigo_mis(indigo_ctx* ctx, int nodes, int edges, const int* d_nindex, const
   if (edge_variant(ctx))
     return edge_device(ctx, kEdgeMis, nodes, edges, d_nindex, d_nlist, nullptr, nullptr, 0, signed_priority, d_status,
                        nullptr);
-  return mis_device(ctx, nodes, d_nindex, d_nlist, signed_priority, d_status, nullptr);
+  return mis_device(ctx, nodes, edges, d_nindex, d_nlist, signed_priority, d_status, nullptr);
 }
 
 int indigo_mis_vertex(int nodes, int edges, const int* d_nindex, const int* d_nlist, int signed_priority,
@@ -408,7 +408,7 @@ int indigo_mis_vertex(int nodes, int edges, const int* d_nindex, const int* d_nl
   if (h_status == nullptr) return set_error(INDIGO_ERR_INVALID_ARG, "mis_vertex: status is NULL");
   DeviceBuffer d;
   IG_TRY(d.alloc(sizeof(int) * static_cast<size_t>(nodes)));
-  IG_TRY(mis_device(ctx, nodes, d_nindex, d_nlist, signed_priority, d.as<int>(), seconds));
+  IG_TRY(mis_device(ctx, nodes, edges, d_nindex, d_nlist, signed_priority, d.as<int>(), seconds));
   IG_HIP_TRY(hipMemcpy(h_status, d.p, sizeof(int) * static_cast<size_t>(nodes), hipMemcpyDeviceToHost));
   if (h_priority != nullptr)
     for (int v = 0; v < nodes; v++) h_priority[v] = mis_hash(static_cast<unsigned>(v) + 712313887u);

@@ -11,6 +11,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 
 namespace indigo {
 
@@ -24,6 +25,17 @@ inline int plan_per_cu(int occupancy, int block, int max_threads_per_cu, bool fu
   int n = std::max(occupancy, 0);
   if (!full_cu && n > 1 && static_cast<long long>(n) * block >= max_threads_per_cu) n -= 1;
   return n;
+}
+
+// Workgroups of a call on a graph of `edges` entries: the power of two nearest
+// per_root * sqrt(edges), at least 64.  A small graph's barriers cost more than its
+// lists.
+inline int graph_grid(int edges, double per_root)
+{
+  const double want = per_root * std::sqrt(static_cast<double>(edges));
+  int cap = 64;
+  while (cap < 4096 && cap * 1.41421356 < want) cap *= 2;
+  return cap;
 }
 
 struct GridLimits {

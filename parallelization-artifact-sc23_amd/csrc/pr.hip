@@ -28,7 +28,6 @@
 // decision (no floating-point atomics).
 #include "pr.hpp"
 
-#include <cmath>
 #include <map>
 #include <string>
 #include <vector>
@@ -399,19 +398,11 @@ size_t pr_workspace_bytes(int nodes, int edges)
          Carver::round(4 * kPrMaxGrid * 8) + Carver::round(kPrMaxGrid * 4) + Carver::round(kPrMaxGrid * 8) + 4096;
 }
 
-// Grid of one call: a sweep's barrier and combine cost more than a small
-// graph's gathers, so the grid grows with the graph, as the power of two
-// nearest 0.2 * sqrt(E) workgroups, at least 64.  Measured on R-MAT 12, 14, 16
-// and 18 (0.1M to 7.6M entries) the best caps were 64, 128, 256 and 512
-// (calls 0.31 -> 0.15, 0.35 -> 0.19, 0.45 -> 0.31 and 0.69 -> 0.64 ms); from
-// about 2^25 entries on the rule exceeds the resident grid, which is kept.
-static int pr_grid_cap(int edges)
-{
-  const double want = 0.2 * std::sqrt(static_cast<double>(edges));
-  int cap = 64;
-  while (cap < kPrMaxGrid && cap * 1.41421356 < want) cap *= 2;
-  return cap;
-}
+// Workgroups of one call, per square root of the entries.  Measured on R-MAT 12, 14,
+// 16 and 18 (0.1M to 7.6M entries) the best caps were 64, 128, 256 and 512 (calls
+// 0.31 -> 0.15, 0.35 -> 0.19, 0.45 -> 0.31 and 0.69 -> 0.64 ms); from about 2^25
+// entries on the rule exceeds the resident grid, which is kept.
+constexpr double kPrGridPerRoot = 0.2;
 
 int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* nlist, const int* degree,
            float* scores, int init_uniform)
@@ -447,7 +438,7 @@ int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   IG_TRY(zero_async(ctx, a.ctl, sizeof(PrControl)));
   IG_TRY(zero_async(ctx, a.exit_it, sizeof(int) * kPrMaxGrid));
   void* args[] = {&a};
-  IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(pr_kernel), kPrBlock, 0, args, pr_grid_cap(edges), nullptr,
+  IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(pr_kernel), kPrBlock, 0, args, graph_grid(edges, kPrGridPerRoot), nullptr,
                      "pr_kernel"));
   return INDIGO_OK;
 }
