@@ -1284,15 +1284,17 @@ int batch_wait(indigo_ctx* ctx)
   if (!ctx->pending_batch.active) return set_error(INDIGO_ERR_INVALID_ARG, "batch: nothing in flight");
   for (;;) {
     const int ntasks = ctx->pending_batch.ntasks;
+    if (ntasks > 0) {
+      BatchControl* ctl = static_cast<BatchControl*>(ctx->pending_batch.ctl);
+      IG_HIP_TRY(hipMemcpyAsync(ctx->host_pinned, &ctl->bar.abort.v, sizeof(unsigned), hipMemcpyDeviceToHost,
+                                ctx->stream));
+      IG_HIP_TRY(hipStreamSynchronize(ctx->stream));
+    }
     const int rc0 = timing_finish(ctx, 3, ntasks);
     if (rc0 != INDIGO_OK || ntasks == 0) {
       ctx->pending_batch.active = false;
       return rc0;
     }
-    BatchControl* ctl = static_cast<BatchControl*>(ctx->pending_batch.ctl);
-    IG_HIP_TRY(hipMemcpyAsync(ctx->host_pinned, &ctl->bar.abort.v, sizeof(unsigned), hipMemcpyDeviceToHost,
-                              ctx->stream));
-    IG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     const unsigned abort_code = *static_cast<unsigned*>(ctx->host_pinned);
     const int rc = check_abort(ctx, reinterpret_cast<const void*>(batch_kernel), abort_code, "batch");
     if (rc != kNotResident) {

@@ -95,11 +95,12 @@ int bfs_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const i
   for (;;) {
     IG_TRY(timing_begin(ctx));
     IG_TRY(bfs_run(ctx, nodes, edges, nindex, nlist, src, dist, &st));
-    IG_TRY(timing_end(ctx, st.launches, 0));
+    IG_TRY(timing_record_stop(ctx));
     const int rc = bfs_collect(ctx, &st);
     if (rc != kNotResident) IG_TRY(rc);
     if (rc == INDIGO_OK) break;
   }
+  IG_TRY(timing_finish(ctx, st.launches, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = st.levels;
   return INDIGO_OK;
@@ -118,11 +119,12 @@ int sssp_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const 
   for (;;) {
     IG_TRY(timing_begin(ctx));
     IG_TRY(sssp_run(ctx, nodes, edges, nindex, nlist, eweight, src, dist));
-    IG_TRY(timing_end(ctx, 2, 0));
+    IG_TRY(timing_record_stop(ctx));
     const int rc = sssp_collect(ctx, &iters, &epochs);
     if (rc != kNotResident) IG_TRY(rc);
     if (rc == INDIGO_OK) break;
   }
+  IG_TRY(timing_finish(ctx, 2, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = iters;
   return INDIGO_OK;
@@ -185,11 +187,12 @@ int mis_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const i
   for (;;) {
     IG_TRY(timing_begin(ctx));
     IG_TRY(mis_run(ctx, nodes, edges, nindex, nlist, signed_priority, status));
-    IG_TRY(timing_end(ctx, 2, 0));
+    IG_TRY(timing_record_stop(ctx));
     const int rc = mis_collect(ctx, &rounds);
     if (rc != kNotResident) IG_TRY(rc);
     if (rc == INDIGO_OK) break;
   }
+  IG_TRY(timing_finish(ctx, 2, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = rounds;
   return INDIGO_OK;
@@ -206,11 +209,12 @@ int pr_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const in
   for (;;) {
     IG_TRY(timing_begin(ctx));
     IG_TRY(pr_run(ctx, nodes, edges, nindex, nlist, degree, scores, init_uniform));
-    IG_TRY(timing_end(ctx, 2, 0));
+    IG_TRY(timing_record_stop(ctx));
     const int rc = pr_collect(ctx, &iters, nullptr);
     if (rc != kNotResident) IG_TRY(rc);
     if (rc == INDIGO_OK) break;
   }
+  IG_TRY(timing_finish(ctx, 2, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = iters;
   if (iterations) *iterations = iters;
@@ -227,8 +231,9 @@ int tc_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const in
   IG_TRY(timing_begin(ctx));
   SeqArgs a{nodes, edges, nindex, nlist, nullptr, 10};
   IG_TRY(run_captured(ctx, seq_key(ctx, 6, a), tc_sequence, &a));
-  IG_TRY(timing_end(ctx, a.launches, 1));
+  IG_TRY(timing_record_stop(ctx));
   IG_TRY(tc_collect(ctx, count));
+  IG_TRY(timing_finish(ctx, a.launches, 1));
   if (seconds) *seconds = wall_seconds() - t0;
   return INDIGO_OK;
 }

@@ -274,11 +274,13 @@ int edge_device(indigo_ctx* ctx, int alg, int nodes, int edges, const int* ninde
                signed_priority ? 0x80000000u : 0u, out, aux, ctl, budget_ticks(ctx), residency_ticks(ctx)};
     void* args[] = {&a};
     IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(k), block, 0, args, 0, nullptr, kernel_name(alg)));
+    IG_TRY(timing_record_stop(ctx));
     IG_HIP_TRY(hipMemcpyAsync(ctx->host_pinned, &ctl->bar.abort.v, sizeof(unsigned), hipMemcpyDeviceToHost,
                               ctx->stream));
     IG_HIP_TRY(hipMemcpyAsync(static_cast<unsigned*>(ctx->host_pinned) + 1, &ctl->sweeps.v, sizeof(unsigned),
                               hipMemcpyDeviceToHost, ctx->stream));
-    IG_TRY(timing_end(ctx, own_sp != nullptr ? 3 : 2, 0));
+    IG_HIP_TRY(hipStreamSynchronize(ctx->stream));
+    IG_TRY(timing_finish(ctx, own_sp != nullptr ? 3 : 2, 0));
     const unsigned* h = static_cast<const unsigned*>(ctx->host_pinned);
     const int rc = check_abort(ctx, reinterpret_cast<const void*>(k), h[0], kernel_name(alg));
     if (rc == INDIGO_OK) {

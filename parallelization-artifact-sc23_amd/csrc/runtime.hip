@@ -128,7 +128,7 @@ int coop_launch(indigo_ctx* ctx, const void* kernel, int block, size_t shmem, vo
   const int grid = plan_grid(per_cu, lim);
   if (name != nullptr) IG_TRY(kernel_begin(ctx, name));
   IG_HIP_TRY(hipLaunchKernel(kernel, dim3(grid), dim3(block), args, static_cast<unsigned>(shmem), ctx->stream));
-  if (name != nullptr) IG_TRY(kernel_end(ctx));
+  ctx->kernel_to_stop = name != nullptr && !ctx->capturing;
   ctx->last_grid = grid;
   ctx->last_per_cu = lim.hint_blocks_per_cu > 0 ? std::min(per_cu, lim.hint_blocks_per_cu) : per_cu;
   if (grid_out) *grid_out = grid;
@@ -178,6 +178,7 @@ int check_graph_args(int nodes, int edges, const void* nindex, const void* nlist
 int timing_begin(indigo_ctx* ctx)
 {
   ctx->kernel_name = nullptr;
+  ctx->kernel_to_stop = false;
   IG_HIP_TRY(hipEventRecord(ctx->ev_start, ctx->stream));
   return INDIGO_OK;
 }
@@ -211,7 +212,7 @@ int timing_finish(indigo_ctx* ctx, int launches, int iterations)
   ctx->last_ms = ms;
   if (ctx->kernel_name != nullptr) {
     float kms = 0.f;
-    IG_HIP_TRY(hipEventElapsedTime(&kms, ctx->ev_k0, ctx->ev_k1));
+    IG_HIP_TRY(hipEventElapsedTime(&kms, ctx->ev_k0, ctx->kernel_to_stop ? ctx->ev_stop : ctx->ev_k1));
     ctx->last_kernel_ms = kms;
     ctx->last_kernel = ctx->kernel_name;
   } else {

@@ -24,6 +24,7 @@ struct indigo_ctx {
   // events around the main kernel launch of the last call (indigo_ctx_last_kernel)
   hipEvent_t ev_k0 = nullptr, ev_k1 = nullptr;
   const char* kernel_name = nullptr;  // set by kernel_begin, a string literal
+  bool kernel_to_stop = false;        // the kernel is the call's last: it ends at ev_stop
   float last_kernel_ms = 0.f;
   const char* last_kernel = "";
   void* ws = nullptr;      // cached device workspace
@@ -138,7 +139,8 @@ inline long long budget_ticks(const indigo_ctx* ctx)
 // (A cooperative launch would add nothing, and on ROCm it fails while
 // another process holds a context on the same GPU.)
 // `name` (a string literal, or null) marks the launch as the call's main
-// kernel, timed by kernel_begin / kernel_end.  full_cu: the kernel is held
+// kernel, timed from kernel_begin to the call's stop event (a mark of its own after
+// it would cost another event): nothing but that event may follow.  full_cu: the kernel is held
 // to 80 scalar registers (IG_SGPR_CAP) and may fill every wave slot of a CU.
 int coop_launch(indigo_ctx* ctx, const void* kernel, int block, size_t shmem, void** args, int max_blocks,
                 int* grid_out, const char* name = nullptr, bool full_cu = false);
