@@ -52,9 +52,16 @@ constexpr float kDamp = 0.85f;
 constexpr int kPrMaxGrid = 4096;
 constexpr int kPrUnroll = 4;  // gathers in flight per lane
 
+// Lists of kPrWaveDeg entries up to kPrHugeDeg by length: class c holds those of
+// kPrWaveDeg << c entries up to twice as many.
+constexpr int kPrClasses = 6;
+static_assert(kPrWaveDeg << kPrClasses == kPrHugeDeg, "the classes cover the lists between short and huge");
+constexpr int kPrClassCap = 512;  // lists of a class that a workgroup buffers while collecting
+
 struct PrControl {
   GridBarrier bar;
   FrontierCounters heavy;
+  PaddedU32 nclass[kPrClasses];
   int iterations;
   int status;
   double last_diff;
@@ -76,7 +83,8 @@ struct PrArgs {
   const int* __restrict__ degree;  // optional caller-provided degrees (PR_GPU contract)
   float* scores;
   float* contrib[2];
-  FrontierQueues heavy;  // lists of >= kPrWaveDeg entries (mid) and >= kPrHugeDeg (huge)
+  int* mid[kPrClasses];  // lists of kPrWaveDeg entries and more, by class
+  FrontierQueues heavy;  // lists of kPrHugeDeg entries and more (huge)
   float2* hpart;         // per huge item: compensated partial (sum, error)
   int hcap;              // huge vertices at most: edges / kPrHugeDeg + 1
   unsigned* hdone;       // per huge vertex: items finished this sweep
@@ -227,7 +235,9 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
   __shared__ float s_ps[kPrBlock / kWave], s_pc[kPrBlock / kWave];
   __shared__ int s_owner;
   __shared__ int s_last;
-  __shared__ HeavyCollector s_emit;
+  __shared__ FrontierEmitterT<64, 64, 64> s_emit;
+  __shared__ BlockQueue<kPrClassCap> s_class[kPrClasses];
+  __shared__ unsigned s_nclass[kPrClasses];
   PrControl* ctl = a.ctl;
   if (!residency_barrier(&ctl->bar, a.start_ticks)) return;
   const long long deadline = now_ticks() + a.budget;
@@ -238,6 +248,15 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
   const float inv_n = 1.0f / static_cast<float>(a.nodes);
   const float base = (1.0f - kDamp) / static_cast<float>(a.nodes);
 
+  const int wave = static_cast<int>(blockIdx.x) * wpb + static_cast<int>(threadIdx.x) / kWave;
+  const int nwaves = static_cast<int>(gridDim.x) * wpb;
+  // A wave's place among the waves moves on by about 4/9 of them a turn.  On R-MAT
+  // graphs a list's length goes with the set bits of its vertex id, so a wave that
+  // kept its place, a multiple of 2^11 vertices apart, met the same kind of
+  // lists every turn (R-MAT 22: 7.06 ms a call, 6.6 with the moves).
+  const int move = (nwaves * 4 / 9) & ~(wpb - 1);
+  auto next_turn = [&](int at) { return at + move < nwaves ? at + move : at + move - nwaves; };
+
   if (tid == 0) ctl->trace.start = now_ticks();
   for (int v = tid; v < a.nodes; v += stride) {
     const float s = a.init_uniform ? inv_n : a.scores[v];
@@ -246,7 +265,19 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
   }
   for (int j = tid; j < a.hcap; j += stride) st_relaxed(&a.hdone[j], 0u);
   trace_level(&ctl->trace, 0, 0u, 0ull, 0);
-  collect_heavy<kPrWaveDeg, kPrHugeDeg, kPrHugeChunk>(s_emit, a.nodes, a.nindex, a.heavy, &ctl->heavy);
+  fe_reset(s_emit);
+  for (int c = 0; c < kPrClasses; c++) bq_reset(s_class[c]);
+  const int runs = a.nodes / kWave + (a.nodes % kWave != 0 ? 1 : 0);
+  for (int w0 = 0, at = wave; w0 < runs; w0 += nwaves, at = next_turn(at)) {
+    const int v = (w0 + at) * kWave + lane;
+    const int deg = w0 + at < runs && v < a.nodes ? a.nindex[v + 1] - a.nindex[v] : 0;
+    if (__ballot(deg >= kPrWaveDeg) == 0ull) continue;
+    for (int c = 0; c < kPrClasses; c++)
+      bq_append(s_class[c], deg >= kPrWaveDeg << c && deg < kPrWaveDeg << (c + 1), v, a.mid[c], &ctl->nclass[c].v);
+    frontier_emit_block<kPrHugeDeg, kPrHugeDeg, kPrHugeChunk>(s_emit, deg >= kPrHugeDeg, v, deg, a.heavy, &ctl->heavy);
+  }
+  for (int c = 0; c < kPrClasses; c++) bq_flush(s_class[c], a.mid[c], &ctl->nclass[c].v);
+  fe_flush(s_emit, a.heavy, &ctl->heavy);
   trace_level(&ctl->trace, 1, 0u, 0ull, 1);
   if (!grid_barrier(&ctl->bar, deadline)) {
     if (tid == 0) ctl->status = 1;
@@ -254,26 +285,30 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
     return;
   }
   trace_level(&ctl->trace, 2, 0u, 0ull, 2);
-  const unsigned nm = ld_relaxed(&ctl->heavy.nm);
+  if (threadIdx.x < kPrClasses) s_nclass[threadIdx.x] = ld_relaxed(&ctl->nclass[threadIdx.x].v);
+  __syncthreads();
   const unsigned long long hp = ld_relaxed(&ctl->heavy.hpack);
   const unsigned nh = huge_count(hp), nch = huge_chunks(hp);
 
+  // mid lists, the longest first, are dealt to the workgroups in turn, and to
+  // their waves in turn: by class, the shares differ by less than a list of each
+  // (unsorted, the workgroups finished a sweep of R-MAT 22 after 660 to 910 us).
+  // This wave's first list is number rest0 of class c0.
+  auto next_list = [&](unsigned& c, unsigned& rest) {
+    while (c > 0 && rest >= s_nclass[c]) rest -= s_nclass[c--];
+    return rest < s_nclass[c];
+  };
+  unsigned c0 = kPrClasses - 1;
+  unsigned rest0 = threadIdx.x / kWave * gridDim.x + blockIdx.x;
+  const bool has_mid = next_list(c0, rest0);
   // short lists: vertices per wave and turn (fewer while waves are free,
   // where lists average enough entries for the groups)
-  const int wave = static_cast<int>(blockIdx.x) * wpb + static_cast<int>(threadIdx.x) / kWave;
-  const int nwaves = static_cast<int>(gridDim.x) * wpb;
   int per = kWave;
   const bool dense = a.nindex[a.nodes] >= kPrLaneDeg * static_cast<long long>(a.nodes);
   const int least = dense ? kWave / kPrGroup : kWave;
   while (per > least && (a.nodes + per / 2 - 1) / (per / 2) <= nwaves) per /= 2;
   const int chunks = (a.nodes + per - 1) / per;
   const bool few = per <= kWave / kPrGroup;
-  // A wave's place among the waves moves on by about 4/9 of them a turn.  On R-MAT
-  // graphs a list's length goes with the set bits of its vertex id, so a wave that
-  // kept its place, a multiple of 2^11 vertices apart, met the same kind of
-  // lists every turn (R-MAT 22: 7.06 ms a call, 6.6 with the moves).
-  const int move = (nwaves * 4 / 9) & ~(wpb - 1);
-  auto next_turn = [&](int at) { return at + move < nwaves ? at + move : at + move - nwaves; };
 
   int it = 0;
   for (;;) {
@@ -326,10 +361,9 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
     }
     trace_level(&ctl->trace, tl + 1, static_cast<unsigned>(it), 0ull, 1);
     // phase A: mid lists, one wave each
-    for (unsigned i0 = 0, at = wave; i0 < nm; i0 += nwaves, at = next_turn(at)) {
-      const unsigned i = i0 + at;
-      if (i >= nm) continue;
-      const int v = a.heavy.mq[i];
+    unsigned c = c0, rest = rest0;
+    for (bool more = has_mid; more; rest += nwaves, more = next_list(c, rest)) {
+      const int v = a.mid[c][rest];
       const int beg = a.nindex[v], end = a.nindex[v + 1];
       const float old = a.scores[v];
       CSum acc;
@@ -390,10 +424,15 @@ static size_t pr_max_chunks(int edges)
   return static_cast<size_t>(edges) / kPrHugeChunk + static_cast<size_t>(edges) / kPrHugeDeg + 2;
 }
 
+// Lists of class c at most.
+static size_t pr_class_cap(int edges, int c) { return static_cast<size_t>(edges) / (kPrWaveDeg << c) + 1; }
+
 size_t pr_workspace_bytes(int nodes, int edges)
 {
   const size_t v = static_cast<size_t>(nodes);
-  return Carver::round(sizeof(PrControl)) + 6 * Carver::round(v * 4) + Carver::round(pr_max_chunks(edges) * 8) +
+  size_t mid = 0;
+  for (int c = 0; c < kPrClasses; c++) mid += Carver::round(pr_class_cap(edges, c) * 4);
+  return Carver::round(sizeof(PrControl)) + mid + 5 * Carver::round(v * 4) + Carver::round(pr_max_chunks(edges) * 8) +
          Carver::round((static_cast<size_t>(edges) / kPrHugeDeg + 1) * 12) + 256 +
          Carver::round(4 * kPrMaxGrid * 8) + Carver::round(kPrMaxGrid * 4) + Carver::round(kPrMaxGrid * 8) + 4096;
 }
@@ -413,7 +452,8 @@ int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   a.contrib[0] = cv.take<float>(nodes);
   a.contrib[1] = cv.take<float>(nodes);
   a.heavy.q = nullptr;
-  a.heavy.mq = cv.take<int>(nodes);
+  a.heavy.mq = nullptr;
+  for (int c = 0; c < kPrClasses; c++) a.mid[c] = cv.take<int>(pr_class_cap(edges, c));
   a.heavy.hq = cv.take<int>(nodes);
   a.heavy.hoff = cv.take<unsigned>(nodes);
   a.hpart = cv.take<float2>(pr_max_chunks(edges));

@@ -266,6 +266,19 @@ def _pr_check(ig, orc, g, scores, iters):
     assert err.sum() <= PR_L1, (g.name, err.sum())
 
 
+@pytest.mark.parametrize("copies", [1, 30])
+def test_pagerank_list_classes(ig, orc, ctx, copies):
+    """Stars around the lengths that separate the classes in which lists of 64
+    entries and more are dealt out, and the split ones (4096)."""
+    sizes = np.tile([62, 63, 125, 126, 254, 511, 1021, 1022, 2046, 4093, 4094, 4095, 9000], copies)
+    k = len(sizes)
+    src = np.concatenate([np.arange(k), np.repeat(np.arange(k), sizes)])
+    dst = np.concatenate([(np.arange(k) + 1) % k, np.arange(k, k + sizes.sum())])
+    g = ig.from_edges(k + int(sizes.sum()), src.astype(np.int32), dst.astype(np.int32))
+    scores, iters = ctx.pagerank(ig.DeviceGraph(g))
+    _pr_check(ig, orc, g, scores, iters)
+
+
 @pytest.mark.parametrize("copies", [1, 3, 40, 700])
 def test_pagerank_list_lengths(ig, orc, ctx, copies):
     """Stars of 1 to 130 leaves, around the lengths at which a list goes from a
