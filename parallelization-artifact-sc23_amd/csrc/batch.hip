@@ -65,7 +65,7 @@
 //         every larger undecided neighbour has, as in the greedy order.
 //   PR  : the Jacobi recurrence of the single-query kernel (FP32 scores,
 //         Neumaier-compensated gathers: one lane per list of fewer than
-//         kPrWaveList entries in entry order, one wave per longer one,
+//         kPrLaneDeg entries in entry order, eight lanes or a wave per longer one,
 //         per-item partials combined in item order for heavy lists),
 //         stopping when the FP64 L1 change is <= 1e-4 or after 100 sweeps;
 //         every gang member adds the members' FP64 partials in the same
@@ -79,9 +79,9 @@
 #include <utility>
 #include <vector>
 
-#include "csum.hpp"
 #include "device_common.hpp"
 #include "emit.hpp"
+#include "gather.hpp"
 #include "unionfind.hpp"
 
 namespace indigo {
@@ -96,10 +96,10 @@ constexpr int kWidenEntries = 4096;  // CSR entries per member of a widened gang
 constexpr int kHeavyDeg = 1024;  // lists this long are split into items
 constexpr int kItem = 1024;      // entries per item
 constexpr int kCcSample = 2;      // CC: neighbours linked per vertex before the giant root is chosen
+constexpr int kCcDepth = 2;       // CC: hops beyond which a find stores the root (100 graphs: 5.1 / 4.7 / 4.7 / 7.6 ms at 5 / 2 / 1 / 0)
 constexpr int kCcSamples = 256;   // CC: vertices sampled to choose it
 constexpr int kCcAfforestMin = 4096;  // CC: smallest graph that takes the Afforest order
-constexpr int kSsspQueue = 1024;  // SSSP: appends that a workgroup buffers per round
-constexpr int kPrWaveList = 32;  // PR: lists walked by a whole wave
+constexpr int kBatchQueue = 2048;  // BFS, SSSP: appends that a workgroup buffers per round
 constexpr float kDamp = 0.85f;
 
 struct alignas(128) GangState {
@@ -295,17 +295,75 @@ IG_DEV unsigned long long wave_or(unsigned long long x)
   return x;
 }
 
-// Wave-collective append of u (where pred) to a queue, adding the degrees of
-// the appended vertices to *mf.
-IG_DEV void append_frontier(bool pred, int u, int deg, int* queue, unsigned* count, unsigned long long* mf)
+// Wave-collective: walks the lists as wave_entries_of does, kFly entries per lane
+// at a time, and hands over the owner lanes, the neighbours and which of them are
+// there: f(o, u, on), arrays of kFly.
+constexpr int kFly = 2;
+
+template <typename F>
+IG_DEV void wave_neighbours_of(int v, bool active, const BatchTask& T, F&& f)
 {
-  wave_append(pred, u, queue, count);
-  const unsigned long long d = wave_sum(static_cast<unsigned long long>(pred ? deg : 0));
-  if (lane_id() == 0 && d != 0ull) atomic_add_relaxed(mf, d);
+  const int lane = lane_id();
+  const int b = active ? T.nindex[v] : 0;
+  const int l = active ? T.nindex[v + 1] - b : 0;
+  const int len = heavy(l) ? 0 : l;
+  const int incl = wave_inclusive_scan(len);
+  const int total = wave_bcast(incl, kWave - 1);
+  const int shift = b - (incl - len);
+  for (int base = 0; base < total; base += kFly * kWave) {
+    int o[kFly], u[kFly];
+    bool on[kFly];
+#pragma unroll
+    for (int q = 0; q < kFly; q++) {
+      const int k = base + q * kWave + lane;
+      on[q] = k < total;
+      o[q] = min(wave_owner(incl, k), kWave - 1);
+      const int e = wave_shfl(shift, o[q]) + k;
+      u[q] = on[q] ? T.nlist[e] : 0;
+    }
+    f(o, u, on);
+  }
+}
+
+// Wave-collective: f as above for the entries [eb, ee) of one list (o is 0).
+template <typename F>
+IG_DEV void item_neighbours(int eb, int ee, const BatchTask& T, F&& f)
+{
+  for (int e0 = eb; e0 < ee; e0 += kFly * kWave) {
+    int o[kFly], u[kFly];
+    bool on[kFly];
+#pragma unroll
+    for (int q = 0; q < kFly; q++) {
+      const int e = e0 + q * kWave + lane_id();
+      on[q] = e < ee;
+      o[q] = 0;
+      u[q] = on[q] ? T.nlist[e] : 0;
+    }
+    f(o, u, on);
+  }
 }
 
 // ---- multi-source BFS -------------------------------------------------------
-IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_acc)[kWave])
+// Wave-collective: level to the slab rows of each lane's sources m, entry v.  The
+// wave takes a row at a time, so the stores of neighbouring vertices (pulls queue
+// them in order) go out together.
+IG_DEV void write_rows(const BatchTask& T, unsigned long long m, int v, int level)
+{
+  unsigned long long rows = wave_or(m);
+  rows = static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<int>(rows >> 32))) << 32 |
+         static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(rows)));
+  for (; rows != 0ull; rows &= rows - 1ull) {
+    const int i = __ffsll(static_cast<long long>(rows)) - 1;
+    if (m >> i & 1ull) T.out[static_cast<size_t>(i) * T.nodes + v] = level;
+  }
+}
+
+// Bound by the latency of its steps (list entry, mask, append).  The appends of a
+// level and their degree sum are gathered in LDS and registers instead of two
+// atomics and a 64-bit wave sum a step, two entries per lane are in flight and the
+// levels are written a row at a time: 100 graphs of 64 sources 32.6 -> 27.2 ms.
+IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_acc)[kWave],
+                    BlockQueue<kBatchQueue>& s_next, BlockSum& s_mf)
 {
   const int V = T.nodes;
   const int lane = lane_id();
@@ -341,7 +399,10 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
       st_relaxed(&T.out[static_cast<size_t>(i) * V + s], 0);
     }
     // a source listed twice is queued by the lane that set its first bit
-    append_frontier(has && old == 0ull, s, has ? T.nindex[s + 1] - T.nindex[s] : 0, queue[0], &qn[0], &mf[0]);
+    const bool first = has && old == 0ull;
+    wave_append(first, s, queue[0], &qn[0]);
+    const unsigned long long d = wave_sum(static_cast<unsigned long long>(first ? T.nindex[s + 1] - T.nindex[s] : 0));
+    if (lane == 0) atomic_add_relaxed(&mf[0], d);
   }
   if (!team_sync(tm)) return false;
   for (int lvl = 1;; lvl++) {
@@ -357,31 +418,49 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
       st_relaxed(&qn[(lvl + 1) & 3], 0u);
       st_relaxed(&mf[(lvl + 1) & 3], 0ull);
     }
+    bq_reset(s_next);
+    bs_reset(s_mf);
+    unsigned long long dsum = 0ull;  // degrees of what this lane appends
+    auto append = [&](bool first, int u) {
+      if (first) dsum += static_cast<unsigned>(T.nindex[u + 1] - T.nindex[u]);
+      bq_append(s_next, first, u, qnext, ncount);
+    };
     if (mcur * 14ull < static_cast<unsigned long long>(T.edges)) {
       // push from the frontier queue
       const int nq = (ncur + kWave - 1) / kWave;
-      auto push = [&](unsigned long long m, int e, bool valid) {
-        bool first = false;
-        int u = 0;
-        if (valid) {
-          u = T.nlist[e];
-          const unsigned long long add = m & ~ld_relaxed(&seen[u]);
-          if (add != 0ull)
-            first = __hip_atomic_fetch_or(&nxt[u], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0ull;
-        }
-        append_frontier(first, u, first ? T.nindex[u + 1] - T.nindex[u] : 0, qnext, ncount, nmf);
+      auto push = [&](const unsigned long long (&m)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+        unsigned long long add[kFly];
+        bool first[kFly];
+#pragma unroll
+        for (int q = 0; q < kFly; q++) add[q] = on[q] ? m[q] & ~ld_relaxed(&seen[u[q]]) : 0ull;
+#pragma unroll
+        for (int q = 0; q < kFly; q++)
+          first[q] = add[q] != 0ull && __hip_atomic_fetch_or(&nxt[u[q]], add[q], __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT) == 0ull;
+#pragma unroll
+        for (int q = 0; q < kFly; q++) append(first[q], u[q]);
       };
       for (int c = ch.first; c < nq; c += ch.step) {
         const int k = c * kWave + lane;
         const bool act = k < ncur;
         const int v = act ? ld_relaxed(&qcur[k]) : 0;
         const unsigned long long m = act ? ld_relaxed(&cur[v]) : 0ull;
-        wave_entries_of(v, act, T.nindex, [&](int o, int e, bool valid) { push(__shfl(m, o, kWave), e, valid); });
+        wave_neighbours_of(v, act, T, [&](const int (&o)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+          unsigned long long om[kFly];
+#pragma unroll
+          for (int q = 0; q < kFly; q++) om[q] = __shfl(m, o[q], kWave);
+          push(om, u, on);
+        });
       }
       for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
         const unsigned long long m = ld_relaxed(&cur[v]);
         if (m == 0ull) return;
-        for (int e0 = eb; e0 < ee; e0 += kWave) push(m, e0 + lane, e0 + lane < ee);
+        item_neighbours(eb, ee, T, [&](const int (&)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+          unsigned long long om[kFly];
+#pragma unroll
+          for (int q = 0; q < kFly; q++) om[q] = m;
+          push(om, u, on);
+        });
       });
     } else {
       // pull: every vertex with sources still missing
@@ -391,53 +470,65 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
         const unsigned long long missing = all & ~sv;
         s_acc[wid][lane] = 0ull;
         wave_lds_sync();
-        wave_entries_of(v, missing != 0ull, T.nindex, [&](int o, int e, bool valid) {
-          if (valid) {
-            const unsigned long long m = ld_relaxed(&cur[T.nlist[e]]);
-            if (m != 0ull) atomicOr(&s_acc[wid][o], m);
-          }
+        wave_neighbours_of(v, missing != 0ull, T, [&](const int (&o)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+          unsigned long long m[kFly];
+#pragma unroll
+          for (int q = 0; q < kFly; q++) m[q] = on[q] ? ld_relaxed(&cur[u[q]]) : 0ull;
+#pragma unroll
+          for (int q = 0; q < kFly; q++)
+            if (m[q] != 0ull) atomicOr(&s_acc[wid][o[q]], m[q]);
         });
         wave_lds_sync();
         const unsigned long long nb = s_acc[wid][lane] & missing;
         if (nb != 0ull) st_relaxed(&nxt[v], nb);
-        append_frontier(nb != 0ull, v, nb != 0ull ? T.nindex[v + 1] - T.nindex[v] : 0, qnext, ncount, nmf);
+        append(nb != 0ull, v);
       }
       for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
         const unsigned long long missing = all & ~ld_relaxed(&seen[v]);
         if (missing == 0ull) return;
         unsigned long long acc = 0ull;
-        for (int e = eb + lane; e < ee; e += kWave) acc |= ld_relaxed(&cur[T.nlist[e]]);
+        item_neighbours(eb, ee, T, [&](const int (&)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+          unsigned long long m[kFly];
+#pragma unroll
+          for (int q = 0; q < kFly; q++) m[q] = on[q] ? ld_relaxed(&cur[u[q]]) : 0ull;
+#pragma unroll
+          for (int q = 0; q < kFly; q++) acc |= m[q];
+        });
         const unsigned long long nb = wave_or(acc) & missing;
         bool first = false;
         if (nb != 0ull && lane == 0)
           first = __hip_atomic_fetch_or(&nxt[v], nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0ull;
-        append_frontier(first, v, first ? T.nindex[v + 1] - T.nindex[v] : 0, qnext, ncount, nmf);
+        append(first, v);
       });
     }
+    bs_add(s_mf, dsum);
+    bs_flush(s_mf, nmf);
+    bq_flush(s_next, qnext, ncount);
     if (!team_sync(tm)) return false;
     // the new frontier: masks, seen bits and levels; the old frontier's masks
     // are cleared (that buffer holds the next level's frontier)
     const int nnext = static_cast<int>(ld_relaxed(ncount));
     for (int k = tm.rank * kBatchBlock + static_cast<int>(threadIdx.x); k < ncur; k += tm.size * kBatchBlock)
       st_relaxed(&fr[(lvl - 1) & 1][ld_relaxed(&qcur[k])], 0ull);
-    for (int k = tm.rank * kBatchBlock + static_cast<int>(threadIdx.x); k < nnext; k += tm.size * kBatchBlock) {
-      const int u = ld_relaxed(&qnext[k]);
-      const unsigned long long sv = ld_relaxed(&seen[u]);
-      const unsigned long long nb = ld_relaxed(&nxt[u]) & ~sv;
-      st_relaxed(&nxt[u], 0ull);
-      st_relaxed(&seen[u], sv | nb);
-      st_relaxed(&nfr[u], nb);
-      for (unsigned long long m = nb; m != 0ull; m &= m - 1ull)
-        T.out[static_cast<size_t>(__ffsll(static_cast<long long>(m)) - 1) * V + u] = lvl;
+    for (int c = ch.first; c * kWave < nnext; c += ch.step) {
+      const int k = c * kWave + lane;
+      const int u = k < nnext ? ld_relaxed(&qnext[k]) : 0;
+      unsigned long long nb = 0ull;
+      if (k < nnext) {
+        const unsigned long long sv = ld_relaxed(&seen[u]);
+        nb = ld_relaxed(&nxt[u]) & ~sv;
+        st_relaxed(&nxt[u], 0ull);
+        st_relaxed(&seen[u], sv | nb);
+        st_relaxed(&nfr[u], nb);
+      }
+      write_rows(T, nb, u, lvl);
     }
     if (!team_sync(tm)) return false;
     if (nnext == 0) break;
   }
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
-    if (v >= V) continue;
-    for (unsigned long long m = all & ~ld_relaxed(&seen[v]); m != 0ull; m &= m - 1ull)
-      T.out[static_cast<size_t>(__ffsll(static_cast<long long>(m)) - 1) * V + v] = INT_MAX;
+    write_rows(T, v < V ? all & ~ld_relaxed(&seen[v]) : 0ull, v, INT_MAX);
   }
   return true;
 }
@@ -489,9 +580,8 @@ struct SsspRows {
 // Wave-collective: relaxes the pairs of each lane's list [beg, beg + len) of vertex v
 // and the sources in m.
 IG_DEV void relax_pairs(const BatchTask& T, const SsspRows& R, int v, int beg, int len, unsigned m,
-                        BlockQueue<kSsspQueue>& s_next)
+                        BlockQueue<kBatchQueue>& s_next)
 {
-  constexpr int kFly = 2;  // pairs in flight per lane
   const int lane = lane_id();
   const int pairs = len * __popc(m);  // (below 1024 * 32)
   const int incl = wave_inclusive_scan(pairs);
@@ -547,7 +637,7 @@ IG_DEV void relax_pairs(const BatchTask& T, const SsspRows& R, int v, int beg, i
   }
 }
 
-IG_DEV bool run_sssp(const BatchTask& T, const Team& tm, BlockQueue<kSsspQueue>& s_next)
+IG_DEV bool run_sssp(const BatchTask& T, const Team& tm, BlockQueue<kBatchQueue>& s_next)
 {
   const int V = T.nodes;
   const int lane = lane_id();
@@ -682,7 +772,7 @@ IG_DEV int giant_root(const BatchTask& T, int* parent, unsigned long long (*s_ac
   int* s_root = reinterpret_cast<int*>(&s_acc[0][0]);  // kCcSamples ints of the task scratch LDS
   const int V = T.nodes;
   for (int i = threadIdx.x; i < kCcSamples; i += blockDim.x)
-    s_root[i] = find_root(parent, static_cast<int>((static_cast<unsigned long long>(i) * 2654435761ull) %
+    s_root[i] = find_root<kCcDepth>(parent, static_cast<int>((static_cast<unsigned long long>(i) * 2654435761ull) %
                                                    static_cast<unsigned>(V)));
   __syncthreads();
   unsigned long long key = 0;  // (count << 32) | ~root: the largest wins
@@ -732,13 +822,13 @@ IG_DEV bool run_cc(const BatchTask& T, const Team& tm, unsigned long long (*s_ac
       const int v = c * kWave + lane;
       if (v < V) {
         const int b = T.nindex[v], e = min(T.nindex[v + 1], b + kCcSample);
-        for (int k = b; k < e; k++) link(parent, v, T.nlist[k]);
+        for (int k = b; k < e; k++) link<kCcDepth>(parent, v, T.nlist[k]);
       }
     }
     if (!team_sync(tm)) return false;
     for (int c = ch.first; c < ch.count; c += ch.step) {
       const int v = c * kWave + lane;
-      if (v < V) st_relaxed(&parent[v], find_root(parent, v));
+      if (v < V) st_relaxed(&parent[v], find_root<kCcDepth>(parent, v));
     }
     if (!team_sync(tm)) return false;
     giant = giant_root(T, parent, s_acc);
@@ -746,19 +836,19 @@ IG_DEV bool run_cc(const BatchTask& T, const Team& tm, unsigned long long (*s_ac
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
     bool todo = v < V;
-    if (aff && todo) todo = T.nindex[v + 1] - T.nindex[v] > kCcSample && find_root(parent, v) != giant;
+    if (aff && todo) todo = T.nindex[v + 1] - T.nindex[v] > kCcSample && find_root<kCcDepth>(parent, v) != giant;
     wave_entries_of(v, todo, T.nindex, [&](int o, int e, bool valid) {
       if (!valid) return;
       const int ov = c * kWave + o;
       const int u = T.nlist[e];
-      if (aff || u < ov) link(parent, ov, u);
+      if (aff || u < ov) link<kCcDepth>(parent, ov, u);
     });
   }
   for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
-    if (aff && find_root(parent, v) == giant) return;
+    if (aff && find_root<kCcDepth>(parent, v) == giant) return;
     for (int e = eb + lane; e < ee; e += kWave) {
       const int u = T.nlist[e];
-      if (aff || u < v) link(parent, v, u);
+      if (aff || u < v) link<kCcDepth>(parent, v, u);
     }
   });
   if (!team_sync(tm)) return false;
@@ -869,6 +959,9 @@ IG_DEV bool run_mis(const BatchTask& T, const Team& tm, int (*s_flag)[kWave])
 }
 
 // ---- PageRank ----------------------------------------------------------------------
+// Bound by the latency of the gathers.  Four masked loads per lane in flight and
+// groups of lanes for lists of 8 to 63 entries, as in the single-query kernel
+// (one lane or a wave per list, a load at a time: 52 -> 36 ms for 100 graphs).
 IG_DEV bool run_pr(const BatchTask& T, const Team& tm, double* s_red)
 {
   const int V = T.nodes;
@@ -906,22 +999,20 @@ IG_DEV bool run_pr(const BatchTask& T, const Team& tm, double* s_red)
     it++;
     const float* cin = contrib[(it - 1) & 1];
     float* cout = contrib[it & 1];
+    auto contribution = [cin](int u) { return ld_relaxed(&cin[u]); };
     double d = 0.0;
     for (int c = ch.first; c < ch.count; c += ch.step) {
       const int v = c * kWave + lane;
       const int beg = v < V ? T.nindex[v] : 0;
       const int deg = v < V ? T.nindex[v + 1] - beg : 0;
-      if (v < V && deg < kPrWaveList) {
-        CSum acc;
-        for (int e = beg; e < beg + deg; e++) acc.add(ld_relaxed(&cin[T.nlist[e]]));
-        d += finish(cout, v, deg, acc.value());
-      }
-      for (unsigned long long m = __ballot(v < V && deg >= kPrWaveList && !heavy(deg)); m != 0ull; m &= m - 1ull) {
+      const float sum = short_sums(contribution, T.nlist, beg, beg + deg, false);
+      if (v < V && deg < kPrWaveDeg) d += finish(cout, v, deg, sum);
+      for (unsigned long long m = __ballot(deg >= kPrWaveDeg && !heavy(deg)); m != 0ull; m &= m - 1ull) {
         const int o = __ffsll(static_cast<long long>(m)) - 1;
         const int x = c * kWave + o;
         const int xb = wave_bcast(beg, o), xd = wave_bcast(deg, o);
         CSum acc;
-        for (int e = xb + lane; e < xb + xd; e += kWave) acc.add(ld_relaxed(&cin[T.nlist[e]]));
+        gather<kWave>(acc, contribution, T.nlist, xb, xb + xd, lane);
         acc = wave_merge(acc);
         if (lane == 0) d += finish(cout, x, xd, acc.value());
       }
@@ -929,7 +1020,7 @@ IG_DEV bool run_pr(const BatchTask& T, const Team& tm, double* s_red)
     if (nitems > 0) {
       for_items(T, tm, nitems, [&](int, int eb, int ee, int i) {
         CSum acc;
-        for (int e = eb + lane; e < ee; e += kWave) acc.add(ld_relaxed(&cin[T.nlist[e]]));
+        gather<kWave>(acc, contribution, T.nlist, eb, ee, lane);
         acc = wave_merge(acc);
         if (lane == 0) {
           st_relaxed(&hpart[i].x, acc.s);
@@ -974,7 +1065,8 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 
   __shared__ unsigned long long s_acc[kBatchWaves][kWave];
   __shared__ int s_flag[kBatchWaves][kWave];
   __shared__ double s_red[kBatchWaves];
-  __shared__ BlockQueue<kSsspQueue> s_next;
+  __shared__ BlockQueue<kBatchQueue> s_next;
+  __shared__ BlockSum s_mf;
   if (!residency_barrier(&ctl->bar, residency_ticks)) return;
   const long long deadline = now_ticks() + budget;
   for (;;) {
@@ -1003,7 +1095,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 
     const Team tm{rank, min(T.gang, static_cast<int>(gridDim.x)), &gangs[t], &ctl->bar, deadline};
     if (!team_sync(tm)) break;  // the gang assembles
     bool ok = true;
-    if (T.alg == INDIGO_QUERY_BFS) ok = run_bfs(T, tm, s_acc);
+    if (T.alg == INDIGO_QUERY_BFS) ok = run_bfs(T, tm, s_acc, s_next, s_mf);
     else if (T.alg == INDIGO_QUERY_SSSP) ok = run_sssp(T, tm, s_next);
     else if (T.alg == INDIGO_QUERY_CC) ok = run_cc(T, tm, s_acc);
     else if (T.alg == INDIGO_QUERY_PR) ok = run_pr(T, tm, s_red);

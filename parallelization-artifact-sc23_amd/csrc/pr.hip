@@ -35,6 +35,7 @@
 #include "device_common.hpp"
 #include "csum.hpp"
 #include "frontier.hpp"
+#include "gather.hpp"
 #include "trace.hpp"
 
 namespace indigo {
@@ -42,15 +43,11 @@ namespace indigo {
 namespace {
 
 constexpr int kPrBlock = 512;
-constexpr int kPrLaneDeg = 8;    // shorter lists: one lane each (twice as long where no list of the wave is longer)
-constexpr int kPrWaveDeg = 64;   // longer lists up to this: one group of lanes each
-constexpr int kPrGroup = 8;      // lanes of a group
 constexpr int kPrHugeDeg = 4096;   // lists split into items
 constexpr int kPrHugeChunk = 2048;  // entries per item, one workgroup each
 constexpr float kDamp = 0.85f;
 
 constexpr int kPrMaxGrid = 4096;
-constexpr int kPrUnroll = 4;  // gathers in flight per lane
 
 // Lists of kPrWaveDeg entries up to kPrHugeDeg by length: class c holds those of
 // kPrWaveDeg << c entries up to twice as many.
@@ -100,77 +97,6 @@ struct PrArgs {
 IG_DEV int deg_of(const PrArgs& a, int v)
 {
   return a.degree ? a.degree[v] : a.nindex[v + 1] - a.nindex[v];
-}
-
-// acc += cin[nlist[e]] for e = beg + first, beg + first + step, ... < end,
-// in that order, with kPrUnroll independent loads in flight per lane: the
-// gathers are latency-bound chains (index, then contribution), so a plain
-// loop would wait out one round trip per window.  Past the end a lane adds 0.
-template <int kStep>
-IG_DEV void gather(CSum& acc, const float* __restrict__ cin, const int* __restrict__ nlist, int beg, int end,
-                   int first)
-{
-  for (int e = beg + first; e < end; e += kPrUnroll * kStep) {
-    int u[kPrUnroll];
-#pragma unroll
-    for (int q = 0; q < kPrUnroll; q++) u[q] = e + q * kStep < end ? nlist[e + q * kStep] : -1;
-    float c[kPrUnroll];
-#pragma unroll
-    for (int q = 0; q < kPrUnroll; q++) c[q] = u[q] >= 0 ? cin[u[q]] : 0.f;
-#pragma unroll
-    for (int q = 0; q < kPrUnroll; q++) acc.add(c[q]);
-  }
-}
-
-// Sum over the kPrGroup lanes of a group, in each of them.
-IG_DEV CSum group_merge(CSum a)
-{
-#pragma unroll
-  for (int d = kPrGroup / 2; d > 0; d >>= 1) {
-    const float s2 = __shfl_xor(a.s, d, kWave);
-    const float c2 = __shfl_xor(a.c, d, kWave);
-    a.merge(s2, c2);
-  }
-  return a;
-}
-
-// Wave-collective: the gathered sum of each lane's list [beg, end) where it has
-// fewer than kPrWaveDeg entries (0 elsewhere).  Lists of fewer than kPrLaneDeg
-// entries are summed by their own lane; the others go kPrGroup lanes to a list,
-// kWave / kPrGroup lists at a time, instead of a wave to a list of 16 to 63
-// (random graph of 2^20 vertices and degree 16: 2.06 -> 1.11 ms a call).  A wave
-// without lists of 2 * kPrLaneDeg entries leaves all to their lanes: on degree 4
-// the few longer ones' extra step cost 5%.
-// few: the wave has at most kWave / kPrGroup lists, all of them grouped.
-IG_DEV float short_sums(const float* __restrict__ cin, const int* __restrict__ nlist, int beg, int end, bool few)
-{
-  const int lane = lane_id();
-  const int deg = end - beg;
-  const bool any = few || __ballot(deg >= 2 * kPrLaneDeg && deg < kPrWaveDeg) != 0ull;
-  const int limit = few ? 1 : (any ? kPrLaneDeg : 2 * kPrLaneDeg);
-  CSum own;
-  if (deg < limit) gather<1>(own, cin, nlist, beg, end, 0);
-  float sum = own.value();
-  if (!any) return sum;
-  const bool grouped = deg >= limit && deg < kPrWaveDeg;
-  const unsigned long long m = __ballot(grouped);
-  const int rows = __popcll(m);
-  const int rank = lanes_below(m);
-  // lane r gets the lane of the r-th grouped list (others push past the rows)
-  const int rest = lane - rank + rows;  // lanes without a grouped list, in order, behind them
-  const int at = __builtin_amdgcn_ds_permute((grouped ? rank : rest) << 2, lane);
-  constexpr int kPer = kWave / kPrGroup;
-  for (int r0 = 0; r0 < rows; r0 += kPer) {
-    const int r = r0 + lane / kPrGroup;
-    const int from = wave_shfl(at, r < kWave ? r : kWave - 1);
-    const int b = wave_shfl(beg, from), e = wave_shfl(end, from);
-    CSum acc;
-    if (r < rows) gather<kPrGroup>(acc, cin, nlist, b, e, lane % kPrGroup);
-    acc = group_merge(acc);
-    const float v = wave_shfl(acc.value(), ((rank - r0) & (kPer - 1)) * kPrGroup);
-    if (grouped && rank >= r0 && rank < r0 + kPer) sum = v;
-  }
-  return sum;
 }
 
 // New score of v from its gathered sum and its old score; writes score and next
@@ -315,6 +241,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
     it++;
     const float* cin = a.contrib[(it - 1) & 1];
     float* cout = a.contrib[it & 1];
+    auto contribution = [cin](int u) { return cin[u]; };
     double* slots = a.partial + (it & 1) * (2 * kPrMaxGrid);
     double d = 0.0;
     const int tl = 3 + 4 * (it - 1);
@@ -332,7 +259,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
       const int beg = a.nindex[v] + static_cast<int>(item - first) * kPrHugeChunk;
       const int end = min(a.nindex[v + 1], beg + kPrHugeChunk);
       CSum acc;
-      gather<kPrBlock>(acc, cin, a.nlist, beg, end, static_cast<int>(threadIdx.x));
+      gather<kPrBlock>(acc, contribution, a.nlist, beg, end, static_cast<int>(threadIdx.x));
       const CSum blk = block_merge(acc, s_ps, s_pc);
       if (threadIdx.x == 0) {
         // the partial and the counter are device-scope accesses, the store
@@ -367,7 +294,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
       const int beg = a.nindex[v], end = a.nindex[v + 1];
       const float old = a.scores[v];
       CSum acc;
-      gather<kWave>(acc, cin, a.nlist, beg, end, lane);
+      gather<kWave>(acc, contribution, a.nlist, beg, end, lane);
       acc = wave_merge(acc);
       if (lane == 0) d += finish_vertex(a, v, old, acc.value(), base, cout);
     }
@@ -379,7 +306,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
       const bool mine = lane < per && c < chunks && v < a.nodes;
       const int beg = mine ? a.nindex[v] : 0, end = mine ? a.nindex[v + 1] : 0;
       const float old = mine ? a.scores[v] : 0.f;  // (in flight beside the gathers)
-      const float sum = short_sums(cin, a.nlist, beg, end, few);
+      const float sum = short_sums(contribution, a.nlist, beg, end, few);
       if (mine && end - beg < kPrWaveDeg) d += finish_vertex(a, v, old, sum, base, cout);
     }
     d = block_sum_f64(d, s_red);

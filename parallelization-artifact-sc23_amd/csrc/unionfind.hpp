@@ -18,7 +18,7 @@
 //     the grid find the same two roots at once).
 // 0.39 to 0.44 and 0.87 ms; 4-neighbour grid of 1024^2 0.67 -> 0.22.  Depths of 1,
 // 2 and 5 gave 0.83, 0.64 and 0.42 ms on the random graph, 0.225, 0.245 and 0.250
-// on R-MAT 22.
+// on R-MAT 22 (the gangs of a batch, whose vertices fewer lanes share, take 2).
 #pragma once
 
 #include "device_common.hpp"
@@ -29,6 +29,7 @@ constexpr int kFindDepth = 5;
 
 // Root of x.  The store replaces x's parent by one of its ancestors, so
 // concurrent finds and links stay valid (x is no root, so no link writes it).
+template <int kDepth = kFindDepth>
 IG_DEV int find_root(int* parent, int x)
 {
   int r = x, p = ld_relaxed(&parent[x]);
@@ -38,7 +39,7 @@ IG_DEV int find_root(int* parent, int x)
     p = ld_relaxed(&parent[r]);
     hops++;
   }
-  if (hops > kFindDepth) st_relaxed(&parent[x], r);
+  if (hops > kDepth) st_relaxed(&parent[x], r);
   return r;
 }
 
@@ -58,18 +59,19 @@ IG_DEV int hook(int* parent, int hi, int lo)
 
 // Joins the trees of a and b.  (Each round the first lane of every wave that still
 // has something to join either joins it or finds that another wave has.)
+template <int kDepth = kFindDepth>
 IG_DEV void link(int* parent, int a, int b)
 {
-  int ra = find_root(parent, a);
-  int rb = find_root(parent, b);
+  int ra = find_root<kDepth>(parent, a);
+  int rb = find_root<kDepth>(parent, b);
   while (ra != rb) {
     const int hi = ra > rb ? ra : rb;
     const int lo = ra > rb ? rb : ra;
     const int now = hook(parent, hi, lo);
     if (now == hi) return;
     // climb from where hi now points
-    ra = find_root(parent, ra == hi && now >= 0 ? now : ra);
-    rb = find_root(parent, rb == hi && now >= 0 ? now : rb);
+    ra = find_root<kDepth>(parent, ra == hi && now >= 0 ? now : ra);
+    rb = find_root<kDepth>(parent, rb == hi && now >= 0 ? now : rb);
   }
 }
 

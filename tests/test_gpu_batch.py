@@ -117,6 +117,30 @@ def test_batch_idle_grid(ig, orc, ctx, nodes, cap):
     _check_against_plain(ctx, [g], [dg], qs)
 
 
+@pytest.mark.parametrize("copies", [1, 3, 40])
+@pytest.mark.parametrize("cap", [1, 0])
+def test_batch_list_lengths(ig, orc, ctx, copies, cap):
+    """Stars around the lengths at which a PageRank list goes from a lane to
+    eight (8, 16), a wave (64) and items (1024), and around the 128 entries of
+    a BFS step, joined in a ring by their centres; the largest appends more
+    than a workgroup buffers (2048)."""
+    from test_gpu_kernels import _pr_check
+
+    sizes = np.tile([1, 5, 6, 13, 14, 61, 62, 125, 126, 127, 1021, 1022, 3000], copies)
+    k = len(sizes)
+    n = k + int(sizes.sum())
+    src = np.concatenate([np.arange(k), np.repeat(np.arange(k), sizes)])
+    dst = np.concatenate([(np.arange(k) + 1) % k, np.arange(k, n)])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32))
+    dg = ig.DeviceGraph(g)
+    rng = np.random.default_rng(copies)
+    qs = [ig.Query("bfs", 0, dg, rng.integers(0, n, 64)), ig.Query("bfs", 0, dg, [k - 1]), ig.Query("cc", 0, dg)]
+    pr = ig.Query("pr", 0, dg)
+    ctx.batch([dg], qs + [pr], max_workgroups=cap)
+    _check_against_plain(ctx, [g], [dg], qs)
+    _pr_check(ig, orc, g, *pr.result())
+
+
 def test_batch_rejects_bad_queries(ig, ctx):
     g = ig.grid(4, 4)
     dg = ig.DeviceGraph(g)
