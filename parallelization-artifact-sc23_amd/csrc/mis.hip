@@ -14,8 +14,9 @@
 // processes the vertices
 // still undecided after round r-1, kept in two worklists by list length:
 // lists shorter than kMidDeg (round 0: every such vertex, in id order) are
-// scanned by one lane each, longer ones (round 0: a static list collected at
-// start) by one wave each, 256 entries per step with ballots.  Vertices that
+// started by one lane each and finished by a group of lanes, longer ones (round
+// 0: a static list collected at start) scanned by one wave each, 256 entries per
+// step with ballots.  Vertices that
 // stay undecided are appended (wave-aggregated) to the next round's lists.
 // Decisions are made in place: a decided state (1 included, 2 excluded) never
 // changes, so a vertex that reads a neighbour's final state may act on it in
@@ -37,7 +38,8 @@ namespace {
 constexpr int kMisBlock = 512;
 
 constexpr int kUndecided = 0, kIncluded = 1, kExcluded = 2;
-constexpr int kMisLaneUnroll = 4;  // entries per step of a one-lane decision
+constexpr int kMisLaneUnroll = 4;  // entries per lane and step of a decision
+constexpr int kMisGroupShift = 3;  // log2 of the lanes that finish a list a lane has started
 
 struct MisControl {
   GridBarrier bar;
@@ -67,55 +69,58 @@ IG_DEV unsigned long long mis_key(int v, unsigned flip)
   return (static_cast<unsigned long long>(p) << 32) | static_cast<unsigned>(v);
 }
 
-// One lane decides vertex v (short list).  Returns the new state.
+// One lane decides vertex v from the first kMisLaneUnroll entries of its (short)
+// list.  Returns the new state, or -1 if it takes the rest of the list.
 IG_DEV int decide_lane(const MisArgs& a, int v, int beg, int end)
 {
   // Only neighbours with a larger key can decide v: a smaller one cannot be
   // included while v is undecided (it would need v excluded first), so their
-  // states are not read.  Four entries' loads are in flight at a time and
+  // states are not read.  The entries' loads are in flight together and
   // evaluated in entry order.
   const unsigned long long kv = mis_key(v, a.flip);
-  for (int e = beg; e < end; e += kMisLaneUnroll) {
-    int su[kMisLaneUnroll];
+  int u[kMisLaneUnroll], su[kMisLaneUnroll];
 #pragma unroll
-    for (int q = 0; q < kMisLaneUnroll; q++) {
-      const int u = e + q < end ? a.nlist[e + q] : v;
-      const bool larger = u != v && mis_key(u, a.flip) > kv;
-      su[q] = larger ? ld_relaxed(&a.status[u]) : kExcluded;
-    }
+  for (int q = 0; q < kMisLaneUnroll; q++) u[q] = beg + q < end ? a.nlist[beg + q] : v;
 #pragma unroll
-    for (int q = 0; q < kMisLaneUnroll; q++) {
-      if (su[q] == kIncluded) return kExcluded;
-      if (su[q] == kUndecided) return kUndecided;
-    }
+  for (int q = 0; q < kMisLaneUnroll; q++)
+    su[q] = u[q] != v && mis_key(u[q], a.flip) > kv ? ld_relaxed(&a.status[u[q]]) : kExcluded;
+#pragma unroll
+  for (int q = 0; q < kMisLaneUnroll; q++) {
+    if (su[q] == kIncluded) return kExcluded;
+    if (su[q] == kUndecided) return kUndecided;
   }
-  return kIncluded;
+  return end - beg > kMisLaneUnroll ? -1 : kIncluded;
 }
-// v has just been included: its larger-key neighbours are all excluded
-// already, so only the smaller-key ones are read, and the undecided among
-// them excluded.  (Storing unconditionally is slower: device-scope stores
-// to already excluded hub neighbours cost more than the reads they save.)
+// v, whose list ends within the first step, has just been included: its larger-key
+// neighbours are all excluded already, so only the smaller-key ones are read, and
+// the undecided among them excluded.  (Storing unconditionally is slower:
+// device-scope stores to already excluded hub neighbours cost more than the reads
+// they save.)
 IG_DEV void exclude_neighbours_lane(const MisArgs& a, int v, int beg, int end)
 {
   const unsigned long long kv = mis_key(v, a.flip);
-  for (int e = beg; e < end; e++) {
-    const int u = a.nlist[e];
-    if (u != v && mis_key(u, a.flip) < kv && ld_relaxed(&a.status[u]) == kUndecided)
-      st_relaxed(&a.status[u], kExcluded);
-  }
+  int u[kMisLaneUnroll], su[kMisLaneUnroll];
+#pragma unroll
+  for (int q = 0; q < kMisLaneUnroll; q++) u[q] = beg + q < end ? a.nlist[beg + q] : v;
+#pragma unroll
+  for (int q = 0; q < kMisLaneUnroll; q++)
+    su[q] = u[q] != v && mis_key(u[q], a.flip) < kv ? ld_relaxed(&a.status[u[q]]) : kExcluded;
+#pragma unroll
+  for (int q = 0; q < kMisLaneUnroll; q++)
+    if (su[q] == kUndecided) st_relaxed(&a.status[u[q]], kExcluded);
 }
 
 // The two together for a vertex per group of 1 << gs lanes (same v, beg, end in a
-// group; beg = end where there is none), four entries per lane in flight; all
+// group; beg = end where there is none; the entries before from have decided nothing), four entries per lane in flight; all
 // lanes of the wave must be converged.  Returns the new state.
-IG_DEV int decide_group(const MisArgs& a, int v, int beg, int end, int gs)
+IG_DEV int decide_group(const MisArgs& a, int v, int beg, int from, int end, int gs)
 {
   const unsigned long long kv = mis_key(v, a.flip);
   const int lane = lane_id();
   const int sub = lane & ((1 << gs) - 1);
   const unsigned long long group = (gs == 6 ? ~0ull : (1ull << (1 << gs)) - 1ull) << (lane - sub);
   int r = beg < end ? -1 : kIncluded;
-  for (int e0 = beg + sub; __ballot(r < 0) != 0ull; e0 += kMisLaneUnroll << gs) {
+  for (int e0 = from + sub; __ballot(r < 0) != 0ull; e0 += kMisLaneUnroll << gs) {
     int su[kMisLaneUnroll];
 #pragma unroll
     for (int q = 0; q < kMisLaneUnroll; q++) {
@@ -251,7 +256,7 @@ __global__ __launch_bounds__(kMisBlock) __attribute__((amdgpu_waves_per_eu(8, 8)
     while (gs < 6 && (static_cast<unsigned long long>(n) << (gs + 1)) <= static_cast<unsigned long long>(stride)) gs++;
     for (unsigned base = 0, at = blockIdx.x; base < n; base += stride >> gs, at = next_place(at, gridDim.x)) {
       const unsigned idx = base + ((at * blockDim.x + threadIdx.x) >> gs);
-      bool keep = false;
+      bool keep = false, rest = false;
       int v = 0, beg = 0, end = 0;
       if (idx < n) {
         v = (r == 0) ? static_cast<int>(idx) : ld_relaxed(&in[idx]);
@@ -261,18 +266,36 @@ __global__ __launch_bounds__(kMisBlock) __attribute__((amdgpu_waves_per_eu(8, 8)
           if (end - beg >= kMidDeg) end = beg = -1;
           else if (beg == end || gs == 0) {
             const int st = decide_lane(a, v, beg, end);
+            rest = st < 0;
             if (st == kIncluded) {
               st_relaxed(&a.status[v], kIncluded);
               exclude_neighbours_lane(a, v, beg, end);
             } else if (st == kExcluded) {
               st_relaxed(&a.status[v], kExcluded);
             } else {
-              keep = true;
+              keep = st == kUndecided;
             }
           }
         }
       }
-      if (gs > 0) keep = decide_group(a, v, beg, end, gs) == kUndecided && (lane & ((1 << gs) - 1)) == 0;
+      if (gs == 0) {
+        // The lists that go on, eight lanes each.  A lane that went on alone, up to
+        // 16 steps to decide and 63 to exclude, kept its wave that long: round 0 of
+        // R-MAT 22 375 us, a call 0.68 ms, now 0.52 (random graph of 2^20 vertices and
+        // degree 16 0.33 -> 0.28; groups of 4 and 16: the same).
+        constexpr int kShift = kMisGroupShift, kPer = kWave >> kShift;
+        const unsigned long long m = __ballot(rest);
+        const int rows = __popcll(m), rank = lanes_below(m);
+        const int of = __builtin_amdgcn_ds_permute((rest ? rank : lane - rank + rows) << 2, lane);
+        for (int r0 = 0; r0 < rows; r0 += kPer) {
+          const int row = r0 + (lane >> kShift);
+          const int o = wave_shfl(of, min(row, kWave - 1));
+          const int gv = wave_shfl(v, o), gb = wave_shfl(beg, o), ge = wave_shfl(end, o);
+          const int st = decide_group(a, gv, gb, gb + kMisLaneUnroll, row < rows ? ge : gb, kShift);
+          bq_append(s_wl, st == kUndecided && (lane & ((1 << kShift) - 1)) == 0, gv, out, &oc->n);
+        }
+      }
+      if (gs > 0) keep = decide_group(a, v, beg, beg, end, gs) == kUndecided && (lane & ((1 << gs) - 1)) == 0;
       bq_append(s_wl, keep, v, out, &oc->n);
     }
     // long lists: one wave each

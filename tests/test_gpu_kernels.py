@@ -219,6 +219,25 @@ def test_mis_lane_groups(ig, orc, ctx, nodes, workgroups, signed):
         ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, 0)
 
 
+@pytest.mark.parametrize("copies", [1, 9, 60])
+@pytest.mark.parametrize("workgroups", [1, 5])
+def test_mis_list_lengths(ig, orc, ctx, copies, workgroups):
+    """Lists around those at which a vertex goes from a lane to eight (4), these
+    take another step (4 + 32) and a wave takes it over (64), on grids that have
+    fewer lanes than vertices."""
+    sizes = np.tile([1, 2, 3, 4, 33, 34, 35, 36, 60, 61, 62, 63], copies)
+    k = len(sizes)
+    n = k + int(sizes.sum())
+    src = np.concatenate([np.arange(k), np.repeat(np.arange(k), sizes)])
+    dst = np.concatenate([(np.arange(k) + 1) % k, np.random.default_rng(copies).permutation(n - k) + k])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32))
+    ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, workgroups)
+    try:
+        assert np.array_equal(ctx.mis(ig.DeviceGraph(g)), orc.mis(g))
+    finally:
+        ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, 0)
+
+
 def test_cc_catalog(ig, orc, ctx):
     for g in catalog(ig):
         assert np.array_equal(ctx.cc(ig.DeviceGraph(g)), orc.cc(g)), g.name
