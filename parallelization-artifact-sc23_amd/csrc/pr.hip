@@ -11,8 +11,8 @@
 //   vertex order (coalesced score / contrib / index traffic), one lane or one
 //   group of lanes to a list;
 //   longer lists, collected once into a static list, one wave each; lists of
-//   kPrHugeDeg or more in kPrHugeChunk-entry items, one workgroup each, whose
-//   partial sums go to a per-item slot; the workgroup that finishes a huge
+//   kPrHugeDeg or more in kPrHugeChunk-entry items, one wave each, whose
+//   partial sums go to a per-item slot; the wave that finishes a huge
 //   vertex's last item (a counter per vertex) combines its item partials in
 //   item order, so no second barrier is needed;
 // then one barrier and the stop test.  Per-vertex sums are FP32 with Neumaier
@@ -44,14 +44,15 @@ namespace {
 
 constexpr int kPrBlock = 512;
 constexpr int kPrHugeDeg = 4096;   // lists split into items
-constexpr int kPrHugeChunk = 2048;  // entries per item, one workgroup each
+constexpr int kPrHugeChunk = 1024;  // entries per item, one wave each
+constexpr int kPrBuckets = 16;      // items are ordered by their first neighbour's part of the ids
 constexpr float kDamp = 0.85f;
 
 constexpr int kPrMaxGrid = 4096;
 
 // Lists of kPrWaveDeg entries up to kPrHugeDeg by length: class c holds those of
 // kPrWaveDeg << c entries up to twice as many.
-constexpr int kPrClasses = 6;
+constexpr int kPrClasses = __builtin_ctz(kPrHugeDeg / kPrWaveDeg);
 static_assert(kPrWaveDeg << kPrClasses == kPrHugeDeg, "the classes cover the lists between short and huge");
 constexpr int kPrClassCap = 512;  // lists of a class that a workgroup buffers while collecting
 
@@ -59,6 +60,7 @@ struct PrControl {
   GridBarrier bar;
   FrontierCounters heavy;
   PaddedU32 nclass[kPrClasses];
+  PaddedU32 nbucket[kPrBuckets];
   int iterations;
   int status;
   double last_diff;
@@ -82,7 +84,8 @@ struct PrArgs {
   float* contrib[2];
   int* mid[kPrClasses];  // lists of kPrWaveDeg entries and more, by class
   FrontierQueues heavy;  // lists of kPrHugeDeg entries and more (huge)
-  float2* hpart;         // per huge item: compensated partial (sum, error)
+  unsigned long long* items;  // huge items by bucket (HugeItem, in two words)
+  float2* hpart;         // per slot: compensated partial (sum, error)
   int hcap;              // huge vertices at most: edges / kPrHugeDeg + 1
   unsigned* hdone;       // per huge vertex: items finished this sweep
   double* hres;          // per huge vertex: |s' - s| of this sweep
@@ -124,24 +127,6 @@ IG_DEV float2 ld_float2(const float2* p)
   return v;
 }
 
-// Workgroup-wide compensated sum of one partial per thread; result valid in
-// thread 0.
-IG_DEV CSum block_merge(CSum acc, float* s_ps, float* s_pc)
-{
-  acc = wave_merge(acc);
-  const int wid = threadIdx.x / kWave;
-  if (lane_id() == 0) {
-    s_ps[wid] = acc.s;
-    s_pc[wid] = acc.c;
-  }
-  __syncthreads();
-  CSum blk;
-  if (threadIdx.x == 0)
-    for (int w = 0; w < kPrBlock / kWave; w++) blk.merge(s_ps[w], s_pc[w]);
-  __syncthreads();
-  return blk;
-}
-
 // FP64 sum of one value per thread; result valid in every thread.
 IG_DEV double block_sum_f64(double x, double* s_red)
 {
@@ -155,12 +140,39 @@ IG_DEV double block_sum_f64(double x, double* s_red)
   return t;
 }
 
+// Part of the list of huge vertex number j: entries [beg, end), partial in slot.
+struct HugeItem {
+  int j, slot, beg, end;
+};
+
+// Items of huge vertex v.
+IG_DEV int huge_items(const PrArgs& a, int v)
+{
+  return static_cast<int>((static_cast<unsigned>(a.nindex[v + 1] - a.nindex[v]) + kPrHugeChunk - 1u) / kPrHugeChunk);
+}
+
+// Item k of huge vertex number j, which is v and whose slots start at first.
+IG_DEV HugeItem huge_item(const PrArgs& a, int j, unsigned first, int k, int v)
+{
+  const int beg = a.nindex[v] + k * kPrHugeChunk, end = a.nindex[v + 1];
+  return {j, static_cast<int>(first) + k, beg, end - beg < kPrHugeChunk ? end : beg + kPrHugeChunk};
+}
+
+IG_DEV unsigned long long pack(int lo, int hi)
+{
+  return static_cast<unsigned long long>(static_cast<unsigned>(hi)) << 32 | static_cast<unsigned>(lo);
+}
+
+IG_DEV void unpack(unsigned long long x, int& lo, int& hi)
+{
+  lo = static_cast<int>(x);
+  hi = static_cast<int>(x >> 32);
+}
+
 __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
 {
   __shared__ double s_red[kPrBlock / kWave];
-  __shared__ float s_ps[kPrBlock / kWave], s_pc[kPrBlock / kWave];
-  __shared__ int s_owner;
-  __shared__ int s_last;
+  __shared__ unsigned s_bucket[kPrBuckets], s_slot[kPrBuckets];
   __shared__ FrontierEmitterT<64, 64, 64> s_emit;
   __shared__ BlockQueue<kPrClassCap> s_class[kPrClasses];
   __shared__ unsigned s_nclass[kPrClasses];
@@ -216,6 +228,49 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
   const unsigned long long hp = ld_relaxed(&ctl->heavy.hpack);
   const unsigned nh = huge_count(hp), nch = huge_chunks(hp);
 
+  // Huge items.  While there is one for a wave at most, it keeps it; otherwise they
+  // are ordered by where in the ids they begin (counted, then placed), so that at
+  // any time the waves gather from one part of the contributions, which the L2s
+  // hold, and not from all of them (R-MAT 22, 16 MB: the items' part of a sweep
+  // 130 -> 56 us, a call 5.87 -> 5.61 ms; with lists of 1024 entries and more in
+  // items 6.0: an item costs three round trips beyond its entries).
+  const bool ordered = nch > static_cast<unsigned>(nwaves);
+  HugeItem own{};
+  if (!ordered && static_cast<unsigned>(wave) < nch) {
+    const int j = huge_owner_wave(a.heavy.hoff, static_cast<int>(nh), static_cast<unsigned>(wave));
+    const unsigned first = ld_relaxed(&a.heavy.hoff[j]);
+    own = huge_item(a, j, first, static_cast<int>(wave - first), ld_relaxed(&a.heavy.hq[j]));
+  }
+  for (int pass = 0; ordered && pass < 2; pass++) {
+    if (threadIdx.x < kPrBuckets) s_bucket[threadIdx.x] = 0u;
+    __syncthreads();
+    for (unsigned j = static_cast<unsigned>(wave); j < nh; j += nwaves) {
+      const int v = ld_relaxed(&a.heavy.hq[j]);
+      const unsigned first = ld_relaxed(&a.heavy.hoff[j]);
+      const int items = huge_items(a, v);
+      for (int k = lane; k < items; k += kWave) {
+        const HugeItem item = huge_item(a, static_cast<int>(j), first, k, v);
+        const unsigned b = static_cast<unsigned>(static_cast<unsigned long long>(a.nlist[item.beg]) * kPrBuckets /
+                                                 static_cast<unsigned>(a.nodes));
+        const unsigned n = atomicAdd(&s_bucket[b], 1u);
+        if (pass == 1) {
+          st_relaxed(&a.items[2 * (s_slot[b] + n)], pack(item.j, item.slot));
+          st_relaxed(&a.items[2 * (s_slot[b] + n) + 1], pack(item.beg, item.end));
+        }
+      }
+    }
+    __syncthreads();
+    if (pass == 0 && threadIdx.x < kPrBuckets)
+      s_slot[threadIdx.x] = atomic_add_relaxed(&ctl->nbucket[threadIdx.x].v, s_bucket[threadIdx.x]);
+    if (!grid_barrier<true>(&ctl->bar, deadline)) {
+      if (tid == 0) ctl->status = 1;
+      if (threadIdx.x == 0) a.exit_it[blockIdx.x] = -1000000;
+      return;
+    }
+    if (pass == 0 && threadIdx.x < kPrBuckets)
+      for (unsigned b = 0; b < threadIdx.x; b++) s_slot[threadIdx.x] += ld_relaxed(&ctl->nbucket[b].v);
+  }
+
   // mid lists, the longest first, are dealt to the workgroups in turn, and to
   // their waves in turn: by class, the shares differ by less than a list of each
   // (unsorted, the workgroups finished a sweep of R-MAT 22 after 660 to 910 us).
@@ -248,43 +303,40 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
     trace_level(&ctl->trace, tl, static_cast<unsigned>(it), 0ull, 0);
 
     // huge items -> partials; the last item of a vertex combines them
-    for (unsigned item = blockIdx.x; item < nch; item += gridDim.x) {
-      if (threadIdx.x == 0) s_owner = huge_owner(a.heavy.hoff, static_cast<int>(nh), item);
-      __syncthreads();
-      const int j = s_owner;
-      const int v = a.heavy.hq[j];
-      const int len = a.nindex[v + 1] - a.nindex[v];
-      const int items = (len + kPrHugeChunk - 1) / kPrHugeChunk;
-      const unsigned first = a.heavy.hoff[j];
-      const int beg = a.nindex[v] + static_cast<int>(item - first) * kPrHugeChunk;
-      const int end = min(a.nindex[v + 1], beg + kPrHugeChunk);
+    for (unsigned p = static_cast<unsigned>(wave); p < nch; p += nwaves) {
+      HugeItem item = own;
+      if (ordered) {
+        unpack(ld_relaxed(&a.items[2 * p]), item.j, item.slot);
+        unpack(ld_relaxed(&a.items[2 * p + 1]), item.beg, item.end);
+      }
+      const int v = a.heavy.hq[item.j];  // (in flight beside the gathers)
+      const int items = huge_items(a, v);
+      const unsigned first = a.heavy.hoff[item.j];
       CSum acc;
-      gather<kPrBlock>(acc, contribution, a.nlist, beg, end, static_cast<int>(threadIdx.x));
-      const CSum blk = block_merge(acc, s_ps, s_pc);
-      if (threadIdx.x == 0) {
+      gather<kWave>(acc, contribution, a.nlist, item.beg, item.end, lane);
+      acc = wave_merge(acc);
+      unsigned k = 0u;
+      if (lane == 0) {
         // the partial and the counter are device-scope accesses, the store
         // completed before the count (agent-scope acquire / release fences
         // would write back and invalidate the XCD's L2, and with it the
         // cached contributions every gather reads: 6.8 -> 9.7 ms)
-        st_float2(&a.hpart[item], make_float2(blk.s, blk.c));
+        st_float2(&a.hpart[item.slot], make_float2(acc.s, acc.c));
         wave_drain();
-        const unsigned k = atomic_add_relaxed(&a.hdone[j], 1u);
-        s_last = k + 1 == static_cast<unsigned>(items);
+        k = atomic_add_relaxed(&a.hdone[item.j], 1u);
       }
-      __syncthreads();
-      if (s_last && threadIdx.x < kWave) {
+      if (wave_bcast(static_cast<int>(k), 0) + 1 == items) {
         CSum tot;
-        for (int k = lane; k < items; k += kWave) {
-          const float2 p = ld_float2(&a.hpart[first + k]);
-          tot.merge(p.x, p.y);
+        for (int q = lane; q < items; q += kWave) {
+          const float2 part = ld_float2(&a.hpart[first + q]);
+          tot.merge(part.x, part.y);
         }
         tot = wave_merge(tot);
         if (lane == 0) {
-          st_relaxed(&a.hres[j], finish_vertex(a, v, a.scores[v], tot.value(), base, cout));
-          st_relaxed(&a.hdone[j], 0u);  // every item of this sweep has counted
+          st_relaxed(&a.hres[item.j], finish_vertex(a, v, a.scores[v], tot.value(), base, cout));
+          st_relaxed(&a.hdone[item.j], 0u);  // every item of this sweep has counted
         }
       }
-      __syncthreads();
     }
     trace_level(&ctl->trace, tl + 1, static_cast<unsigned>(it), 0ull, 1);
     // phase A: mid lists, one wave each
@@ -359,7 +411,8 @@ size_t pr_workspace_bytes(int nodes, int edges)
   const size_t v = static_cast<size_t>(nodes);
   size_t mid = 0;
   for (int c = 0; c < kPrClasses; c++) mid += Carver::round(pr_class_cap(edges, c) * 4);
-  return Carver::round(sizeof(PrControl)) + mid + 5 * Carver::round(v * 4) + Carver::round(pr_max_chunks(edges) * 8) +
+  return Carver::round(sizeof(PrControl)) + mid + 5 * Carver::round(v * 4) + Carver::round(pr_max_chunks(edges) * 16) +
+         Carver::round(pr_max_chunks(edges) * 8) +
          Carver::round((static_cast<size_t>(edges) / kPrHugeDeg + 1) * 12) + 256 +
          Carver::round(4 * kPrMaxGrid * 8) + Carver::round(kPrMaxGrid * 4) + Carver::round(kPrMaxGrid * 8) + 4096;
 }
@@ -383,6 +436,7 @@ int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   for (int c = 0; c < kPrClasses; c++) a.mid[c] = cv.take<int>(pr_class_cap(edges, c));
   a.heavy.hq = cv.take<int>(nodes);
   a.heavy.hoff = cv.take<unsigned>(nodes);
+  a.items = cv.take<unsigned long long>(2 * pr_max_chunks(edges));
   a.hpart = cv.take<float2>(pr_max_chunks(edges));
   a.hcap = edges / kPrHugeDeg + 1;  // every huge list holds kPrHugeDeg entries or more
   a.hdone = cv.take<unsigned>(static_cast<size_t>(a.hcap));

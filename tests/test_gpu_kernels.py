@@ -298,6 +298,26 @@ def test_pagerank_list_classes(ig, orc, ctx, copies):
     _pr_check(ig, orc, g, scores, iters)
 
 
+@pytest.mark.parametrize("workgroups", [1, 2, 13, 0])
+def test_pagerank_items(ig, orc, ctx, workgroups):
+    """Lists of 4 to 71 items of 1024 entries and a few entries on either side,
+    on grids with fewer waves than items, which order them, and with more."""
+    sizes = np.array([4094, 4095, 5118, 5119, 8190, 8191, 20000, 64 * 1024 - 2, 65 * 1024 - 1, 72000])
+    k = len(sizes)
+    n = k + 100000
+    rng = np.random.default_rng(5)
+    src = np.concatenate([np.arange(k), np.repeat(np.arange(k), sizes)])
+    dst = np.concatenate([(np.arange(k) + 1) % k] + [rng.permutation(n - k)[:s] + k for s in sizes])
+    src, dst = np.concatenate([src, np.arange(k, n)]), np.concatenate([dst, np.arange(k, n) % k])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32))
+    ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, workgroups)
+    try:
+        scores, iters = ctx.pagerank(ig.DeviceGraph(g))
+    finally:
+        ctx.set_hint(ig._lib.HINT_MAX_WORKGROUPS, 0)
+    _pr_check(ig, orc, g, scores, iters)
+
+
 @pytest.mark.parametrize("copies", [1, 3, 40, 700])
 def test_pagerank_list_lengths(ig, orc, ctx, copies):
     """Stars of 1 to 130 leaves, around the lengths at which a list goes from a
