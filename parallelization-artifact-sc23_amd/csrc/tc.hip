@@ -107,6 +107,7 @@ static_assert(kTcHugeChunk % kTcBlock == 0, "tc_pack_huge moves whole items");
 // ties with 2^15.
 int wave_work_for(int edges) { return edges < (1 << 24) ? 1 << 13 : 1 << 14; }
 constexpr int kPartItems = 2048;    // items per workgroup-pass part (1024 and 4096: slower)
+constexpr int kPartBuckets = 64;    // order in which the parts are taken
 constexpr int kUnroll = 4;          // windows of 64 per step over a long list
 constexpr int kLongList = 128;      // lists walked by the whole wave (64, 96: slower; 160, 192: the same)
 constexpr int kWalk = 4;            // windows of 64 in flight per step of that walk (2 and 8: slower);
@@ -137,6 +138,7 @@ struct TcControl {
   int error;
   int hub_bin;             // hubs: min(degree, kHubKeys) >= hub_bin
   int pad[24];
+  unsigned part_n[kPartBuckets], part_at[kPartBuckets];  // parts per bucket, and placed so far
   unsigned grab[kGrabStripes][32];  // stripe s: grabs of chunks s, s + kGrabStripes, ... (first word used)
 };
 
@@ -963,6 +965,73 @@ IG_DEV unsigned long long tiny_tasks(unsigned long long mask, const int2 rl, int
   return cnt;
 }
 
+// Parts: at most one per vertex plus one per kPartItems list entries.
+size_t part_words(int nodes, int edges)
+{
+  return static_cast<size_t>(nodes) + 2 * (static_cast<size_t>(edges) / kPartItems) + 64;
+}
+
+// Large graphs: the workgroup pass takes its parts ordered by where the list of
+// their first item lies, so that at any time the workgroups read lists of one
+// stretch of olist, a share of which the L2s still hold (that pass runs at the
+// fabric's rate of misses: R-MAT 22 9.82 -> 9.58 ms a call, R-MAT 20 2.326 -> 2.293;
+// below 2^24 entries the two launches cost more than they give, 0.767 -> 0.785 on
+// R-MAT 18).  Parts of 1024 and 512 items, which span less, gave 9.78 and 10.2.
+// The ordered parts take the place of the selections' outcome bytes, where these
+// hold them.
+bool order_parts(int nodes, int edges)
+{
+  return edges >= (1 << 24) && part_words(nodes, edges) * 8 <= static_cast<size_t>(edges);
+}
+
+// Bucket of part p: the part of olist in which its first item's list lies.
+IG_DEV int part_bucket(unsigned long long p, const int2* __restrict__ dk, const int2* __restrict__ orng,
+                       const int2* __restrict__ orngk, const int* __restrict__ olist, const int* __restrict__ ilist, int edges)
+{
+  const int v = static_cast<int>(p >> 32);
+  const int lo = static_cast<int>(p & 0xffffffffull) * kPartItems;
+  const int2 r = orng[v];
+  const int key = lo < r.y ? row_get(olist, r.x, lo, narrow_key(dk[v].y)) : ilist[r.x + lo - r.y];
+  return min(static_cast<int>(static_cast<long long>(orngk[key].x) * kPartBuckets / edges), kPartBuckets - 1);
+}
+
+// Counts the parts of every bucket, then (kPlace) writes them in bucket order: a
+// workgroup reserves its share of each bucket with one atomic.
+template <bool kPlace>
+__global__ __launch_bounds__(kMidBlock) void tc_order_parts(const int2* __restrict__ dk, const int2* __restrict__ orng,
+                                                            const int2* __restrict__ orngk,
+                                                            const int* __restrict__ olist, const int* __restrict__ ilist,
+                                                            const unsigned long long* __restrict__ parts, int edges,
+                                                            unsigned long long* out, TcControl* ctl)
+{
+  __shared__ unsigned s_n[kPartBuckets], s_at[kPartBuckets];
+  const unsigned n = ctl->nmid;
+  const unsigned stride = gridDim.x * kMidBlock;
+  if (threadIdx.x < kPartBuckets) s_n[threadIdx.x] = 0u;
+  __syncthreads();
+  for (unsigned k = blockIdx.x * kMidBlock + threadIdx.x; k < n; k += stride)
+    atomicAdd(&s_n[part_bucket(parts[k], dk, orng, orngk, olist, ilist, edges)], 1u);
+  __syncthreads();
+  if (threadIdx.x < kPartBuckets) {
+    const unsigned i = threadIdx.x;
+    if (!kPlace) {
+      if (s_n[i] != 0u) atomic_add_relaxed(&ctl->part_n[i], s_n[i]);
+    } else {
+      unsigned at = 0u;
+      for (unsigned b = 0; b < i; b++) at += ctl->part_n[b];
+      s_at[i] = at + (s_n[i] != 0u ? atomic_add_relaxed(&ctl->part_at[i], s_n[i]) : 0u);
+      s_n[i] = 0u;
+    }
+  }
+  if (!kPlace) return;
+  __syncthreads();
+  for (unsigned k = blockIdx.x * kMidBlock + threadIdx.x; k < n; k += stride) {
+    const unsigned long long p = parts[k];
+    const int b = part_bucket(p, dk, orng, orngk, olist, ilist, edges);
+    out[s_at[b] + atomicAdd(&s_n[b], 1u)] = p;
+  }
+}
+
 // Wave-collective: appends the parts (x << 32 | part) of each lane's task.
 IG_DEV void append_parts(int parts, int x, unsigned long long* queue, unsigned* count)
 {
@@ -1136,12 +1205,6 @@ int grid_for(long long items, int per_block, int cap)
 constexpr size_t kListPad = kWalk * kWave + 16;
 size_t list_words(int edges) { return static_cast<size_t>(edges) + kListPad; }
 
-// Parts: at most one per vertex plus one per kPartItems list entries.
-size_t part_words(int nodes, int edges)
-{
-  return static_cast<size_t>(nodes) + 2 * (static_cast<size_t>(edges) / kPartItems) + 64;
-}
-
 size_t hcnt_words(int edges)
 {
   const size_t e = static_cast<size_t>(edges);
@@ -1230,9 +1293,18 @@ int tc_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   const int hint = ctx->hints[INDIGO_HINT_TC_LDS_LIST];
   const int mid_list = hint > 0 && hint < kMidSlots / 4 ? hint : kMidSlots / 4;
   const int big_list = hint > 0 && hint < kBigSlots / 4 ? hint : kBigSlots / 4;
+  const unsigned long long* parts = mid;
+  if (order_parts(nodes, edges)) {
+    const int gp = share_grid(ctx, ctx->compute_units, kMidBlock);
+    unsigned long long* ordered = reinterpret_cast<unsigned long long*>(up);
+    tc_order_parts<false><<<gp, kMidBlock, 0, s>>>(dk, orng, orngk, olist, ilist, mid, edges, ordered, ctl);
+    tc_order_parts<true><<<gp, kMidBlock, 0, s>>>(dk, orng, orngk, olist, ilist, mid, edges, ordered, ctl);
+    parts = ordered;
+    n_launch += 2;
+  }
   IG_TRY(kernel_begin(ctx, "tc_count_group<512, 8192>"));
   tc_count_group<kMidBlock, kMidSlots><<<share_grid(ctx, ctx->compute_units * 4, kMidBlock), kMidBlock, 0, s>>>(
-      dk, orng, orngk, olist, ilen, ilist, mid, &ctl->nmid, &ctl->next_mid, mid_list, ctl);
+      dk, orng, orngk, olist, ilen, ilist, parts, &ctl->nmid, &ctl->next_mid, mid_list, ctl);
   IG_TRY(kernel_end(ctx));
   tc_count_group<kBigBlock, kBigSlots><<<share_grid(ctx, ctx->compute_units, kBigBlock), kBigBlock, 0, s>>>(
       dk, orng, orngk, olist, ilen, ilist, big, &ctl->nbig, &ctl->next_big, big_list, ctl);

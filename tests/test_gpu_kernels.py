@@ -372,6 +372,19 @@ def test_tc_clique_unions(ig, ctx):
         assert ctx.tc(ig.DeviceGraph(g)) == want, seed
 
 
+@pytest.mark.parametrize("hubs", [0, 100])
+@pytest.mark.parametrize("sizes", [[2048] * 4, [2049] * 4, [2049] * 4 + [700] * 9])
+def test_tc_ordered_parts(ig, ctx, sizes, hubs):
+    """Just below and above the 2^24 entries from which the workgroup pass
+    orders its parts, with all lists 16-bit and with nearly none."""
+    g = cliques(ig, sizes, seed=len(sizes))
+    ctx.set_hint(ig._lib.HINT_TC_HUBS, hubs)
+    try:
+        assert ctx.tc(ig.DeviceGraph(g)) == sum(k * (k - 1) * (k - 2) // 6 for k in sizes)
+    finally:
+        ctx.set_hint(ig._lib.HINT_TC_HUBS, 0)
+
+
 def test_tc_rmat16(ig, orc, ctx):
     g = ig.rmat(16, 16, seed=6)
     assert ctx.tc(ig.DeviceGraph(g)) == orc.tc(g)
