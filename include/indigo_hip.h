@@ -172,7 +172,7 @@ int indigo_ctx_copy_ms(indigo_ctx* ctx, void* d_dst, const void* d_src, size_t b
 int indigo_ctx_last_grid(indigo_ctx* ctx, int* grid, int* per_cu);
 /* Per-level trace of the last BFS or SSSP call (first 256 levels): start of
  * each level in microseconds since the kernel began, frontier size, its
- * degree sum, and the mode (0 top-down, 1 bottom-up, 2 one-workgroup phase,
+ * degree sum, and the mode (0 top-down, 1 bottom-up, 2 team phase,
  * 3 SSSP far-pile split).  After an MIS call, one entry per round: its start,
  * the undecided vertices with short lists and (as degree_sum) those with
  * long lists.  Any output pointer may be NULL. */
@@ -184,7 +184,7 @@ int indigo_ctx_trim(indigo_ctx* ctx);
 int indigo_ctx_set_hint(indigo_ctx* ctx, int key, int value);
 #define INDIGO_HINT_BFS_DIRECTION 1 /* 0 auto, 1 top-down only, 2 allow bottom-up */
 #define INDIGO_HINT_SSSP_DELTA 2    /* 0 auto, else near-far split increment */
-#define INDIGO_HINT_SMALL_FRONTIER 3 /* 0 auto, 1 off: never use the one-workgroup mode (BFS, SSSP) */
+#define INDIGO_HINT_SMALL_FRONTIER 3 /* 0 auto, 1 off: never use the team mode (BFS, SSSP) */
 #define INDIGO_HINT_BUDGET_MS 4      /* bound on device-side waits in ms (0: 60000) */
 #define INDIGO_HINT_BLOCKS_PER_CU 5  /* cap on co-resident workgroups per CU of persistent kernels (0: occupancy) */
 #define INDIGO_HINT_TC_LDS_LIST 6    /* entries of an oriented list TC hashes in LDS at once (0: 2048 or 8192 by

@@ -185,7 +185,7 @@ IG_DEV int wave_owner(int incl, int k)
 //     / RMWs, which bypass the non-coherent caches).  Completion of those
 //     accesses (s_waitcnt 0 in every wave before the workgroup barrier) is
 //     then all the ordering a barrier needs: about 2.5 us.
-// Waiters back off exponentially so that long waits (one-workgroup phases)
+// Waiters back off exponentially so that long waits (team phases)
 // do not flood the memory channel of the generation counter.
 struct alignas(128) PaddedU32 {
   unsigned int v;
@@ -275,7 +275,7 @@ IG_DEV bool residency_barrier(GridBarrier* gb, long long ticks)
 }
 
 // Same as grid_barrier's abort test, for loops that run between barriers
-// (one-workgroup phases): true when the kernel must stop.
+// (team phases): true when the kernel must stop.
 IG_DEV bool kernel_aborted(GridBarrier* gb, long long deadline)
 {
   if (__hip_atomic_load(&gb->abort.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return true;

@@ -48,7 +48,7 @@ struct alignas(128) FrontierCounters {
 
 // Per-level trace written by workgroup 0 of a traversal kernel: wall-clock
 // tick at the start of the level, frontier size, its degree sum and the mode
-// (0 top-down, 1 bottom-up, 2 one-workgroup phase, 3 far-pile split).
+// (0 top-down, 1 bottom-up, 2 team phase, 3 far-pile split).
 constexpr int kTraceMax = 256;
 struct LevelTrace {
   int n;

@@ -10,7 +10,7 @@
 // the queue takes the slot alone (its kernels are ordinary launches), and so
 // does a BFS or SSSP request on a deep, sparse graph (average degree below
 // 6, at least 65536 vertices: grids, road networks), on the single-query
-// kernels: their one-workgroup phase runs the thousands of narrow levels at
+// kernels: their team phase runs the thousands of narrow levels at
 // workgroup-barrier cost (the batched engine's gangs pay a device barrier
 // per level: 82 ms against about 45 for a 2048^2 grid's BFS), and the
 // batched Bellman-Ford rounds re-relax such graphs many times over, while

@@ -79,7 +79,7 @@ struct SsspArgs {
   int edges;
   int src;
   int delta_hint;
-  int allow_small;  // the one-workgroup phase may run (INDIGO_HINT_SMALL_FRONTIER != 1)
+  int allow_small;  // the team phase may run (INDIGO_HINT_SMALL_FRONTIER != 1)
   const int* __restrict__ nindex;
   const int* __restrict__ nlist;
   const int* __restrict__ eweight;

@@ -81,7 +81,7 @@ class Context:
 
     def last_trace(self) -> list[tuple[float, int, float, int]]:
         """Per-level (start_us, frontier, degree_sum, mode) of the last BFS /
-        SSSP call; mode 0 top-down, 1 bottom-up, 2 one-workgroup, 3 split."""
+        SSSP call; mode 0 top-down, 1 bottom-up, 2 team, 3 split."""
         m = 256
         us = (ctypes.c_float * m)()
         nf = (ctypes.c_uint * m)()
