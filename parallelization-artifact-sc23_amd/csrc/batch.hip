@@ -56,12 +56,11 @@
 //         component minima), then flattening; graphs of average degree 8 or
 //         more link in Afforest order and skip the giant component's lists.
 //   MIS : the greedy fixed point in descending (hash(v + 712313887), v)
-//         order; per round a decide phase (a vertex joins when no neighbour
-//         is included and no undecided neighbour has a larger key) and an
-//         exclude phase.  A heavy vertex's items raise per-vertex flags
-//         (blocked, has an included neighbour) in the decide phase, and the
-//         vertex is decided from them in the exclude phase.  Deferring a
-//         decision by a phase changes no result: a vertex decides only once
+//         order; rounds of decisions in place, as the single-query kernel's (a
+//         vertex joins when its larger neighbours are all excluded, and is
+//         excluded once one of them is included).  A heavy vertex's items
+//         raise per-vertex flags, by which it is decided in the next round.
+//         Deferring a decision changes no result: a vertex decides only once
 //         every larger undecided neighbour has, as in the greedy order.
 //   PR  : the Jacobi recurrence of the single-query kernel (FP32 scores,
 //         Neumaier-compensated gathers: one lane per list of fewer than
@@ -82,6 +81,7 @@
 #include "device_common.hpp"
 #include "emit.hpp"
 #include "gather.hpp"
+#include "mis_decide.hpp"
 #include "unionfind.hpp"
 
 namespace indigo {
@@ -95,6 +95,7 @@ constexpr int kGangShift = 18;   // CSR entries per gang member
 constexpr int kWidenEntries = 4096;  // CSR entries per member of a widened gang (widen_floor)
 constexpr int kHeavyDeg = 1024;  // lists this long are split into items
 constexpr int kItem = 1024;      // entries per item
+constexpr int kMisWaveList = 64;   // MIS: lists finished by a whole wave
 constexpr int kCcSample = 2;      // CC: neighbours linked per vertex before the giant root is chosen
 constexpr int kCcDepth = 2;       // CC: hops beyond which a find stores the root (100 graphs: 5.1 / 4.7 / 4.7 / 7.6 ms at 5 / 2 / 1 / 0)
 constexpr int kCcSamples = 256;   // CC: vertices sampled to choose it
@@ -860,27 +861,32 @@ IG_DEV bool run_cc(const BatchTask& T, const Team& tm, unsigned long long (*s_ac
 }
 
 // ---- MIS -------------------------------------------------------------------------
-IG_DEV unsigned long long mis_key(int v)
-{
-  return (static_cast<unsigned long long>(mis_hash(static_cast<unsigned>(v) + 712313887u)) << 32) |
-         static_cast<unsigned>(v);
-}
+struct MisView {
+  const int* nlist;
+  int* status;
+  unsigned flip;
+};
 
-IG_DEV bool run_mis(const BatchTask& T, const Team& tm, int (*s_flag)[kWave])
+// Rounds of decisions in place, as the single-query kernel's: a lane looks at the
+// first entries of a list, eight lanes (a wave from kMisWaveList entries on) finish
+// what they leave open, and a vertex that joins excludes its smaller neighbours.  A
+// heavy vertex's items gather flags (1: a larger neighbour not excluded, 2: one
+// included), by which its own chunk decides it in the next round; the flags of
+// even and odd rounds are apart.  One barrier a round.  (Rounds of two phases that
+// each read all entries of the undecided vertices: 12.6 ms for 100 graphs, now 2.6.)
+IG_DEV bool run_mis(const BatchTask& T, const Team& tm)
 {
   const int V = T.nodes;
   const int lane = lane_id();
-  const int wid = threadIdx.x / kWave;
-  int* status = T.out;
-  unsigned* blocked = static_cast<unsigned*>(T.scratch);  // heavy vertices: a blocking neighbour seen
-  unsigned* near_in = blocked + V;                         // heavy vertices: an included neighbour seen
+  const MisView a{T.nlist, T.out, 0u};
+  unsigned* flags[2] = {static_cast<unsigned*>(T.scratch), static_cast<unsigned*>(T.scratch) + V};
   const Chunks ch = team_chunks(tm, V);
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
     if (v < V) {
-      st_relaxed(&status[v], 0);
-      st_relaxed(&blocked[v], 0u);
-      st_relaxed(&near_in[v], 0u);
+      st_relaxed(&a.status[v], kUndecided);
+      st_relaxed(&flags[0][v], 0u);
+      st_relaxed(&flags[1][v], 0u);
     }
   }
   int nitems = 0;
@@ -888,70 +894,61 @@ IG_DEV bool run_mis(const BatchTask& T, const Team& tm, int (*s_flag)[kWave])
   for (int r = 0;; r++) {
     unsigned* flag = &tm.gs->flag[r % 3];
     if (tm.rank == 0 && threadIdx.x == 0) st_relaxed(&tm.gs->flag[(r + 1) % 3], 0u);
-    // decide (lists shorter than kHeavyDeg) and gather the heavy vertices' flags
+    unsigned* seen = flags[(r + 1) & 1];  // the last round's flags
+    bool still = false;
     for (int c = ch.first; c < ch.count; c += ch.step) {
       const int v = c * kWave + lane;
-      const int deg = v < V ? T.nindex[v + 1] - T.nindex[v] : 0;
-      const bool und = v < V && !heavy(deg) && ld_relaxed(&status[v]) == 0;
-      s_flag[wid][lane] = 0;
-      wave_lds_sync();
-      wave_entries_of(v, und, T.nindex, [&](int o, int e, bool valid) {
-        if (!valid) return;
-        const int ov = c * kWave + o;
-        const int u = T.nlist[e];
-        // only larger keys can block (or be included next to) an undecided
-        // vertex: a smaller one cannot be included before it is decided
-        if (u != ov && mis_key(u) > mis_key(ov) && ld_relaxed(&status[u]) != 2) s_flag[wid][o] = 1;
-      });
-      wave_lds_sync();
-      if (und && s_flag[wid][lane] == 0) st_relaxed(&status[v], 1);
+      const bool und = v < V && ld_relaxed(&a.status[v]) == kUndecided;
+      if (__ballot(und) == 0ull) continue;
+      const int beg = und ? T.nindex[v] : 0;
+      const int end = und ? T.nindex[v + 1] : 0;
+      bool rest = false;
+      if (und) {
+        int st = kUndecided;
+        if (!heavy(end - beg)) {
+          st = decide_lane(a, v, beg, end);
+          rest = st < 0;
+        } else if (r > 0) {
+          const unsigned f = ld_relaxed(&seen[v]);
+          st_relaxed(&seen[v], 0u);
+          st = (f & 2u) != 0u ? kExcluded : ((f & 1u) != 0u ? kUndecided : kIncluded);
+        }
+        if (st == kIncluded || st == kExcluded) st_relaxed(&a.status[v], st);
+        if (st == kIncluded && !heavy(end - beg)) exclude_neighbours_lane(a, v, beg, end);
+        still |= st == kUndecided;
+      }
+      constexpr int kPer = kWave >> kMisGroupShift;
+      const bool grouped = rest && end - beg < kMisWaveList;
+      const unsigned long long m = __ballot(grouped);
+      const int rows = __popcll(m), rank = lanes_below(m);
+      const int of = __builtin_amdgcn_ds_permute((grouped ? rank : lane - rank + rows) << 2, lane);
+      for (int r0 = 0; r0 < rows; r0 += kPer) {
+        const int row = r0 + (lane >> kMisGroupShift);
+        const int o = wave_shfl(of, min(row, kWave - 1));
+        const int gv = wave_shfl(v, o), gb = wave_shfl(beg, o), ge = wave_shfl(end, o);
+        still |= decide_group(a, gv, gb, gb + kMisLaneUnroll, row < rows ? ge : gb, kMisGroupShift) == kUndecided;
+      }
+      for (unsigned long long w = __ballot(rest && !grouped); w != 0ull; w &= w - 1ull) {
+        const int o = __ffsll(static_cast<long long>(w)) - 1;
+        const int wb = wave_bcast(beg, o);
+        still |= decide_group(a, wave_bcast(v, o), wb, wb + kMisLaneUnroll, wave_bcast(end, o), 6) == kUndecided;
+      }
     }
+    set_flag(flag, still);
     for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
-      if (ld_relaxed(&status[v]) != 0) return;
-      const unsigned long long kv = mis_key(v);
-      bool blk = false, inc = false;
+      if (ld_relaxed(&a.status[v]) != kUndecided) return;
+      const unsigned long long kv = mis_key(v, a.flip);
+      unsigned f = 0u;
       for (int e = eb + lane; e < ee; e += kWave) {
         const int u = T.nlist[e];
-        if (u == v || mis_key(u) < kv) continue;  // smaller keys cannot decide v
-        const int su = ld_relaxed(&status[u]);
-        inc |= su == 1;
-        blk |= su != 2;
+        if (u == v || mis_key(u, a.flip) < kv) continue;  // smaller keys cannot decide v
+        const int su = ld_relaxed(&a.status[u]);
+        f |= su == kIncluded ? 3u : (su == kUndecided ? 1u : 0u);
       }
-      const bool any_blk = __ballot(blk) != 0ull, any_inc = __ballot(inc) != 0ull;
-      if (lane == 0 && any_blk) st_relaxed(&blocked[v], 1u);
-      if (lane == 0 && any_inc) st_relaxed(&near_in[v], 1u);
+      f = (__ballot((f & 1u) != 0u) != 0ull ? 1u : 0u) | (__ballot((f & 2u) != 0u) != 0ull ? 2u : 0u);
+      if (lane == 0 && f != 0u)
+        __hip_atomic_fetch_or(&flags[r & 1][v], f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     });
-    if (!team_sync(tm)) return false;
-    // exclude the undecided neighbours of included vertices; decide the heavy
-    // vertices from their flags
-    for (int c = ch.first; c < ch.count; c += ch.step) {
-      const int v = c * kWave + lane;
-      const int deg = v < V ? T.nindex[v + 1] - T.nindex[v] : 0;
-      const bool und = v < V && ld_relaxed(&status[v]) == 0;
-      const bool hv = und && heavy(deg);
-      s_flag[wid][lane] = 0;
-      wave_lds_sync();
-      wave_entries_of(v, und && !hv, T.nindex, [&](int o, int e, bool valid) {
-        if (!valid) return;
-        const int u = T.nlist[e];
-        // an included neighbour of an undecided vertex has a larger key
-        if (mis_key(u) > mis_key(c * kWave + o) && ld_relaxed(&status[u]) == 1) s_flag[wid][o] = 1;
-      });
-      wave_lds_sync();
-      bool still = false;
-      if (und && !hv) {
-        if (s_flag[wid][lane] != 0) st_relaxed(&status[v], 2);
-        else still = true;
-      }
-      if (hv) {
-        if (ld_relaxed(&near_in[v]) != 0u) st_relaxed(&status[v], 2);
-        else if (ld_relaxed(&blocked[v]) == 0u) st_relaxed(&status[v], 1);
-        else still = true;
-        st_relaxed(&blocked[v], 0u);
-        st_relaxed(&near_in[v], 0u);
-      }
-      set_flag(flag, still);
-    }
     if (!team_sync(tm)) return false;
     if (ld_relaxed(flag) == 0u) break;
   }
@@ -1063,7 +1060,6 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 
 {
   __shared__ int s_task, s_rank;
   __shared__ unsigned long long s_acc[kBatchWaves][kWave];
-  __shared__ int s_flag[kBatchWaves][kWave];
   __shared__ double s_red[kBatchWaves];
   __shared__ BlockQueue<kBatchQueue> s_next;
   __shared__ BlockSum s_mf;
@@ -1099,7 +1095,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 
     else if (T.alg == INDIGO_QUERY_SSSP) ok = run_sssp(T, tm, s_next);
     else if (T.alg == INDIGO_QUERY_CC) ok = run_cc(T, tm, s_acc);
     else if (T.alg == INDIGO_QUERY_PR) ok = run_pr(T, tm, s_red);
-    else ok = run_mis(T, tm, s_flag);
+    else ok = run_mis(T, tm);
     if (!ok) break;
   }
 }

@@ -141,6 +141,23 @@ def test_batch_list_lengths(ig, orc, ctx, copies, cap):
     _pr_check(ig, orc, g, *pr.result())
 
 
+@pytest.mark.parametrize("leaves", [3001, 40000])
+@pytest.mark.parametrize("cap", [1, 6, 0])
+def test_batch_mis_list_lengths(ig, ctx, leaves, cap):
+    """Lists around those at which a vertex goes from a lane to eight (4), to a
+    wave (64) and to items (1024), from shared leaves, on gangs of one and more."""
+    sizes = np.array([2, 3, 4, 34, 35, 60, 61, 62, 125, 1020, 1021, 1022, 1023, 2046, 3000] * 3)
+    k = len(sizes)
+    rng = np.random.default_rng(leaves)
+    src = np.concatenate([np.arange(k), np.repeat(np.arange(k), sizes)])
+    dst = np.concatenate([(np.arange(k) + 1) % k] + [rng.permutation(leaves)[:s] + k for s in sizes])
+    g = ig.from_edges(k + leaves, src.astype(np.int32), dst.astype(np.int32))
+    dg = ig.DeviceGraph(g)
+    qs = [ig.Query("mis", 0, dg)]
+    ctx.batch([dg], qs, max_workgroups=cap)
+    _check_against_plain(ctx, [g], [dg], qs)
+
+
 def test_batch_rejects_bad_queries(ig, ctx):
     g = ig.grid(4, 4)
     dg = ig.DeviceGraph(g)
