@@ -162,7 +162,7 @@ IG_DEV void bottom_up(const BfsArgs& a, int L, unsigned nheavy, const FrontierQu
 // is idle meanwhile).
 struct SmallLds {
   TeamShare<kSmallCap> share;
-  int abort_flag;
+  PhaseStop stop;
 };
 
 // A team of workgroups (one, or up to kTeamMax) advances levels alone while
@@ -193,7 +193,7 @@ IG_DEV int team_phase(const BfsArgs& a, int L, unsigned n, const Team& tm, const
   constexpr int kFly = 4;  // entries in flight per lane
   const int t = static_cast<int>(threadIdx.x);
   TeamShare<kSmallCap>& F = S.share;
-  if (t == 0) S.abort_flag = 0;
+  if (t == 0) S.stop.clear();
   unsigned entries = 0;
   int cn = share_load(F, L & 1, tm, static_cast<int>(n), a.nindex, [&](int i) { return ld_relaxed(&in.q[i]); }, &entries);
   TeamSum sum;
@@ -203,7 +203,7 @@ IG_DEV int team_phase(const BfsArgs& a, int L, unsigned n, const Team& tm, const
   // queue's lists are not empty)
   if (*aborted || sum.most > static_cast<unsigned>(kSmallCap)) return L;
   for (;;) {
-    if ((L & 63) == 0 && t == 0) S.abort_flag = kernel_aborted(&ctl->bar, deadline) ? 1 : 0;
+    if ((L & 63) == 0 && t == 0) S.stop.post(L, kernel_aborted(&ctl->bar, deadline));
     int shift = 0;  // g = 1 << shift lanes per slot
     while (shift < 6 && (cn << (shift + 1)) <= kBfsBlock) shift++;
     const int sub = t & ((1 << shift) - 1);
@@ -233,7 +233,7 @@ IG_DEV int team_phase(const BfsArgs& a, int L, unsigned n, const Team& tm, const
       }
     }
     __syncthreads();
-    if (S.abort_flag) {
+    if (S.stop.at(L)) {
       *aborted = true;
       return L;
     }
@@ -326,6 +326,10 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
         bool aborted = false;
         unsigned last = 0;
         const int L2 = team_phase(a, L, ic.n, tm, in, out, oc, ctl, deadline, &aborted, &last, s_lds.small);
+        if (aborted) {  // (the same in all of a workgroup)
+          if (tid == 0) ctl->status = 1;
+          return;
+        }
         if (tm.rank == 0 && threadIdx.x == 0) {
           st_relaxed(&ctl->level_base, L2);
           st_relaxed(&ctl->last_m, last);

@@ -166,7 +166,7 @@ struct SsspTeamLds {
   int far[2][kFarCap];
   int nfar[2];
   unsigned far_min[2];
-  int abort_flag;
+  PhaseStop stop;
 };
 
 // Wave-collective: parks each lane's vertices u[q] (distance d[q]) with `park` in
@@ -228,7 +228,7 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
   const int t = static_cast<int>(threadIdx.x);
   TeamShare<kShareCap>& F = S.share;
   if (t == 0) {
-    S.abort_flag = 0;
+    S.stop.clear();
     for (int p = 0; p < 2; p++) {
       S.nfar[p] = 0;
       S.far_min[p] = static_cast<unsigned>(kInf);
@@ -244,7 +244,7 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
   // (a share of more vertices than the LDS holds has more entries, too)
   if (sum.most > static_cast<unsigned>(kShareCap)) return true;
   for (;;) {
-    if ((it & 63) == 0 && t == 0) S.abort_flag = kernel_aborted(&ctl->bar, deadline) ? 1 : 0;
+    if ((it & 63) == 0 && t == 0) S.stop.post(it, kernel_aborted(&ctl->bar, deadline));
     *last = sum.total;
     if (sum.total == 0u) {
       // near frontier empty: move the split and re-file the far piles
@@ -343,7 +343,7 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
       }
     }
     __syncthreads();
-    if (S.abort_flag) return false;
+    if (S.stop.at(it - 1)) return false;  // (a turn is one near iteration or split)
     const unsigned long long c = F.cnt[it % 3];
     const bool full = (c & 0xffffffffull) > static_cast<unsigned long long>(kShareCap);
     cn = full ? kShareCap : static_cast<int>(c & 0xffffffffull);
@@ -482,8 +482,9 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
       if (tm.rank >= 0) {
         int it2 = it, T2 = T, epoch2 = epoch;
         unsigned last = 0;
-        const bool ok =
-            team_near(a, it2, n, tm, T2, epoch2, delta, in, out, oc, ctl, deadline, &last, s_lds.small);
+        // (false: the kernel's abort mark is set, and the barrier below says so
+        // to the whole workgroup; a return here spilled 42 registers instead of 15)
+        const bool ok = team_near(a, it2, n, tm, T2, epoch2, delta, in, out, oc, ctl, deadline, &last, s_lds.small);
         if (ok && tm.rank == 0 && threadIdx.x == 0) {
           st_relaxed(&ctl->it_base, it2);
           st_relaxed(&ctl->split_base, T2);

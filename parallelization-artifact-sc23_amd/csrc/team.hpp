@@ -15,6 +15,7 @@
 #pragma once
 
 #include "device_common.hpp"
+#include "phase_stop.hpp"
 
 namespace indigo {
 
