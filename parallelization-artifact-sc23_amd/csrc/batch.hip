@@ -833,6 +833,10 @@ IG_DEV bool run_cc(const BatchTask& T, const Team& tm, unsigned long long (*s_ac
     }
     if (!team_sync(tm)) return false;
     giant = giant_root(T, parent, s_acc);
+    // Nobody links before all have chosen: a member that sampled parents another
+    // had begun to hook could choose another root, and of an edge between the two
+    // roots' trees each end would be skipped, by the member that chose its tree.
+    if (!team_sync(tm)) return false;
   }
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;

@@ -158,6 +158,34 @@ def test_batch_mis_list_lengths(ig, ctx, leaves, cap):
     _check_against_plain(ctx, [g], [dg], qs)
 
 
+@pytest.mark.parametrize("gang", [1, 7, 64, 256])
+@pytest.mark.parametrize("parts, bridges", [(2, 0), (2, 1), (3, 2), (5, 4)])
+def test_batch_cc_large_parts(ig, orc, ctx, parts, bridges, gang):
+    """Components of about the same size on interleaved ids, none or all of them
+    joined by single edges that no end has among its first two entries: the
+    sampled links leave several candidates for the giant root, and only the
+    skipping pass can join them."""
+    rng = np.random.default_rng(parts * 10 + bridges)
+    n = 60000 // parts * parts
+    m = 6 * n // parts
+    src = np.concatenate([rng.integers(0, n // parts, m) * parts + p for p in range(parts)])
+    dst = np.concatenate([rng.integers(0, n // parts, m) * parts + p for p in range(parts)])
+    g = ig.from_edges(n, src.astype(np.int32), dst.astype(np.int32))
+    deg, beg = g.degree, g.nindex
+    mid = np.flatnonzero((deg >= 8) & (np.arange(n) > n // 2))
+    mid = mid[g.nlist[beg[mid] + 1] < n // 2]  # two entries in the lower half: a bridge in the upper half comes later
+    ends = [mid[mid % parts == p][:2] for p in range(parts)]
+    a = np.array([ends[p][0] for p in range(bridges)], np.int32)
+    b = np.array([ends[p + 1][1] for p in range(bridges)], np.int32)
+    g = ig.from_edges(n, np.concatenate([src, a]).astype(np.int32), np.concatenate([dst, b]).astype(np.int32))
+    dg = ig.DeviceGraph(g)
+    want = orc.cc(g)
+    qs = [ig.Query("cc", 0, dg, gang=gang) for _ in range(8)]
+    ctx.batch([dg], qs)
+    for q in qs:
+        assert np.array_equal(q.result(), want)
+
+
 def test_batch_rejects_bad_queries(ig, ctx):
     g = ig.grid(4, 4)
     dg = ig.DeviceGraph(g)
