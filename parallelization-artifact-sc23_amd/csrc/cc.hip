@@ -48,6 +48,10 @@ constexpr int kSample = 2;         // neighbours linked per vertex before the gi
 constexpr int kGiantSamples = 1024;  // vertices sampled to choose it
 constexpr long long kAfforestDeg = 8;  // average degree from which the Afforest order is used
 
+// The trees start as cc_init's chains (find_root's marks).
+IG_DEV int find_v(int* parent, int x) { return find_root<kFindDepth, kFindMark>(parent, x); }
+IG_DEV void link_v(int* parent, int a, int b) { link<kFindDepth, kFindMark>(parent, a, b); }
+
 struct CcControl {
   FrontierCounters heavy;  // deferred long lists (mid / huge queues)
   int giant;               // root of the most frequent component in the sample
@@ -73,14 +77,14 @@ __global__ __launch_bounds__(kCcBlock) void cc_sample(int nodes, const int* __re
 {
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < nodes; v += gridDim.x * blockDim.x) {
     const int beg = nindex[v], end = min(nindex[v + 1], nindex[v] + kSample);
-    for (int e = beg; e < end; e++) link(parent, v, nlist[e]);
+    for (int e = beg; e < end; e++) link_v(parent, v, nlist[e]);
   }
 }
 
 __global__ __launch_bounds__(kCcBlock) void cc_compress(int nodes, int* parent)
 {
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < nodes; v += gridDim.x * blockDim.x)
-    st_relaxed(&parent[v], find_root(parent, v));
+    st_relaxed(&parent[v], find_v(parent, v));
 }
 
 // One workgroup: the most frequent root among kGiantSamples vertices spread
@@ -100,7 +104,7 @@ __global__ __launch_bounds__(kCcBlock) void cc_giant(int nodes, int* parent, CcC
   __syncthreads();
   for (int i = threadIdx.x; i < kGiantSamples; i += blockDim.x) {
     const int v = static_cast<int>((static_cast<unsigned long long>(i) * 2654435761ull) % static_cast<unsigned>(nodes));
-    const int r = find_root(parent, v);
+    const int r = find_v(parent, v);
     int k = static_cast<int>((static_cast<unsigned>(r) * 2654435769u) % kSlots);
     for (;;) {
       const int old = atomicCAS(&s_root[k], -1, r);
@@ -146,7 +150,7 @@ __global__ __launch_bounds__(kCcBlock) void cc_link(int nodes, const int* __rest
     const int beg = valid ? nindex[v] : 0;
     const int deg = valid ? nindex[v + 1] - beg : 0;
     // lists of vertices already joined to the giant root are skipped
-    const bool todo = deg > first && (!kSkip || find_root(parent, v) != giant);
+    const bool todo = deg > first && (!kSkip || find_v(parent, v) != giant);
     const bool long_list = todo && deg >= kMidDeg;
     frontier_emit_block(s_emit, long_list, v, deg, heavy, &ctl->heavy);
     const int rest = todo && !long_list ? deg - first : 0;
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(kCcBlock) void cc_link(int nodes, const int* __rest
       const int ov = c * kWave + o;
       if (k < total) {
         const int u = nlist[obeg + (k - oexcl)];
-        if (kSkip || u < ov) link(parent, ov, u);
+        if (kSkip || u < ov) link_v(parent, ov, u);
       }
     }
   }
@@ -176,7 +180,7 @@ __global__ __launch_bounds__(kCcBlock) void cc_link_heavy(const int* __restrict_
   auto visit = [&](int v, int e, bool active) {
     if (active) {
       const int u = nlist[e];
-      if (kSkip || u < v) link(parent, v, u);
+      if (kSkip || u < v) link_v(parent, v, u);
     }
   };
   expand_huge(heavy, huge_count(hp), huge_chunks(hp), nindex, visit);
@@ -186,7 +190,7 @@ __global__ __launch_bounds__(kCcBlock) void cc_link_heavy(const int* __restrict_
 __global__ __launch_bounds__(kCcBlock) void cc_flatten(int nodes, int* parent, int* label)
 {
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < nodes; v += gridDim.x * blockDim.x)
-    label[v] = find_root(parent, v);
+    label[v] = find_v(parent, v);
 }
 
 int grid_for(long long items, int per_block, int cap = 1 << 20)

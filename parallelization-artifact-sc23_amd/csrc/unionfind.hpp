@@ -19,28 +19,33 @@
 // 0.39 to 0.44 and 0.87 ms; 4-neighbour grid of 1024^2 0.67 -> 0.22.  Depths of 1,
 // 2 and 5 gave 0.83, 0.64 and 0.42 ms on the random graph, 0.225, 0.245 and 0.250
 // on R-MAT 22 (the gangs of a batch, whose vertices fewer lanes share, take 2).
+//   * where trees start as chains (cc.hip hooks every vertex under its smallest
+//     neighbour), a find of more than kFindMark hops also stores the ancestor it has
+//     reached, into its own start vertex and so without a queue.  The finds that pass there
+//     take that far a hop, and the whole chain's finds, all under way at once, end
+//     after a number of steps that is its length's logarithm instead of its root: paths
+//     of 2^16 and 2^20 vertices and a ring of 2^22 0.284, 1.42 and 5.06 ms without
+//     the marks, 0.061, 0.255 and 0.88 with them (path halving: 0.108, 0.73 and 2.5), meshes of
+//     65536 x 16 and 16 x 65536 0.249 and 0.356 -> 0.140 and 0.121, road 2048^2 0.82
+//     either way (marks from 8 and 32 hops on: 0.91 and 0.86; the path of 2^20 0.27 and
+//     0.30).  The edge form and the gangs of a batch start from single vertices and
+//     do without (a gang of one on the 16384 x 64 mesh 31 ms, with marks 50).
 #pragma once
 
 #include "device_common.hpp"
+#include "find_walk.hpp"
 
 namespace indigo {
 
 constexpr int kFindDepth = 5;
+constexpr int kFindMark = 64;
 
-// Root of x.  The store replaces x's parent by one of its ancestors, so
-// concurrent finds and links stay valid (x is no root, so no link writes it).
-template <int kDepth = kFindDepth>
+// Root of x.
+template <int kDepth = kFindDepth, int kMark = 0>
 IG_DEV int find_root(int* parent, int x)
 {
-  int r = x, p = ld_relaxed(&parent[x]);
-  int hops = 0;
-  while (p != r) {
-    r = p;
-    p = ld_relaxed(&parent[r]);
-    hops++;
-  }
-  if (hops > kDepth) st_relaxed(&parent[x], r);
-  return r;
+  return find_walk<kDepth, kMark>(
+      x, [parent](int v) { return ld_relaxed(&parent[v]); }, [parent](int v, int p) { st_relaxed(&parent[v], p); });
 }
 
 // Hooks root hi under lo.  Returns hi on success, where hi points by now if it is
@@ -59,19 +64,19 @@ IG_DEV int hook(int* parent, int hi, int lo)
 
 // Joins the trees of a and b.  (Each round the first lane of every wave that still
 // has something to join either joins it or finds that another wave has.)
-template <int kDepth = kFindDepth>
+template <int kDepth = kFindDepth, int kMark = 0>
 IG_DEV void link(int* parent, int a, int b)
 {
-  int ra = find_root<kDepth>(parent, a);
-  int rb = find_root<kDepth>(parent, b);
+  int ra = find_root<kDepth, kMark>(parent, a);
+  int rb = find_root<kDepth, kMark>(parent, b);
   while (ra != rb) {
     const int hi = ra > rb ? ra : rb;
     const int lo = ra > rb ? rb : ra;
     const int now = hook(parent, hi, lo);
     if (now == hi) return;
     // climb from where hi now points
-    ra = find_root<kDepth>(parent, ra == hi && now >= 0 ? now : ra);
-    rb = find_root<kDepth>(parent, rb == hi && now >= 0 ? now : rb);
+    ra = find_root<kDepth, kMark>(parent, ra == hi && now >= 0 ? now : ra);
+    rb = find_root<kDepth, kMark>(parent, rb == hi && now >= 0 ? now : rb);
   }
 }
 
