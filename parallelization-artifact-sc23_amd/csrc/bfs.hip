@@ -413,7 +413,7 @@ int bfs_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int*
   void* args[] = {&a};
   int grid = 0;
   IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(bfs_kernel), kBfsBlock, 0, args,
-                     graph_grid(edges, kBfsGridPerRoot), &grid, "bfs_kernel"));
+                     graph_grid(nodes, edges, kBfsGridPerRoot), &grid, "bfs_kernel"));
   if (stats) {
     stats->launches = 2;
     stats->grid = grid;

@@ -255,7 +255,7 @@ int mis_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int*
   IG_TRY(zero_async(ctx, a.ctl, sizeof(MisControl)));
   void* args[] = {&a};
   IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(mis_kernel), kMisBlock, 0, args,
-                     graph_grid(edges, kMisGridPerRoot), nullptr, "mis_kernel", true));
+                     graph_grid(nodes, edges, kMisGridPerRoot), nullptr, "mis_kernel", true));
   return INDIGO_OK;
 }
 

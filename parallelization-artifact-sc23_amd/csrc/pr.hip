@@ -459,8 +459,8 @@ int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   IG_TRY(zero_async(ctx, a.ctl, sizeof(PrControl)));
   IG_TRY(zero_async(ctx, a.exit_it, sizeof(int) * kPrMaxGrid));
   void* args[] = {&a};
-  IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(pr_kernel), kPrBlock, 0, args, graph_grid(edges, kPrGridPerRoot), nullptr,
-                     "pr_kernel"));
+  IG_TRY(coop_launch(ctx, reinterpret_cast<const void*>(pr_kernel), kPrBlock, 0, args,
+                     graph_grid(nodes, edges, kPrGridPerRoot), nullptr, "pr_kernel"));
   return INDIGO_OK;
 }
 
