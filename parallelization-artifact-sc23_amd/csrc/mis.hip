@@ -166,7 +166,9 @@ __global__ __launch_bounds__(kMisBlock) __attribute__((amdgpu_waves_per_eu(8, 8)
           beg = a.nindex[v];
           end = a.nindex[v + 1];
           if (end - beg >= kMidDeg) end = beg = -1;
-          else if (beg == end || gs == 0) {
+          // (isolated vertices without the steps below: 2^24 of them 0.147 -> 0.085 ms)
+          else if (beg == end) st_relaxed(&a.status[v], kIncluded);
+          else if (gs == 0) {
             const int st = decide_lane(a, v, beg, end);
             rest = st < 0;
             if (st == kIncluded) {
