@@ -27,6 +27,9 @@ inline int plan_per_cu(int occupancy, int block, int max_threads_per_cu, bool fu
   return n;
 }
 
+// Bound of graph_grid, by which its callers size what they hold per workgroup.
+constexpr int kMaxGraphGrid = 4096;
+
 // Workgroups of a call: the power of two nearest per_root * sqrt(work), at least 64, on a
 // graph of `work` entries.  A small graph's barriers cost more than its lists.
 // Below an average degree of 1.5 the passes over all vertices are the work, at
@@ -38,7 +41,7 @@ inline int graph_grid(int nodes, int edges, double per_root)
 {
   const double want = per_root * std::sqrt(std::max(static_cast<double>(edges), 1.5 * nodes));
   int cap = 64;
-  while (cap < 4096 && cap * 1.41421356 < want) cap *= 2;
+  while (cap < kMaxGraphGrid && cap * 1.41421356 < want) cap *= 2;
   return cap;
 }
 

@@ -48,7 +48,7 @@ constexpr int kPrHugeChunk = 1024;  // entries per item, one wave each
 constexpr int kPrBuckets = 16;      // items are ordered by their first neighbour's part of the ids
 constexpr float kDamp = 0.85f;
 
-constexpr int kPrMaxGrid = 4096;
+constexpr int kPrMaxGrid = kMaxGraphGrid;  // slots of one workgroup each
 
 // Lists of kPrWaveDeg entries up to kPrHugeDeg by length: class c holds those of
 // kPrWaveDeg << c entries up to twice as many.

@@ -37,15 +37,16 @@ int main()
   check(1 << 16, 1 << 10, 0.2, 64);
   // bounds, and the rounding: up from sqrt(2) times a power of two on
   check(1, 0, 0.2, 64);
-  check(1, INT_MAX, 0.4, 4096);
-  check(INT_MAX, 0, 0.4, 4096);
+  check(1, INT_MAX, 0.4, indigo::kMaxGraphGrid);
+  check(INT_MAX, 0, 0.4, indigo::kMaxGraphGrid);
+  check(INT_MAX, INT_MAX, 1e9, indigo::kMaxGraphGrid);
   check(1, 204799, 0.2, 64);
   check(1, 204801, 0.2, 128);
   // never fewer workgroups for more vertices or more entries
   for (int v = 1; v < 1 << 25; v = v * 3 / 2 + 1)
     for (int e = 0; e < 1 << 28; e = e * 3 / 2 + 1) {
       const int g = graph_grid(v, e, 0.2);
-      if (g < 64 || g > 4096 || graph_grid(v, e + 1, 0.2) < g || graph_grid(v + 1, e, 0.2) < g) {
+      if (g < 64 || g > indigo::kMaxGraphGrid || graph_grid(v, e + 1, 0.2) < g || graph_grid(v + 1, e, 0.2) < g) {
         std::fprintf(stderr, "graph_grid(%d, %d) not monotonic or out of range\n", v, e);
         failures++;
       }
