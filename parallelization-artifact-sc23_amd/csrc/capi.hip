@@ -83,6 +83,14 @@ int check_src(int src, int nodes)
   return INDIGO_OK;
 }
 
+// The result `rc` of a call whose kernels have ended; its times are those of
+// this call whether or not it succeeded.
+int call_end(indigo_ctx* ctx, int rc, int launches, int iterations = 0)
+{
+  const int timed = timing_finish(ctx, launches, iterations);
+  return rc != INDIGO_OK ? rc : timed;
+}
+
 // ---- BFS -------------------------------------------------------------------
 int bfs_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* nlist, int src, int* dist,
                double* seconds)
@@ -97,10 +105,10 @@ int bfs_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const i
     IG_TRY(bfs_run(ctx, nodes, edges, nindex, nlist, src, dist, &st));
     IG_TRY(timing_record_stop(ctx));
     const int rc = bfs_collect(ctx, &st);
-    if (rc != kNotResident) IG_TRY(rc);
-    if (rc == INDIGO_OK) break;
+    if (rc == kNotResident) continue;
+    IG_TRY(call_end(ctx, rc, st.launches));
+    break;
   }
-  IG_TRY(timing_finish(ctx, st.launches, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = st.levels;
   return INDIGO_OK;
@@ -121,10 +129,10 @@ int sssp_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const 
     IG_TRY(sssp_run(ctx, nodes, edges, nindex, nlist, eweight, src, dist));
     IG_TRY(timing_record_stop(ctx));
     const int rc = sssp_collect(ctx, &iters, &epochs);
-    if (rc != kNotResident) IG_TRY(rc);
-    if (rc == INDIGO_OK) break;
+    if (rc == kNotResident) continue;
+    IG_TRY(call_end(ctx, rc, 2));
+    break;
   }
-  IG_TRY(timing_finish(ctx, 2, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = iters;
   return INDIGO_OK;
@@ -189,10 +197,10 @@ int mis_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const i
     IG_TRY(mis_run(ctx, nodes, edges, nindex, nlist, signed_priority, status));
     IG_TRY(timing_record_stop(ctx));
     const int rc = mis_collect(ctx, &rounds);
-    if (rc != kNotResident) IG_TRY(rc);
-    if (rc == INDIGO_OK) break;
+    if (rc == kNotResident) continue;
+    IG_TRY(call_end(ctx, rc, 2));
+    break;
   }
-  IG_TRY(timing_finish(ctx, 2, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = rounds;
   return INDIGO_OK;
@@ -211,10 +219,10 @@ int pr_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const in
     IG_TRY(pr_run(ctx, nodes, edges, nindex, nlist, degree, scores, init_uniform));
     IG_TRY(timing_record_stop(ctx));
     const int rc = pr_collect(ctx, &iters, nullptr);
-    if (rc != kNotResident) IG_TRY(rc);
-    if (rc == INDIGO_OK) break;
+    if (rc == kNotResident) continue;
+    IG_TRY(call_end(ctx, rc, 2));
+    break;
   }
-  IG_TRY(timing_finish(ctx, 2, 0));
   if (seconds) *seconds = wall_seconds() - t0;
   ctx->last_iterations = iters;
   if (iterations) *iterations = iters;
@@ -232,8 +240,7 @@ int tc_device(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const in
   SeqArgs a{nodes, edges, nindex, nlist, nullptr, 10};
   IG_TRY(run_captured(ctx, seq_key(ctx, 6, a), tc_sequence, &a));
   IG_TRY(timing_record_stop(ctx));
-  IG_TRY(tc_collect(ctx, count));
-  IG_TRY(timing_finish(ctx, a.launches, 1));
+  IG_TRY(call_end(ctx, tc_collect(ctx, count), a.launches, 1));
   if (seconds) *seconds = wall_seconds() - t0;
   return INDIGO_OK;
 }
