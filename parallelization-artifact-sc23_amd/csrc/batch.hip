@@ -125,6 +125,7 @@ struct BatchTask {
   int2* items;    // heavy-list items (vertex, first entry)
   int item;       // lists of this many entries or more are split into items of as many
   int nsrc;
+  int rows;       // SSSP: sources of one pass, a power of two (scratch_bytes)
   int src[INDIGO_MAX_BFS_SOURCES];
 };
 
@@ -300,6 +301,8 @@ IG_DEV unsigned long long wave_or(unsigned long long x)
 // at a time, and hands over the owner lanes, the neighbours and which of them are
 // there: f(o, u, on), arrays of kFly.
 constexpr int kFly = 2;
+constexpr int kLaneFly = 2;                  // SSSP: sources of an entry that its lane takes alone
+constexpr int kGroupFly = 2;                 // SSSP: steps in flight that take a group of lanes per entry
 
 template <typename F>
 IG_DEV void wave_neighbours_of(int v, bool active, const BatchTask& T, F&& f)
@@ -536,20 +539,18 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
 
 // ---- multi-source SSSP -------------------------------------------------------
 // The distances live vertex-major, row[v * G + i] for source i (G = nsrc rounded up
-// to a power of two), beside the distances at which they were last expanded
-// (done): a queued vertex expands the sources whose distance is below that.  A
-// wave takes the (list entry, source) pairs of its vertices one per lane, all
-// sources of an entry in neighbouring lanes, so only active pairs cost anything
-// and an entry's distances are runs of consecutive words.  With a lane per entry
-// that walked its sources over source-major rows, every distance was a line of
-// its own and each source a chain of three round trips.  Batches of 512 and 24
-// graphs (16 sources each): 805 and 61 -> 376 and 5.7 ms; R-MAT 18 and 14 alone 12.0
-// and 9.1 -> 3.8 and 1.5.  (Deferring distances above a threshold that grows by
-// twice the mean weight over the degree a round saved relaxations but no time.)
-// Vertices with split lists (heavy; for SSSP the lists are split into short items,
-// each entry being nsrc pairs) have their active sources in masks instead, which
-// their items read.  The rows are turned into the output's source-major slab at
-// the end.
+// to a power of two), so an entry's are runs of consecutive words; they are turned into
+// the output's source-major slab at the end.  A queued vertex has its active sources,
+// those whose distance fell in the round before, in a mask.  relax_lists has how a wave
+// takes its vertices' lists.  With a lane per entry that walked its sources over
+// source-major rows, every distance was a line of its own: 1024 queries of 16 sources on
+// random graphs of 2^13 vertices and degree 32 255 ms, now 62; R-MAT 14 97 -> 37; 24 uneven
+// graphs, all algorithms, 61 -> 5.9.  What is bound by latency instead gains little, or
+// loses: gangs of one 0.8 to 1.6 times as fast, 1024 trees of 2^13 vertices with 32 sources,
+// where every distance falls once, 8.3 -> 11.7 ms.  (Deferring distances above a
+// threshold that grows by twice the mean weight over the degree a round saved relaxations
+// but no time.)  Split lists are split into short items, each entry being nsrc pairs.
+// A pass takes T.rows sources.
 
 // The n-th (from 0) set bit of m.
 IG_DEV int nth_bit(unsigned m, int n)
@@ -568,189 +569,263 @@ IG_DEV int nth_bit(unsigned m, int n)
 }
 
 struct SsspRows {
-  int* row;         // [V << shift]
-  int* done;        // [V << shift]
-  unsigned* stamp;  // [V] last round for which the vertex was queued
-  unsigned* mask;   // heavy vertices: sources active in the next round
+  int* row;        // [V << shift]
+  unsigned* mask;  // [V] sources active in the next round
   int shift;
-  unsigned round;  // the next round
   int* qnext;
   unsigned* ncount;
 };
 
-// Wave-collective: relaxes the pairs of each lane's list [beg, beg + len) of vertex v
-// and the sources in m.
-IG_DEV void relax_pairs(const BatchTask& T, const SsspRows& R, int v, int beg, int len, unsigned m,
+constexpr unsigned long long kTwoInf = 0x7fffffff7fffffffull;  // two entries of INT_MAX
+
+IG_DEV int* row_of(const SsspRows& R, int v, int i) { return &R.row[(static_cast<size_t>(v) << R.shift) + i]; }
+
+// A wave's block of 64 list entries: neighbour, weight, owner and the owner's active
+// sources; and the sources for which the neighbour's distance fell.
+struct SsspBlock {
+  int4 entry[kWave];
+  unsigned gain[kWave];
+};
+
+// Wave-collective: relaxes each lane's list [beg, beg + len) of vertex v for the
+// sources in m, in blocks of 64 entries: an entry per lane is looked up, the block's
+// (entry, source) pairs are relaxed, and each entry's improvements are added to its
+// neighbour's mask for the next round, with one atomic and, where the mask was
+// empty, one append to the queue.  (Both with every step of the pairs: a gang of one on
+// a star of 2^18 leaves 19.6 ms for 16 sources, by the block 8.4.)
+//
+// The pairs of a block are taken in one of three ways, by how many sources are active:
+//   * at most kLaneFly per entry: by the entry's lane, all loads in flight together (16
+//     sources on a path: 4.7 us a round by pairs, 3.5);
+//   * half of all: 64 >> shift entries a step, a lane for each source, active or not (what
+//     has not fallen since it was last relaxed improves nothing);
+//   * else exactly the active pairs, one per lane, which finds its entry and source with
+//     7 permutes through LDS (left to the entries' lanes, R-MAT 14 as above took 53 ms).
+// More steps in flight than this spill registers: 24 graphs 5.9 -> 6.2 ms.
+IG_DEV void relax_lists(const BatchTask& T, const SsspRows& R, int v, int beg, int len, unsigned m, SsspBlock& B,
                         BlockQueue<kBatchQueue>& s_next)
 {
   const int lane = lane_id();
-  const int pairs = len * __popc(m);  // (below 1024 * 32)
-  const int incl = wave_inclusive_scan(pairs);
-  const int total = wave_bcast(incl, kWave - 1);
-  for (int base = 0; base < total; base += kFly * kWave) {
-    int u[kFly], nd[kFly], start[kFly];
-    size_t at[kFly];
-    bool on[kFly];
-    unsigned bit[kFly];
-#pragma unroll
-    for (int q = 0; q < kFly; q++) {
-      const int k = base + q * kWave + lane;
-      on[q] = k < total;
-      const int o = min(wave_owner(incl, k), kWave - 1);
-      const unsigned om = static_cast<unsigned>(wave_shfl(static_cast<int>(m), o));
-      const int ov = wave_shfl(v, o), ob = wave_shfl(beg, o);
-      const unsigned rem = static_cast<unsigned>(k - wave_shfl(incl - pairs, o));
-      const unsigned pop = __popc(om);
-      const unsigned entry = on[q] ? rem / pop : 0u;
-      const int rank = static_cast<int>(rem - entry * pop);
-      const int i = nth_bit(om, rank);
-      const int e = on[q] ? ob + static_cast<int>(entry) : 0;
-      start[q] = lane - rank;  // (the lane of the entry's first pair, below 0 in the step before)
-      bit[q] = 1u << i;
-      at[q] = static_cast<size_t>(i);
-      u[q] = on[q] ? T.nlist[e] : 0;
-      nd[q] = on[q] ? T.eweight[e] + ld_relaxed(&R.row[(static_cast<size_t>(ov) << R.shift) + i]) : 0;
+  const int entries = m != 0u ? len : 0;
+  const int incl = wave_inclusive_scan(entries);
+  const int count = wave_bcast(incl, kWave - 1);
+  for (int base = 0; base < count; base += kWave) {
+    const int k = base + lane;
+    const int o = min(wave_owner(incl, k), kWave - 1);
+    const int ov = wave_shfl(v, o);
+    const unsigned om = static_cast<unsigned>(wave_shfl(static_cast<int>(m), o));
+    const int e = wave_shfl(beg - (incl - entries), o) + k;
+    int4 mine = make_int4(0, 0, ov, 0);
+    if (k < count) {
+      mine.x = T.nlist[e];
+      mine.y = T.eweight[e];
+      mine.w = static_cast<int>(om);
     }
+    const int left = min(kWave, count - base);
+    const int pop = __popc(static_cast<unsigned>(mine.w));
+    unsigned gain = 0u;
+    if (__ballot(pop > kLaneFly) == 0ull) {
+      unsigned bits = static_cast<unsigned>(mine.w);
+      int i[kLaneFly], d[kLaneFly], old[kLaneFly];
 #pragma unroll
-    for (int q = 0; q < kFly; q++) {
-      at[q] += static_cast<size_t>(u[q]) << R.shift;
-      on[q] = on[q] && nd[q] < ld_relaxed(&R.row[at[q]]);
-    }
-#pragma unroll
-    for (int q = 0; q < kFly; q++) {
-      const unsigned long long all = __ballot(on[q]);
-      if (all == 0ull) continue;
-      bool first = false;
-      if (on[q]) {
-        // (whether or not this lane's minimum is the one that lowers the
-        // distance: one of this round does)
-        atomic_min_relaxed(&R.row[at[q]], nd[q]);
-        const unsigned queued = ld_relaxed(&R.stamp[u[q]]);
-        if (T.nindex[u[q] + 1] - T.nindex[u[q]] >= T.item)
-          __hip_atomic_fetch_or(&R.mask[u[q]], bit[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // the first improving lane of the entry queues u
-        const unsigned long long run = all & ((1ull << lane) - 1ull) & (~0ull << max(start[q], 0));
-        first = run == 0ull && queued != R.round &&
-                __hip_atomic_exchange(&R.stamp[u[q]], R.round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != R.round;
+      for (int q = 0; q < kLaneFly; q++) {
+        i[q] = bits != 0u ? __ffs(static_cast<int>(bits)) - 1 : 0;
+        d[q] = bits != 0u ? ld_relaxed(row_of(R, ov, i[q])) : 0;
+        old[q] = bits != 0u ? ld_relaxed(row_of(R, mine.x, i[q])) : INT_MIN;
+        bits &= bits - 1u;
       }
-      bq_append(s_next, first, u[q], R.qnext, R.ncount);
+#pragma unroll
+      for (int q = 0; q < kLaneFly; q++) {
+        const int nd = d[q] + mine.y;
+        if (nd < old[q]) {
+          atomic_min_relaxed(row_of(R, mine.x, i[q]), nd);
+          gain |= 1u << i[q];
+        }
+      }
+    } else {
+      B.entry[lane] = mine;
+      B.gain[lane] = 0u;
+      const int pair_incl = wave_inclusive_scan(pop);
+      const int pairs = wave_bcast(pair_incl, kWave - 1);
+      wave_lds_sync();
+      if ((left << R.shift) <= 2 * pairs) {
+        const int per = kWave >> R.shift;  // entries a step
+        const int src = lane & ((1 << R.shift) - 1);
+        const unsigned group = R.shift == 5 ? ~0u : (1u << (1 << R.shift)) - 1u;
+        for (int j = 0; j < left; j += kGroupFly * per) {
+          int at[kGroupFly], d[kGroupFly], old[kGroupFly];
+          int2 to[kGroupFly];  // neighbour, weight
+#pragma unroll
+          for (int q = 0; q < kGroupFly; q++) {
+            at[q] = j + q * per + (lane >> R.shift);
+            const int4 entry = B.entry[min(at[q], kWave - 1)];
+            to[q] = make_int2(entry.x, entry.y);
+            d[q] = at[q] < left ? ld_relaxed(row_of(R, entry.z, src)) : INT_MAX;
+            old[q] = at[q] < left ? ld_relaxed(row_of(R, entry.x, src)) : INT_MIN;
+          }
+#pragma unroll
+          for (int q = 0; q < kGroupFly; q++) {
+            const int nd = d[q] + to[q].y;
+            const bool on = d[q] != INT_MAX && nd < old[q];
+            const unsigned long long all = __ballot(on);
+            if (on) atomic_min_relaxed(row_of(R, to[q].x, src), nd);
+            if (src == 0 && at[q] < left) B.gain[at[q]] = static_cast<unsigned>(all >> lane) & group;
+          }
+        }
+      } else {
+        for (int p0 = 0; p0 < pairs; p0 += kWave) {
+          const int p = p0 + lane;
+          const int at = min(wave_owner(pair_incl, p), kWave - 1);
+          const int rank = p - wave_shfl(pair_incl - pop, at);
+          const int4 entry = B.entry[at];
+          const int i = nth_bit(static_cast<unsigned>(entry.w), rank) & 31;  // (any, past the pairs)
+          const int d = p < pairs ? ld_relaxed(row_of(R, entry.z, i)) : 0;
+          const int old = p < pairs ? ld_relaxed(row_of(R, entry.x, i)) : INT_MIN;
+          if (d + entry.y < old) {
+            atomic_min_relaxed(row_of(R, entry.x, i), d + entry.y);
+            atomicOr(&B.gain[at], 1u << i);
+          }
+        }
+      }
+      wave_lds_sync();
+      gain = B.gain[lane];
     }
+    // (whether or not this wave's minimum is the one that lowered a distance: one of
+    // this round's is)
+    const bool first = gain != 0u && __hip_atomic_fetch_or(&R.mask[mine.x], gain, __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_AGENT) == 0u;
+    bq_append(s_next, first, mine.x, R.qnext, R.ncount);
   }
 }
 
-IG_DEV bool run_sssp(const BatchTask& T, const Team& tm, BlockQueue<kBatchQueue>& s_next)
+// Gang-collective over the members of w: round r over its queue of ncur vertices; *count gets
+// the next one's.
+IG_DEV bool sssp_round(const BatchTask& T, const Team& w, SsspRows& R, unsigned* base, int r, int nitems, int ncur,
+                       int* count, SsspBlock& B, BlockQueue<kBatchQueue>& s_next)
+{
+  const int lane = lane_id();
+  const size_t Vs = static_cast<size_t>(T.nodes);
+  unsigned* act[3] = {base, base + Vs, base + 2 * Vs};  // masks of active sources by round mod 3
+  int* queue[2] = {reinterpret_cast<int*>(base + 3 * Vs), reinterpret_cast<int*>(base + 4 * Vs)};
+  unsigned* qn = w.gs->qn;
+  const Chunks ch = team_chunks(w, T.nodes);
+  unsigned* cur = act[r % 3];
+  const int* qcur = queue[r & 1];
+  R.mask = act[(r + 1) % 3];
+  R.qnext = queue[(r + 1) & 1];
+  R.ncount = &qn[(r + 1) & 3];
+  if (w.rank == 0 && threadIdx.x == 0) st_relaxed(&qn[(r + 2) & 3], 0u);
+  bq_reset(s_next);
+  // few queued vertices: fewer per wave
+  int per = kWave;
+  while (per > 4 && ncur <= per / 2 * ch.step) per /= 2;
+  // the queue, then the items of split lists, a lane each
+  for (int c = ch.first, i0 = ch.first;;) {
+    int v = 0, beg = 0, len = 0;
+    unsigned m = 0u;
+    if (c * per < ncur) {
+      const int k = c * per + lane;
+      if (lane < per && k < ncur) {
+        v = ld_relaxed(&qcur[k]);
+        m = ld_relaxed(&cur[v]);
+        beg = T.nindex[v];
+        len = T.nindex[v + 1] - beg;
+        if (len >= T.item) len = 0;
+        if (len > 0) st_relaxed(&cur[v], 0u);  // (no one else reads it)
+      }
+      c += ch.step;
+    } else if (i0 < nitems) {
+      const int i = i0 + lane * ch.step;
+      if (i < nitems) {
+        v = ld_relaxed(&T.items[i].x);
+        beg = ld_relaxed(&T.items[i].y);
+        m = ld_relaxed(&cur[v]);
+        len = min(T.item, T.nindex[v + 1] - beg);
+        if (beg == T.nindex[v]) st_relaxed(&act[(r + 2) % 3][v], 0u);  // the last round's
+      }
+      i0 += kWave * ch.step;
+    } else {
+      break;
+    }
+    relax_lists(T, R, v, beg, len, m, B, s_next);
+  }
+  bq_flush(s_next, R.qnext, R.ncount);
+  if (!team_sync(w)) return false;
+  *count = static_cast<int>(ld_relaxed(R.ncount));
+  return true;
+}
+
+// One pass: the distances from the sources [s0, s0 + n).
+IG_DEV bool sssp_pass(const BatchTask& T, const Team& tm, int s0, int n, int* nitems, SsspBlock& B,
+                      BlockQueue<kBatchQueue>& s_next)
 {
   const int V = T.nodes;
   const int lane = lane_id();
   const size_t Vs = static_cast<size_t>(V);
-  unsigned* base = static_cast<unsigned*>(T.scratch);
-  unsigned* act[3] = {base, base + Vs, base + 2 * Vs};  // heavy vertices' masks by round mod 3
-  int* queue[3] = {reinterpret_cast<int*>(base + 3 * Vs), reinterpret_cast<int*>(base + 4 * Vs),
-                   reinterpret_cast<int*>(base + 5 * Vs)};
   SsspRows R;
-  R.shift = sssp_row_shift(T.nsrc);
-  R.stamp = base + 6 * Vs;
-  R.row = reinterpret_cast<int*>(base + 7 * Vs);
-  R.done = R.row + (Vs << R.shift);
+  R.shift = sssp_row_shift(T.rows);
+  // (one source a pass: the distances are its slab row)
+  R.row = T.rows == 1 ? T.out + s0 * Vs : static_cast<int*>(T.scratch);
+  unsigned* base = static_cast<unsigned*>(T.scratch) + (T.rows == 1 ? 0 : Vs << R.shift);
   unsigned* qn = tm.gs->qn;
   const Chunks ch = team_chunks(tm, V);
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
     if (v < V) {
-      st_relaxed(&act[0][v], 0u);
-      st_relaxed(&act[1][v], 0u);
-      st_relaxed(&act[2][v], 0u);
-      st_relaxed(&R.stamp[v], 0u);
+      st_relaxed(&base[v], 0u);
+      st_relaxed(&base[Vs + v], 0u);
+      st_relaxed(&base[2 * Vs + v], 0u);
     }
-    const size_t end = min(Vs, static_cast<size_t>(c + 1) * kWave) << R.shift;
-    for (size_t k = (static_cast<size_t>(c) * kWave << R.shift) + lane; k < end; k += kWave) {
-      st_relaxed(&R.row[k], INT_MAX);
-      st_relaxed(&R.done[k], INT_MAX);
+    if (T.rows == 1) {
+      if (v < V) st_relaxed(&R.row[v], INT_MAX);
+    } else {
+      const size_t end = min(Vs, static_cast<size_t>(c + 1) * kWave) << R.shift >> 1;
+      for (size_t k = (static_cast<size_t>(c) * kWave << R.shift >> 1) + lane; k < end; k += kWave)
+        st_relaxed(reinterpret_cast<unsigned long long*>(R.row) + k, kTwoInf);
     }
   }
-  int nitems = 0;
-  if (!build_items(T, tm, &nitems)) return false;
+  if (tm.rank == 0 && threadIdx.x < 4) st_relaxed(&qn[threadIdx.x], 0u);
+  if (s0 == 0) {
+    if (!build_items(T, tm, nitems)) return false;  // (ends with a team barrier)
+  } else if (!team_sync(tm)) {
+    return false;
+  }
   if (tm.rank == 0 && threadIdx.x < kWave) {
-    const bool has = lane < T.nsrc;
-    const int i = lane;
-    const int s = has ? T.src[i] : 0;
+    const bool has = lane < n;
+    const int s = has ? T.src[s0 + lane] : 0;
     unsigned old = 1u;
     if (has) {
-      st_relaxed(&R.row[(static_cast<size_t>(s) << R.shift) + i], 0);
-      old = __hip_atomic_fetch_or(&act[0][s], 1u << i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      st_relaxed(&R.row[(static_cast<size_t>(s) << R.shift) + lane], 0);
+      old = __hip_atomic_fetch_or(&base[s], 1u << lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    wave_append(old == 0u, s, queue[0], &qn[0]);
+    wave_append(old == 0u, s, reinterpret_cast<int*>(base + 3 * Vs), &qn[0]);
   }
   if (!team_sync(tm)) return false;
-  const int G = 1 << R.shift;
-  const int eps = kWave >> R.shift;  // vertices per step of the mask pass
-  const unsigned group = G == 32 ? ~0u : (1u << G) - 1u;
+  int ncur = static_cast<int>(ld_relaxed(&qn[0]));
   for (int r = 0;; r++) {
-    const unsigned* cur = act[r % 3];
-    unsigned* prev = act[(r + 2) % 3];  // round r-1's masks: cleared now
-    const int* qcur = queue[r % 3];
-    const int* qprev = queue[(r + 2) % 3];
-    R.mask = act[(r + 1) % 3];
-    R.qnext = queue[(r + 1) % 3];
-    R.ncount = &qn[(r + 1) & 3];
-    R.round = static_cast<unsigned>(r) + 1u;
-    const int ncur = static_cast<int>(ld_relaxed(&qn[r & 3]));
-    const int nprev = r > 0 && (nitems > 0 || r == 1) ? static_cast<int>(ld_relaxed(&qn[(r + 3) & 3])) : 0;
-    bq_reset(s_next);
-    if (tm.rank == 0 && threadIdx.x == 0) st_relaxed(&qn[(r + 2) & 3], 0u);
-    for (int k = tm.rank * kBatchBlock + static_cast<int>(threadIdx.x); k < nprev; k += tm.size * kBatchBlock)
-      st_relaxed(&prev[ld_relaxed(&qprev[k])], 0u);
-    // few queued vertices: fewer per wave
-    int per = kWave;
-    while (per > 4 && ncur <= per / 2 * ch.step) per /= 2;
-    for (int c = ch.first; c * per < ncur; c += ch.step) {
-      const int k = c * per + lane;
-      const bool a = lane < per && k < ncur;
-      const int v = a ? ld_relaxed(&qcur[k]) : 0;
-      const int beg = a ? T.nindex[v] : 0;
-      const int deg = a ? T.nindex[v + 1] - beg : 0;
-      const int len = deg < T.item ? deg : 0;
-      // the sources whose distance fell since the vertex was last expanded
-      unsigned m = 0u;
-      for (int t = 0; t * eps < per; t++) {
-        const int from = t * eps + (lane >> R.shift);
-        const size_t x = (static_cast<size_t>(wave_shfl(v, from)) << R.shift) + (lane & (G - 1));
-        bool open = wave_shfl(len, from) > 0;
-        if (open) {
-          const int now = ld_relaxed(&R.row[x]);
-          open = now < ld_relaxed(&R.done[x]);
-          if (open) st_relaxed(&R.done[x], now);
-        }
-        const unsigned long long all = __ballot(open);
-        if (lane / eps == t) m = static_cast<unsigned>(all >> ((lane % eps) << R.shift)) & group;
-      }
-      relax_pairs(T, R, v, beg, len, m, s_next);
-    }
-    // items: 64 of the wave's checked at a time
-    const int run = T.item / kWave;  // entries per lane
-    for (int i0 = ch.first; i0 < nitems; i0 += kWave * ch.step) {
-      const int i = i0 + lane * ch.step;
-      const int v = i < nitems ? ld_relaxed(&T.items[i].x) : 0;
-      const int eb = i < nitems ? ld_relaxed(&T.items[i].y) : 0;
-      const unsigned m = i < nitems ? ld_relaxed(&cur[v]) : 0u;
-      for (unsigned long long left = __ballot(m != 0u); left != 0ull; left &= left - 1ull) {
-        const int from = __ffsll(static_cast<long long>(left)) - 1;
-        const int iv = wave_bcast(v, from), b = wave_bcast(eb, from) + lane * run;
-        const int end = min(wave_bcast(eb, from) + T.item, T.nindex[iv + 1]);
-        relax_pairs(T, R, iv, b, max(0, min(run, end - b)), static_cast<unsigned>(wave_bcast(static_cast<int>(m), from)),
-                    s_next);
-      }
-    }
-    bq_flush(s_next, R.qnext, R.ncount);
-    if (!team_sync(tm)) return false;
-    if (ld_relaxed(R.ncount) == 0u) break;
+    int count = 0;
+    if (!sssp_round(T, tm, R, base, r, *nitems, ncur, &count, B, s_next)) return false;
+    if (count == 0) break;
+    ncur = count;
   }
+  if (T.rows == 1) return true;
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
     if (v >= V) continue;
-    for (int i = 0; i < T.nsrc; i++)
-      T.out[static_cast<size_t>(i) * V + v] = ld_relaxed(&R.row[(static_cast<size_t>(v) << R.shift) + i]);
+    for (int i = 0; i < n; i += 2) {
+      const unsigned long long two = ld_relaxed(reinterpret_cast<unsigned long long*>(row_of(R, v, i)));
+      T.out[(s0 + i) * Vs + v] = static_cast<int>(two);
+      if (i + 1 < n) T.out[(s0 + i + 1) * Vs + v] = static_cast<int>(two >> 32);
+    }
   }
+  return true;
+}
+
+IG_DEV bool run_sssp(const BatchTask& T, const Team& tm, SsspBlock* s_block, BlockQueue<kBatchQueue>& s_next)
+{
+  int nitems = 0;
+  for (int s0 = 0; s0 < T.nsrc; s0 += T.rows)
+    if (!sssp_pass(T, tm, s0, min(T.rows, T.nsrc - s0), &nitems, s_block[threadIdx.x / kWave], s_next)) return false;
   return true;
 }
 
@@ -1063,7 +1138,10 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 
                                                             long long residency_ticks)
 {
   __shared__ int s_task, s_rank;
-  __shared__ unsigned long long s_acc[kBatchWaves][kWave];
+  __shared__ union {
+    unsigned long long acc[kBatchWaves][kWave];  // BFS, CC
+    SsspBlock block[kBatchWaves];                // SSSP
+  } s_wave;
   __shared__ double s_red[kBatchWaves];
   __shared__ BlockQueue<kBatchQueue> s_next;
   __shared__ BlockSum s_mf;
@@ -1095,39 +1173,58 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(8, 
     const Team tm{rank, min(T.gang, static_cast<int>(gridDim.x)), &gangs[t], &ctl->bar, deadline};
     if (!team_sync(tm)) break;  // the gang assembles
     bool ok = true;
-    if (T.alg == INDIGO_QUERY_BFS) ok = run_bfs(T, tm, s_acc, s_next, s_mf);
-    else if (T.alg == INDIGO_QUERY_SSSP) ok = run_sssp(T, tm, s_next);
-    else if (T.alg == INDIGO_QUERY_CC) ok = run_cc(T, tm, s_acc);
+    if (T.alg == INDIGO_QUERY_BFS) ok = run_bfs(T, tm, s_wave.acc, s_next, s_mf);
+    else if (T.alg == INDIGO_QUERY_SSSP) ok = run_sssp(T, tm, s_wave.block, s_next);
+    else if (T.alg == INDIGO_QUERY_CC) ok = run_cc(T, tm, s_wave.acc);
     else if (T.alg == INDIGO_QUERY_PR) ok = run_pr(T, tm, s_red);
     else ok = run_mis(T, tm);
     if (!ok) break;
   }
 }
 
+// Sources that one pass of an SSSP takes, at most `most` (a power of two).
+int pass_rows(const indigo_query& Q, int most)
+{
+  return Q.alg == INDIGO_QUERY_SSSP ? std::min(1 << sssp_row_shift(Q.nsrc), most) : 1;
+}
+
 // Entries per item: lists that long tie a wave up.  An entry of a multi-source SSSP
 // is a pair per source, so its items hold about kItem pairs.
-int item_entries(int alg, int nsrc)
+int item_entries(int alg, int rows)
 {
-  return alg == INDIGO_QUERY_SSSP ? std::max(kWave, kItem >> sssp_row_shift(nsrc)) : kItem;
+  return alg == INDIGO_QUERY_SSSP ? std::max(kWave, kItem >> sssp_row_shift(rows)) : kItem;
 }
 
 size_t items_cap(int edges, int item) { return 2 * (static_cast<size_t>(edges) / item) + 2; }
 
 // Per-task scratch: the algorithm's arrays (alg_bytes), then the heavy items.
-size_t alg_bytes(int alg, int nodes, int edges, int nsrc)
+size_t alg_bytes(int alg, int nodes, int edges, int rows)
 {
   const size_t v = static_cast<size_t>(nodes);
   size_t b = 0;
   if (alg == INDIGO_QUERY_BFS) b = 4 * v * 8 + 2 * v * 4;             // seen, 2 frontiers, next; 2 queues
-  else if (alg == INDIGO_QUERY_SSSP) b = 7 * v * 4 + ((2 * v * 4) << sssp_row_shift(nsrc));  // 3 masks, 3 queues, stamps; rows
+  else if (alg == INDIGO_QUERY_SSSP) b = 5 * v * 4 + (rows == 1 ? 0 : v * 4 * rows);  // 3 masks, 2 queues; rows
   else if (alg == INDIGO_QUERY_MIS) b = 2 * v * 4;                   // heavy-vertex flags
   else if (alg == INDIGO_QUERY_PR) b = 2 * kMaxGang * 8 + 2 * v * 4 + items_cap(edges, kItem) * 8;  // slots, contrib, partials
   return Carver::round(b);
 }
 
-size_t scratch_bytes(int alg, int nodes, int edges, int nsrc)
+size_t scratch_bytes(int alg, int nodes, int edges, int rows)
 {
-  return alg_bytes(alg, nodes, edges, nsrc) + Carver::round(items_cap(edges, item_entries(alg, nsrc)) * sizeof(int2));
+  return alg_bytes(alg, nodes, edges, rows) + Carver::round(items_cap(edges, item_entries(alg, rows)) * sizeof(int2));
+}
+
+// Workspace of a batch whose SSSPs take at most `most` sources a pass.
+size_t workspace_bytes(const indigo_graph_ref* graphs, const indigo_query* queries, int nqueries, int most)
+{
+  const size_t n = static_cast<size_t>(nqueries);
+  size_t bytes = Carver::round(sizeof(BatchControl)) + Carver::round(n * sizeof(GangState)) +
+                 Carver::round(n * sizeof(BatchTask)) + 4096;
+  for (int q = 0; q < nqueries; q++) {
+    const indigo_graph_ref& G = graphs[queries[q].graph];
+    bytes += scratch_bytes(queries[q].alg, G.nodes, G.edges, pass_rows(queries[q], most));
+  }
+  return bytes;
 }
 
 }  // namespace
@@ -1312,20 +1409,15 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
                                   : gang_for(queries[q].alg, G.nodes, G.edges, grid_cap);
   }
   widen_gangs(gang, graphs, queries, grid_cap);
-  size_t scratch_total = 0;
-  for (int q = 0; q < nqueries; q++)
-    scratch_total += scratch_bytes(queries[q].alg, graphs[queries[q].graph].nodes, graphs[queries[q].graph].edges,
-                                   queries[q].nsrc);
   const size_t n = static_cast<size_t>(nqueries);
-  const size_t bytes = Carver::round(sizeof(BatchControl)) + Carver::round(n * sizeof(GangState)) +
-                       Carver::round(n * sizeof(BatchTask)) + scratch_total + 4096;
-  IG_TRY(ensure_workspace(ctx, bytes));
+  const int most = INDIGO_MAX_SSSP_SOURCES;
+  IG_TRY(ensure_workspace(ctx, workspace_bytes(graphs, queries, nqueries, most)));
   IG_TRY(ensure_host_pinned(ctx, n * sizeof(BatchTask)));
   Carver cv(ctx->ws);
   BatchControl* ctl = cv.take<BatchControl>(1);
   GangState* gangs = cv.take<GangState>(n);
   BatchTask* d_tasks = cv.take<BatchTask>(n);
-  unsigned char* scratch = cv.take<unsigned char>(scratch_total + 256);
+  unsigned char* scratch = cv.take<unsigned char>(0);
   BatchTask* h_tasks = static_cast<BatchTask*>(ctx->host_pinned);
   size_t off = 0;
   for (size_t i = 0; i < n; i++) {
@@ -1337,14 +1429,15 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
     T.gang = gang[order[i]];
     T.nodes = G.nodes;
     T.edges = G.edges;
-    T.item = item_entries(Q.alg, Q.nsrc);
+    T.rows = pass_rows(Q, most);
+    T.item = item_entries(Q.alg, T.rows);
     T.nindex = G.d_nindex;
     T.nlist = G.d_nlist;
     T.eweight = G.d_eweight;
     T.out = Q.d_out;
     T.scratch = scratch + off;
-    T.items = reinterpret_cast<int2*>(scratch + off + alg_bytes(Q.alg, G.nodes, G.edges, Q.nsrc));
-    off += scratch_bytes(Q.alg, G.nodes, G.edges, Q.nsrc);
+    T.items = reinterpret_cast<int2*>(scratch + off + alg_bytes(Q.alg, G.nodes, G.edges, T.rows));
+    off += scratch_bytes(Q.alg, G.nodes, G.edges, T.rows);
     T.nsrc = (Q.alg == INDIGO_QUERY_BFS || Q.alg == INDIGO_QUERY_SSSP) ? Q.nsrc : 0;
     for (int s = 0; s < T.nsrc; s++) T.src[s] = Q.src[s];
   }
