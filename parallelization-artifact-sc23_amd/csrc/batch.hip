@@ -550,7 +550,7 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
 // where every distance falls once, 8.3 -> 11.7 ms.  (Deferring distances above a
 // threshold that grows by twice the mean weight over the degree a round saved relaxations
 // but no time.)  Split lists are split into short items, each entry being nsrc pairs.
-// A pass takes T.rows sources.
+// Sources are taken T.rows at a time, all of them where the rows fit the memory.
 
 // The n-th (from 0) set bit of m.
 IG_DEV int nth_bit(unsigned m, int n)
@@ -1239,6 +1239,11 @@ static int gang_cap(int alg, int nodes, int edges, bool widen)
   return static_cast<long long>(edges) < 6LL * nodes ? 16 : 128;
 }
 
+size_t batch_workspace_bytes(const indigo_graph_ref* graphs, const indigo_query* queries, int nqueries)
+{
+  return workspace_bytes(graphs, queries, nqueries, INDIGO_MAX_SSSP_SOURCES);
+}
+
 int batch_gang(int alg, int nodes, int edges)
 {
   if (alg < INDIGO_QUERY_BFS || alg > INDIGO_QUERY_PR || nodes < 0 || edges < 0) return 0;
@@ -1410,8 +1415,16 @@ int batch_launch(indigo_ctx* ctx, const indigo_graph_ref* graphs, int ngraphs, c
   }
   widen_gangs(gang, graphs, queries, grid_cap);
   const size_t n = static_cast<size_t>(nqueries);
-  const int most = INDIGO_MAX_SSSP_SOURCES;
-  IG_TRY(ensure_workspace(ctx, workspace_bytes(graphs, queries, nqueries, most)));
+  // SSSPs of several sources take passes of half as many while their rows do not
+  // fit the memory (one source a pass needs 20 bytes a vertex)
+  int most = INDIGO_MAX_SSSP_SOURCES;
+  for (;;) {
+    const int rc = ensure_workspace(ctx, workspace_bytes(graphs, queries, nqueries, most));
+    if (rc == INDIGO_OK) break;
+    if (rc != INDIGO_ERR_OUT_OF_MEMORY || most == 1) return rc;
+    clear_error();
+    most /= 2;
+  }
   IG_TRY(ensure_host_pinned(ctx, n * sizeof(BatchTask)));
   Carver cv(ctx->ws);
   BatchControl* ctl = cv.take<BatchControl>(1);

@@ -20,6 +20,9 @@ int batch_wait(indigo_ctx* ctx);
 // Workgroups that any persistent kernel of the library can keep resident on
 // the whole device (the base of the serving slots' shares).
 int batch_grid_limit(indigo_ctx* ctx, int* limit);
+// Workspace that a launch of these queries (alg, graph and nsrc suffice) takes where the memory
+// allows; with less, SSSPs of several sources take several passes.
+size_t batch_workspace_bytes(const indigo_graph_ref* graphs, const indigo_query* queries, int nqueries);
 // The engine's gang size for a query (before clamping to the grid).
 int batch_gang(int alg, int nodes, int edges);
 

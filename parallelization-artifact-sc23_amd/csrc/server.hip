@@ -205,6 +205,41 @@ struct Server {
 
   bool is_long(const indigo_request& r) const { return est_us(r) > kLongUs; }
 
+  // Workspace of the largest batched launch that max_batch requests arriving one after the
+  // other can make (BFS and SSSP requests on the same graph merged as in dispatch_batch).
+  size_t batch_bytes() const
+  {
+    std::vector<int> order;
+    for (int i = 0; i < nreqs; i++)
+      if (reqs[i].alg != INDIGO_QUERY_TC && !single(reqs[i])) order.push_back(i);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return reqs[a].arrival < reqs[b].arrival; });
+    const size_t window = static_cast<size_t>(std::max(1, cfg.max_batch));
+    size_t most = 0;
+    std::vector<indigo_query> queries;
+    for (size_t from = 0; from < order.size(); from += std::max<size_t>(1, window / 2)) {
+      std::map<std::pair<int, int>, size_t> open;
+      queries.clear();
+      for (size_t i = from; i < std::min(order.size(), from + window); i++) {
+        const indigo_request& r = reqs[order[i]];
+        const bool multi = r.alg == INDIGO_QUERY_BFS || r.alg == INDIGO_QUERY_SSSP;
+        const int cap = r.alg == INDIGO_QUERY_BFS ? INDIGO_MAX_BFS_SOURCES : INDIGO_MAX_SSSP_SOURCES;
+        const auto it = multi ? open.find({r.alg, r.graph}) : open.end();
+        if (it != open.end() && queries[it->second].nsrc < cap) {
+          queries[it->second].nsrc++;
+          continue;
+        }
+        indigo_query q{};
+        q.alg = r.alg;
+        q.graph = r.graph;
+        q.nsrc = 1;
+        if (multi) open[{r.alg, r.graph}] = queries.size();
+        queries.push_back(q);
+      }
+      most = std::max(most, batch_workspace_bytes(graphs, queries.data(), static_cast<int>(queries.size())));
+    }
+    return most;
+  }
+
   size_t out_bytes(const indigo_request& r) const
   {
     const size_t v = static_cast<size_t>(graphs[r.graph].nodes);
@@ -522,8 +557,9 @@ int serve_run(const indigo_graph_ref* graphs, int ngraphs, indigo_request* reqs,
     // the GPU is shared: give persistent grids time to assemble
     s.ctx->hints[INDIGO_HINT_RESIDENCY_MS] = 2000;
   }
-  // workspaces sized up front for the largest triangle count, so that no
-  // slot reallocates (hipFree waits for the device) while others run
+  // workspaces sized up front for the largest triangle count, single query and
+  // batch, so that no slot reallocates (hipFree waits for the device) while others run; a
+  // batch's, where it does not fit, grows with the launches that need it
   size_t ws = 0;
   for (int i = 0; i < nreqs; i++)
   {
@@ -531,8 +567,17 @@ int serve_run(const indigo_graph_ref* graphs, int ngraphs, indigo_request* reqs,
     if (reqs[i].alg == INDIGO_QUERY_TC) ws = std::max(ws, tc_workspace_bytes(G.nodes, G.edges));
     if (sv.single(reqs[i])) ws = std::max(ws, sv.single_workspace_bytes(reqs[i]));
   }
+  ws = std::max(ws, size_t(1) << 28);
   for (Slot& s : sv.slots)
-    if (rc == INDIGO_OK && s.ctx != nullptr) rc = ensure_workspace(s.ctx, std::max(ws, size_t(1) << 28));
+    if (rc == INDIGO_OK && s.ctx != nullptr) rc = ensure_workspace(s.ctx, ws);
+  const size_t batch = sv.batch_bytes();
+  for (size_t i = 0; rc == INDIGO_OK && batch > ws && i < sv.slots.size(); i++) {
+    rc = ensure_workspace(sv.slots[i].ctx, batch);
+    if (rc != INDIGO_ERR_OUT_OF_MEMORY) continue;
+    clear_error();
+    rc = ensure_workspace(sv.slots[i].ctx, ws);
+    break;
+  }
   int limit = 0;
   if (rc == INDIGO_OK) rc = batch_grid_limit(sv.slots[0].ctx, &limit);
   sv.grid_per_slot = std::max(1, limit / nslots);
