@@ -290,17 +290,34 @@ IG_DEV void set_flag(unsigned* flag, bool any)
   if (__ballot(any) != 0ull && lane_id() == 0) st_relaxed(flag, 1u);
 }
 
+// Or of the 64 lanes' words, the same in all (all lanes must be active): the steps of
+// wave_inclusive_scan, whose last lane has the whole.
+IG_DEV unsigned wave_or32(unsigned x)
+{
+  int y = static_cast<int>(x);
+  y |= __builtin_amdgcn_update_dpp(0, y, 0x111, 0xf, 0xf, false);  // row_shr:1
+  y |= __builtin_amdgcn_update_dpp(0, y, 0x112, 0xf, 0xf, false);  // row_shr:2
+  y |= __builtin_amdgcn_update_dpp(0, y, 0x114, 0xf, 0xf, false);  // row_shr:4
+  y |= __builtin_amdgcn_update_dpp(0, y, 0x118, 0xf, 0xf, false);  // row_shr:8
+  y |= __builtin_amdgcn_update_dpp(0, y, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  y |= __builtin_amdgcn_update_dpp(0, y, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return static_cast<unsigned>(wave_bcast(y, kWave - 1));
+}
+
 IG_DEV unsigned long long wave_or(unsigned long long x)
 {
-#pragma unroll
-  for (int d = kWave / 2; d > 0; d >>= 1) x |= __shfl_xor(x, d, kWave);
-  return x;
+  return static_cast<unsigned long long>(wave_or32(static_cast<unsigned>(x >> 32))) << 32 |
+         wave_or32(static_cast<unsigned>(x));
 }
 
 // Wave-collective: walks the lists as wave_entries_of does, kFly entries per lane
 // at a time, and hands over the owner lanes, the neighbours and which of them are
 // there: f(o, u, on), arrays of kFly.
 constexpr int kFly = 2;
+// BFS: entries of a narrow level, for one member (one step of 64 per wave; below kHeavyDeg);
+// SSSP: vertices of a narrow round, left again above four times as many.
+constexpr unsigned long long kNarrow = 512;
+constexpr int kNarrowQueue = 32;
 constexpr int kLaneFly = 2;                  // SSSP: sources of an entry that its lane takes alone
 constexpr int kGroupFly = 2;                 // SSSP: steps in flight that take a group of lanes per entry
 
@@ -353,12 +370,18 @@ IG_DEV void item_neighbours(int eb, int ee, const BatchTask& T, F&& f)
 // them in order) go out together.
 IG_DEV void write_rows(const BatchTask& T, unsigned long long m, int v, int level)
 {
+  // ... and few sources per vertex each lane its own: a path's frontier of 128 vertices for
+  // 64 64 sources cost a BFS 64 turns of the wave a level (10.5 -> 7.8 us).
   unsigned long long rows = wave_or(m);
-  rows = static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(static_cast<int>(rows >> 32))) << 32 |
-         static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(rows)));
-  for (; rows != 0ull; rows &= rows - 1ull) {
-    const int i = __ffsll(static_cast<long long>(rows)) - 1;
-    if (m >> i & 1ull) T.out[static_cast<size_t>(i) * T.nodes + v] = level;
+  const int bits = wave_bcast(wave_inclusive_scan(__popcll(m)), kWave - 1);
+  if (4 * bits >= kWave * __popcll(rows)) {
+    for (; rows != 0ull; rows &= rows - 1ull) {
+      const int i = __ffsll(static_cast<long long>(rows)) - 1;
+      if (m >> i & 1ull) T.out[static_cast<size_t>(i) * T.nodes + v] = level;
+    }
+  } else {
+    for (; m != 0ull; m &= m - 1ull)
+      T.out[static_cast<size_t>(__ffsll(static_cast<long long>(m)) - 1) * T.nodes + v] = level;
   }
 }
 
@@ -366,8 +389,12 @@ IG_DEV void write_rows(const BatchTask& T, unsigned long long m, int v, int leve
 // level and their degree sum are gathered in LDS and registers instead of two
 // atomics and a 64-bit wave sum a step, two entries per lane are in flight and the
 // levels are written a row at a time: 100 graphs of 64 sources 32.6 -> 27.2 ms.
-IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_acc)[kWave],
-                    BlockQueue<kBatchQueue>& s_next, BlockSum& s_mf)
+// Gang-collective over the members of w: level lvl from its frontier of ncur vertices with
+// mcur entries; *count and *entries get the next one's, which each member has read when
+// the level ends.
+IG_DEV bool bfs_level(const BatchTask& T, const Team& w, int lvl, int nitems, unsigned long long all, int ncur,
+                      unsigned long long mcur, int* count, unsigned long long* entries,
+                      unsigned long long (*s_acc)[kWave], BlockQueue<kBatchQueue>& s_next, BlockSum& s_mf)
 {
   const int V = T.nodes;
   const int lane = lane_id();
@@ -377,6 +404,152 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
   unsigned long long* fr[2] = {seen + Vs, seen + 2 * Vs};  // frontier masks by level parity
   unsigned long long* nxt = seen + 3 * Vs;                 // next-level masks
   int* queue[2] = {reinterpret_cast<int*>(seen + 4 * Vs), reinterpret_cast<int*>(seen + 4 * Vs) + V};
+  unsigned* qn = w.gs->qn;
+  unsigned long long* mf = w.gs->mf;
+  const Chunks ch = team_chunks(w, V);
+  const unsigned long long* cur = fr[(lvl - 1) & 1];
+  unsigned long long* nfr = fr[lvl & 1];
+  const int* qcur = queue[(lvl - 1) & 1];
+  int* qnext = queue[lvl & 1];
+  unsigned* ncount = &qn[lvl & 3];
+  unsigned long long* nmf = &mf[lvl & 3];
+  if (w.rank == 0 && threadIdx.x == 0) {
+    st_relaxed(&qn[(lvl + 1) & 3], 0u);
+    st_relaxed(&mf[(lvl + 1) & 3], 0ull);
+  }
+  // Narrow levels append straight to the queue: the buffer's four workgroup barriers cost
+  // them more than its atomics save (path of 2^15 vertices, one workgroup: 2.8 -> 2.6 us a level).
+  const bool direct = mcur <= kNarrow * static_cast<unsigned long long>(w.size);
+  if (!direct) {
+    if (threadIdx.x == 0) s_mf.v = 0ull;
+    bq_reset(s_next);
+  }
+  int dsum = 0;  // degrees of what this lane appends
+  auto append = [&](bool first, int u) {
+    if (first) dsum += T.nindex[u + 1] - T.nindex[u];
+    if (direct) wave_append(first, u, qnext, ncount);
+    else bq_append(s_next, first, u, qnext, ncount);
+  };
+  if (mcur * 14ull < static_cast<unsigned long long>(T.edges)) {
+    // push from the frontier queue
+    const int nq = (ncur + kWave - 1) / kWave;
+    auto push = [&](const unsigned long long (&m)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+      unsigned long long add[kFly];
+      bool first[kFly];
+#pragma unroll
+      for (int q = 0; q < kFly; q++) add[q] = on[q] ? m[q] & ~ld_relaxed(&seen[u[q]]) : 0ull;
+#pragma unroll
+      for (int q = 0; q < kFly; q++)
+        first[q] = add[q] != 0ull && __hip_atomic_fetch_or(&nxt[u[q]], add[q], __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_AGENT) == 0ull;
+#pragma unroll
+      for (int q = 0; q < kFly; q++) append(first[q], u[q]);
+    };
+    for (int c = ch.first; c < nq; c += ch.step) {
+      const int k = c * kWave + lane;
+      const bool act = k < ncur;
+      const int v = act ? ld_relaxed(&qcur[k]) : 0;
+      const unsigned long long m = act ? ld_relaxed(&cur[v]) : 0ull;
+      wave_neighbours_of(v, act, T, [&](const int (&o)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+        unsigned long long om[kFly];
+#pragma unroll
+        for (int q = 0; q < kFly; q++) om[q] = __shfl(m, o[q], kWave);
+        push(om, u, on);
+      });
+    }
+    // (a heavy vertex alone has kHeavyDeg entries)
+    if (mcur >= static_cast<unsigned long long>(kHeavyDeg)) for_items(T, w, nitems, [&](int v, int eb, int ee, int) {
+      const unsigned long long m = ld_relaxed(&cur[v]);
+      if (m == 0ull) return;
+      item_neighbours(eb, ee, T, [&](const int (&)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+        unsigned long long om[kFly];
+#pragma unroll
+        for (int q = 0; q < kFly; q++) om[q] = m;
+        push(om, u, on);
+      });
+    });
+  } else {
+    // pull: every vertex with sources still missing
+    for (int c = ch.first; c < ch.count; c += ch.step) {
+      const int v = c * kWave + lane;
+      const unsigned long long sv = v < V ? ld_relaxed(&seen[v]) : all;
+      const unsigned long long missing = all & ~sv;
+      s_acc[wid][lane] = 0ull;
+      wave_lds_sync();
+      wave_neighbours_of(v, missing != 0ull, T, [&](const int (&o)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+        unsigned long long m[kFly];
+#pragma unroll
+        for (int q = 0; q < kFly; q++) m[q] = on[q] ? ld_relaxed(&cur[u[q]]) : 0ull;
+#pragma unroll
+        for (int q = 0; q < kFly; q++)
+          if (m[q] != 0ull) atomicOr(&s_acc[wid][o[q]], m[q]);
+      });
+      wave_lds_sync();
+      const unsigned long long nb = s_acc[wid][lane] & missing;
+      if (nb != 0ull) st_relaxed(&nxt[v], nb);
+      append(nb != 0ull, v);
+    }
+    for_items(T, w, nitems, [&](int v, int eb, int ee, int) {
+      const unsigned long long missing = all & ~ld_relaxed(&seen[v]);
+      if (missing == 0ull) return;
+      unsigned long long acc = 0ull;
+      item_neighbours(eb, ee, T, [&](const int (&)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
+        unsigned long long m[kFly];
+#pragma unroll
+        for (int q = 0; q < kFly; q++) m[q] = on[q] ? ld_relaxed(&cur[u[q]]) : 0ull;
+#pragma unroll
+        for (int q = 0; q < kFly; q++) acc |= m[q];
+      });
+      const unsigned long long nb = wave_or(acc) & missing;
+      bool first = false;
+      if (nb != 0ull && lane == 0)
+        first = __hip_atomic_fetch_or(&nxt[v], nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0ull;
+      append(first, v);
+    });
+  }
+  // (a vertex is appended once a level: the sum stays below 2^31)
+  const int degrees = wave_bcast(wave_inclusive_scan(dsum), kWave - 1);
+  if (direct) {
+    if (degrees != 0 && lane == 0) atomic_add_relaxed(nmf, static_cast<unsigned long long>(degrees));
+  } else {
+    if (degrees != 0 && lane == 0) atomicAdd(&s_mf.v, static_cast<unsigned long long>(degrees));
+    bq_flush<false>(s_next, qnext, ncount);
+    if (threadIdx.x == 0 && s_mf.v != 0ull) atomic_add_relaxed(nmf, s_mf.v);
+  }
+  if (!team_sync(w)) return false;
+  // the new frontier: masks, seen bits and levels; the old frontier's masks
+  // are cleared (that buffer holds the next level's frontier)
+  const int nnext = static_cast<int>(ld_relaxed(ncount));
+  *count = nnext;
+  *entries = ld_relaxed(nmf);
+  for (int k = w.rank * kBatchBlock + static_cast<int>(threadIdx.x); k < ncur; k += w.size * kBatchBlock)
+    st_relaxed(&fr[(lvl - 1) & 1][ld_relaxed(&qcur[k])], 0ull);
+  for (int c = ch.first; c * kWave < nnext; c += ch.step) {
+    const int k = c * kWave + lane;
+    const int u = k < nnext ? ld_relaxed(&qnext[k]) : 0;
+    unsigned long long nb = 0ull;
+    if (k < nnext) {
+      const unsigned long long sv = ld_relaxed(&seen[u]);
+      nb = ld_relaxed(&nxt[u]) & ~sv;
+      st_relaxed(&nxt[u], 0ull);
+      st_relaxed(&seen[u], sv | nb);
+      st_relaxed(&nfr[u], nb);
+    }
+    write_rows(T, nb, u, lvl);
+  }
+  return team_sync(w);
+}
+
+IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_acc)[kWave],
+                    BlockQueue<kBatchQueue>& s_next, BlockSum& s_mf)
+{
+  const int V = T.nodes;
+  const int lane = lane_id();
+  const size_t Vs = static_cast<size_t>(V);
+  unsigned long long* seen = static_cast<unsigned long long*>(T.scratch);
+  unsigned long long* fr[2] = {seen + Vs, seen + 2 * Vs};  // frontier masks by level parity
+  unsigned long long* nxt = seen + 3 * Vs;                 // next-level masks
+  int* queue0 = reinterpret_cast<int*>(seen + 4 * Vs);
   unsigned* qn = tm.gs->qn;
   unsigned long long* mf = tm.gs->mf;
   const unsigned long long all = T.nsrc >= 64 ? ~0ull : ((1ull << T.nsrc) - 1ull);
@@ -404,131 +577,38 @@ IG_DEV bool run_bfs(const BatchTask& T, const Team& tm, unsigned long long (*s_a
     }
     // a source listed twice is queued by the lane that set its first bit
     const bool first = has && old == 0ull;
-    wave_append(first, s, queue[0], &qn[0]);
+    wave_append(first, s, queue0, &qn[0]);
     const unsigned long long d = wave_sum(static_cast<unsigned long long>(first ? T.nindex[s + 1] - T.nindex[s] : 0));
     if (lane == 0) atomic_add_relaxed(&mf[0], d);
   }
   if (!team_sync(tm)) return false;
+  int ncur = static_cast<int>(ld_relaxed(&qn[0]));
+  unsigned long long mcur = ld_relaxed(&mf[0]);
+  // (member 0 may go ahead from here: all have read the counters)
+  if (tm.size > 1 && !team_sync(tm)) return false;
   for (int lvl = 1;; lvl++) {
-    const unsigned long long* cur = fr[(lvl - 1) & 1];
-    unsigned long long* nfr = fr[lvl & 1];
-    const int* qcur = queue[(lvl - 1) & 1];
-    int* qnext = queue[lvl & 1];
-    unsigned* ncount = &qn[lvl & 3];
-    unsigned long long* nmf = &mf[lvl & 3];
-    const int ncur = static_cast<int>(ld_relaxed(&qn[(lvl - 1) & 3]));
-    const unsigned long long mcur = ld_relaxed(&mf[(lvl - 1) & 3]);
-    if (tm.rank == 0 && threadIdx.x == 0) {
-      st_relaxed(&qn[(lvl + 1) & 3], 0u);
-      st_relaxed(&mf[(lvl + 1) & 3], 0ull);
+    // narrow levels are member 0's, at workgroup barriers, until one is wider; the
+    // others wait for it (a chain of 4096 cliques of 12, on the 128 members that its
+    // entries give it: 75 ms a BFS, now 29)
+    const bool solo = tm.size > 1 && mcur <= kNarrow;
+    Team w = tm;
+    w.size = solo ? 1 : tm.size;  // (member 0 keeps its rank)
+    int nnext = 0;
+    unsigned long long mnext = 0ull;
+    if (solo && tm.rank != 0) {
+      if (!team_sync(tm)) return false;
+      lvl = static_cast<int>(ld_relaxed(&tm.gs->flag[0]));
+      nnext = static_cast<int>(ld_relaxed(&qn[lvl & 3]));
+      mnext = ld_relaxed(&mf[lvl & 3]);
+    } else if (!bfs_level(T, w, lvl, nitems, all, ncur, mcur, &nnext, &mnext, s_acc, s_next, s_mf)) {
+      return false;
+    } else if (solo && (nnext == 0 || mnext > kNarrow)) {
+      if (threadIdx.x == 0) st_relaxed(&tm.gs->flag[0], static_cast<unsigned>(lvl));
+      if (!team_sync(tm)) return false;
     }
-    bq_reset(s_next);
-    bs_reset(s_mf);
-    unsigned long long dsum = 0ull;  // degrees of what this lane appends
-    auto append = [&](bool first, int u) {
-      if (first) dsum += static_cast<unsigned>(T.nindex[u + 1] - T.nindex[u]);
-      bq_append(s_next, first, u, qnext, ncount);
-    };
-    if (mcur * 14ull < static_cast<unsigned long long>(T.edges)) {
-      // push from the frontier queue
-      const int nq = (ncur + kWave - 1) / kWave;
-      auto push = [&](const unsigned long long (&m)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
-        unsigned long long add[kFly];
-        bool first[kFly];
-#pragma unroll
-        for (int q = 0; q < kFly; q++) add[q] = on[q] ? m[q] & ~ld_relaxed(&seen[u[q]]) : 0ull;
-#pragma unroll
-        for (int q = 0; q < kFly; q++)
-          first[q] = add[q] != 0ull && __hip_atomic_fetch_or(&nxt[u[q]], add[q], __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT) == 0ull;
-#pragma unroll
-        for (int q = 0; q < kFly; q++) append(first[q], u[q]);
-      };
-      for (int c = ch.first; c < nq; c += ch.step) {
-        const int k = c * kWave + lane;
-        const bool act = k < ncur;
-        const int v = act ? ld_relaxed(&qcur[k]) : 0;
-        const unsigned long long m = act ? ld_relaxed(&cur[v]) : 0ull;
-        wave_neighbours_of(v, act, T, [&](const int (&o)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
-          unsigned long long om[kFly];
-#pragma unroll
-          for (int q = 0; q < kFly; q++) om[q] = __shfl(m, o[q], kWave);
-          push(om, u, on);
-        });
-      }
-      for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
-        const unsigned long long m = ld_relaxed(&cur[v]);
-        if (m == 0ull) return;
-        item_neighbours(eb, ee, T, [&](const int (&)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
-          unsigned long long om[kFly];
-#pragma unroll
-          for (int q = 0; q < kFly; q++) om[q] = m;
-          push(om, u, on);
-        });
-      });
-    } else {
-      // pull: every vertex with sources still missing
-      for (int c = ch.first; c < ch.count; c += ch.step) {
-        const int v = c * kWave + lane;
-        const unsigned long long sv = v < V ? ld_relaxed(&seen[v]) : all;
-        const unsigned long long missing = all & ~sv;
-        s_acc[wid][lane] = 0ull;
-        wave_lds_sync();
-        wave_neighbours_of(v, missing != 0ull, T, [&](const int (&o)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
-          unsigned long long m[kFly];
-#pragma unroll
-          for (int q = 0; q < kFly; q++) m[q] = on[q] ? ld_relaxed(&cur[u[q]]) : 0ull;
-#pragma unroll
-          for (int q = 0; q < kFly; q++)
-            if (m[q] != 0ull) atomicOr(&s_acc[wid][o[q]], m[q]);
-        });
-        wave_lds_sync();
-        const unsigned long long nb = s_acc[wid][lane] & missing;
-        if (nb != 0ull) st_relaxed(&nxt[v], nb);
-        append(nb != 0ull, v);
-      }
-      for_items(T, tm, nitems, [&](int v, int eb, int ee, int) {
-        const unsigned long long missing = all & ~ld_relaxed(&seen[v]);
-        if (missing == 0ull) return;
-        unsigned long long acc = 0ull;
-        item_neighbours(eb, ee, T, [&](const int (&)[kFly], const int (&u)[kFly], const bool (&on)[kFly]) {
-          unsigned long long m[kFly];
-#pragma unroll
-          for (int q = 0; q < kFly; q++) m[q] = on[q] ? ld_relaxed(&cur[u[q]]) : 0ull;
-#pragma unroll
-          for (int q = 0; q < kFly; q++) acc |= m[q];
-        });
-        const unsigned long long nb = wave_or(acc) & missing;
-        bool first = false;
-        if (nb != 0ull && lane == 0)
-          first = __hip_atomic_fetch_or(&nxt[v], nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0ull;
-        append(first, v);
-      });
-    }
-    bs_add(s_mf, dsum);
-    bs_flush(s_mf, nmf);
-    bq_flush(s_next, qnext, ncount);
-    if (!team_sync(tm)) return false;
-    // the new frontier: masks, seen bits and levels; the old frontier's masks
-    // are cleared (that buffer holds the next level's frontier)
-    const int nnext = static_cast<int>(ld_relaxed(ncount));
-    for (int k = tm.rank * kBatchBlock + static_cast<int>(threadIdx.x); k < ncur; k += tm.size * kBatchBlock)
-      st_relaxed(&fr[(lvl - 1) & 1][ld_relaxed(&qcur[k])], 0ull);
-    for (int c = ch.first; c * kWave < nnext; c += ch.step) {
-      const int k = c * kWave + lane;
-      const int u = k < nnext ? ld_relaxed(&qnext[k]) : 0;
-      unsigned long long nb = 0ull;
-      if (k < nnext) {
-        const unsigned long long sv = ld_relaxed(&seen[u]);
-        nb = ld_relaxed(&nxt[u]) & ~sv;
-        st_relaxed(&nxt[u], 0ull);
-        st_relaxed(&seen[u], sv | nb);
-        st_relaxed(&nfr[u], nb);
-      }
-      write_rows(T, nb, u, lvl);
-    }
-    if (!team_sync(tm)) return false;
     if (nnext == 0) break;
+    ncur = nnext;
+    mcur = mnext;
   }
   for (int c = ch.first; c < ch.count; c += ch.step) {
     const int v = c * kWave + lane;
@@ -572,6 +652,7 @@ struct SsspRows {
   int* row;        // [V << shift]
   unsigned* mask;  // [V] sources active in the next round
   int shift;
+  bool direct;  // narrow round: appends go straight to the queue
   int* qnext;
   unsigned* ncount;
 };
@@ -694,7 +775,8 @@ IG_DEV void relax_lists(const BatchTask& T, const SsspRows& R, int v, int beg, i
     // this round's is)
     const bool first = gain != 0u && __hip_atomic_fetch_or(&R.mask[mine.x], gain, __ATOMIC_RELAXED,
                                                            __HIP_MEMORY_SCOPE_AGENT) == 0u;
-    bq_append(s_next, first, mine.x, R.qnext, R.ncount);
+    if (R.direct) wave_append(first, mine.x, R.qnext, R.ncount);
+    else bq_append(s_next, first, mine.x, R.qnext, R.ncount);
   }
 }
 
@@ -715,7 +797,8 @@ IG_DEV bool sssp_round(const BatchTask& T, const Team& w, SsspRows& R, unsigned*
   R.qnext = queue[(r + 1) & 1];
   R.ncount = &qn[(r + 1) & 3];
   if (w.rank == 0 && threadIdx.x == 0) st_relaxed(&qn[(r + 2) & 3], 0u);
-  bq_reset(s_next);
+  R.direct = ncur <= kWave;  // (as a BFS's narrow levels)
+  if (!R.direct) bq_reset(s_next);
   // few queued vertices: fewer per wave
   int per = kWave;
   while (per > 4 && ncur <= per / 2 * ch.step) per /= 2;
@@ -749,7 +832,7 @@ IG_DEV bool sssp_round(const BatchTask& T, const Team& w, SsspRows& R, unsigned*
     }
     relax_lists(T, R, v, beg, len, m, B, s_next);
   }
-  bq_flush(s_next, R.qnext, R.ncount);
+  if (!R.direct) bq_flush<false>(s_next, R.qnext, R.ncount);
   if (!team_sync(w)) return false;
   *count = static_cast<int>(ld_relaxed(R.ncount));
   return true;
@@ -802,9 +885,30 @@ IG_DEV bool sssp_pass(const BatchTask& T, const Team& tm, int s0, int n, int* ni
   }
   if (!team_sync(tm)) return false;
   int ncur = static_cast<int>(ld_relaxed(&qn[0]));
+  bool solo = false;
   for (int r = 0;; r++) {
+    // narrow rounds are member 0's, as a BFS's narrow levels (unless lists are split); here all
+    // meet before it goes ahead, having read the count
+    if (!solo && tm.size > 1 && *nitems == 0 && ncur <= kNarrowQueue) {
+      solo = true;
+      if (!team_sync(tm)) return false;
+    }
     int count = 0;
-    if (!sssp_round(T, tm, R, base, r, *nitems, ncur, &count, B, s_next)) return false;
+    if (solo && tm.rank != 0) {
+      if (!team_sync(tm)) return false;
+      solo = false;
+      r = static_cast<int>(ld_relaxed(&tm.gs->flag[0]));
+      count = static_cast<int>(ld_relaxed(&qn[(r + 1) & 3]));
+    } else {
+      Team w = tm;
+      w.size = solo ? 1 : tm.size;
+      if (!sssp_round(T, w, R, base, r, *nitems, ncur, &count, B, s_next)) return false;
+      if (solo && (count == 0 || count > 4 * kNarrowQueue)) {
+        if (threadIdx.x == 0) st_relaxed(&tm.gs->flag[0], static_cast<unsigned>(r));
+        if (!team_sync(tm)) return false;
+        solo = false;
+      }
+    }
     if (count == 0) break;
     ncur = count;
   }

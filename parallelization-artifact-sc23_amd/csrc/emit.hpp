@@ -61,16 +61,19 @@ IG_DEV void bq_append(BlockQueue<kCap>& B, bool pred, int item, int* gq, C* gcou
 }
 
 // Workgroup-collective: reserves this workgroup's range with one atomic and
-// copies the buffered items out.
-template <int kCap, typename C>
+// copies the buffered items out.  kClosed: ends with a barrier, after which B may be
+// reset; without, the caller's next barrier has to come first.
+template <bool kClosed = true, int kCap, typename C>
 IG_DEV void bq_flush(BlockQueue<kCap>& B, int* gq, C* gcount)
 {
   __syncthreads();
   const int n = B.count < kCap ? B.count : kCap;
-  if (threadIdx.x == 0 && n > 0) B.base = static_cast<int>(atomic_add_relaxed(gcount, static_cast<C>(n)));
-  __syncthreads();
-  for (int i = threadIdx.x; i < n; i += blockDim.x) st_relaxed(&gq[B.base + i], B.buf[i]);
-  __syncthreads();
+  if (n > 0) {
+    if (threadIdx.x == 0) B.base = static_cast<int>(atomic_add_relaxed(gcount, static_cast<C>(n)));
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += blockDim.x) st_relaxed(&gq[B.base + i], B.buf[i]);
+  }
+  if (kClosed) __syncthreads();
 }
 
 // Workgroup-level 64-bit sum flushed with one atomic.
