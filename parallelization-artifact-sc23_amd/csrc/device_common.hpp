@@ -286,6 +286,17 @@ IG_DEV bool kernel_aborted(GridBarrier* gb, long long deadline)
   return false;
 }
 
+// Thread 0 of workgroup 0, while `outside` of group 0's workgroups (those b with b % 8 == 0)
+// and all of the other groups' are on their way to a grid barrier that the rest have yet
+// to enter: waits until they have arrived there, so that what they read before is free to
+// change, or until the kernel must stop.
+IG_DEV void wait_arrived(GridBarrier* gb, unsigned outside, long long deadline)
+{
+  const unsigned groups = gridDim.x < 8u ? gridDim.x : 8u;
+  while (ld_relaxed(&gb->top.v) != groups - 1u || ld_relaxed(&gb->group[0].v) != outside)
+    if (kernel_aborted(gb, deadline)) return;
+}
+
 // MIS priority: the suite's integer hash (include/mis_vertex_cuda.h:174-179,
 // xor-shift-multiply by 0x45d9f3b twice) of v + 712313887 (init kernels, e.g.
 // MIS_CUDA_V_Topo_Push_Determ_IntType_NonPersist_Atomic_Thread.cu:51).

@@ -36,6 +36,7 @@
 // delta defaults to a sampled mean weight x 32 / mean degree (at least 1).
 #include "sssp.hpp"
 
+#include "far_piles.hpp"
 #include "frontier.hpp"
 #include "team.hpp"
 #include "trace.hpp"
@@ -194,7 +195,7 @@ IG_DEV void team_park(const SsspArgs& a, SsspControl* ctl, SsspTeamLds& S, const
   for (int q = 0; q < kFly; q++) {
     if (park[q]) {
       if (slot < kFarCap) S.far[p][slot] = u[q];
-      else st_relaxed(&a.far[epoch % 3][atomic_add_relaxed(&ctl->far_cnt[epoch % 3].v, 1u)], u[q]);
+      else st_relaxed(&a.far[pile_of(epoch)][atomic_add_relaxed(&ctl->far_cnt[pile_of(epoch)].v, 1u)], u[q]);
       slot++;
     }
   }
@@ -224,6 +225,7 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
                       const FrontierQueues& in, const FrontierQueues& out, FrontierCounters* oc, SsspControl* ctl,
                       long long deadline, unsigned* last, SsspTeamLds& S)
 {
+  const int entry = epoch;  // (what others may still read, see split_waits)
   constexpr int kFly = 2;  // entries in flight per lane (3 and 4 spilled: 1024^2 road 8.9 ms a call, 9.3 and 11.9)
   const int t = static_cast<int>(threadIdx.x);
   TeamShare<kShareCap>& F = S.share;
@@ -249,9 +251,9 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
     if (sum.total == 0u) {
       // near frontier empty: move the split and re-file the far piles
       const int p = epoch & 1;
-      const int* gfar = a.far[epoch % 3];
-      const unsigned ng = ld_relaxed(&ctl->far_cnt[epoch % 3].v);
-      unsigned least = min(S.far_min[p], ld_relaxed(&ctl->far_min[epoch % 3].v));
+      const int* gfar = a.far[pile_of(epoch)];
+      const unsigned ng = ld_relaxed(&ctl->far_cnt[pile_of(epoch)].v);
+      unsigned least = min(S.far_min[p], ld_relaxed(&ctl->far_min[pile_of(epoch)].v));
       if (!team_min(&ctl->team, tm, static_cast<unsigned>(it) + 1u, least, &ctl->bar, deadline, F, &least)) return false;
       if (least >= static_cast<unsigned>(kInf) || ng > static_cast<unsigned>(tm.size * kFarCap)) break;
       trace_level(&ctl->trace, it, ng + S.nfar[p], 0ull, 3);
@@ -266,9 +268,9 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
         S.nfar[p ^ 1] = 0;
         S.far_min[p ^ 1] = static_cast<unsigned>(kInf);
         if (tm.rank == 0) {
-          // the pile two epochs on was consumed by the previous split
-          st_relaxed(&ctl->far_cnt[(epoch + 1) % 3].v, 0u);
-          st_relaxed(&ctl->far_min[(epoch + 1) % 3].v, static_cast<unsigned>(kInf));
+          if (split_waits(entry, epoch - 1)) wait_others(&ctl->bar, tm, deadline);
+          st_relaxed(&ctl->far_cnt[pile_cleared(epoch - 1)].v, 0u);
+          st_relaxed(&ctl->far_min[pile_cleared(epoch - 1)].v, static_cast<unsigned>(kInf));
           ctl->epochs++;
         }
       }
@@ -361,11 +363,11 @@ IG_DEV bool team_near(const SsspArgs& a, int& it, unsigned n, const Team& tm, in
   const int own = min(S.nfar[epoch & 1], kFarCap);
   __syncthreads();
   if (t == 0 && own > 0) {
-    S.nfar[0] = static_cast<int>(atomic_add_relaxed(&ctl->far_cnt[epoch % 3].v, static_cast<unsigned>(own)));
-    atomic_min_relaxed(&ctl->far_min[epoch % 3].v, S.far_min[epoch & 1]);
+    S.nfar[0] = static_cast<int>(atomic_add_relaxed(&ctl->far_cnt[pile_of(epoch)].v, static_cast<unsigned>(own)));
+    atomic_min_relaxed(&ctl->far_min[pile_of(epoch)].v, S.far_min[epoch & 1]);
   }
   __syncthreads();
-  for (int i = t; i < own; i += kSsspBlock) st_relaxed(&a.far[epoch % 3][S.nfar[0] + i], S.far[epoch & 1][i]);
+  for (int i = t; i < own; i += kSsspBlock) st_relaxed(&a.far[pile_of(epoch)][S.nfar[0] + i], S.far[epoch & 1][i]);
   for (int base = 0; base < cn; base += kSsspBlock) {
     const int i = base + t;
     const int d = i < cn ? F.deg[it & 1][i] : 0;
@@ -445,7 +447,7 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
   }
   const int delta = ld_relaxed(&ctl->delta);
   int T = delta;  // split: near holds distances < T
-  int epoch = 1;  // far pile generation (farstamp value); far[epoch % 3] is current
+  int epoch = 1;  // far pile generation (farstamp value); far[pile_of(epoch)] is current
   int it = 0;     // near iterations and splits (stamp values start at 1)
   int R = 0;      // pass: counters rotate and queues alternate by it
   int declined = -1;           // iteration that a team has left to the grid
@@ -460,9 +462,9 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
     const FrontierQueues& in = a.fq[R & 1];
     const FrontierQueues& out = a.fq[(R + 1) & 1];
     if (tid == 0) counters_clear(&ctl->cnt[(R + 2) % 3]);
-    int* far = a.far[epoch % 3];
-    unsigned* far_cnt = &ctl->far_cnt[epoch % 3].v;
-    unsigned* far_min = &ctl->far_min[epoch % 3].v;
+    int* far = a.far[pile_of(epoch)];
+    unsigned* far_cnt = &ctl->far_cnt[pile_of(epoch)].v;
+    unsigned* far_min = &ctl->far_min[pile_of(epoch)].v;
     const bool split = static_cast<unsigned long long>(n) + nm + nh == 0;
     const unsigned long long m = ld_relaxed(&ic->m);
     const unsigned nfar = split ? ld_relaxed(far_cnt) : 0u;
@@ -518,13 +520,13 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
       T = Tn > kInf ? kInf : static_cast<int>(Tn);
       it++;
       const int nepoch = epoch + 1;
-      int* nfar = a.far[nepoch % 3];
-      unsigned* nfar_cnt = &ctl->far_cnt[nepoch % 3].v;
-      unsigned* nfar_min = &ctl->far_min[nepoch % 3].v;
+      int* nfar = a.far[pile_of(nepoch)];
+      unsigned* nfar_cnt = &ctl->far_cnt[pile_of(nepoch)].v;
+      unsigned* nfar_min = &ctl->far_min[pile_of(nepoch)].v;
       if (tid == 0) {
-        // pile (epoch + 2) % 3 was consumed by the previous split, one barrier ago
-        st_relaxed(&ctl->far_cnt[(epoch + 2) % 3].v, 0u);
-        st_relaxed(&ctl->far_min[(epoch + 2) % 3].v, static_cast<unsigned>(kInf));
+        // (consumed by the previous split, one barrier ago)
+        st_relaxed(&ctl->far_cnt[pile_cleared(epoch)].v, 0u);
+        st_relaxed(&ctl->far_min[pile_cleared(epoch)].v, static_cast<unsigned>(kInf));
       }
       se_reset(s_emit);
       for (unsigned base = blockIdx.x * blockDim.x; base < nf; base += stride) {

@@ -49,6 +49,14 @@ IG_DEV int team_limit()
   return per < 1 ? 1 : (per < kTeamMax ? per : kTeamMax);
 }
 
+// Rank 0's thread 0: waits until every workgroup outside the team has arrived at the
+// barrier that ends the pass (the members' all have b % 8 == 0).  Waits no longer once the
+// kernel must stop, which the phase's own look finds within 64 turns.
+IG_DEV void wait_others(GridBarrier* gb, const Team& tm, long long deadline)
+{
+  wait_arrived(gb, ((gridDim.x + 7u) >> 3) - static_cast<unsigned>(tm.size), deadline);
+}
+
 // What an exchange tells: over all members the entries (sum, maximum) and the
 // vertices, and the vertices of lower ranks.
 struct TeamSum {
