@@ -29,6 +29,7 @@
 // neighbours get their level but never enter a frontier.
 #include "bfs.hpp"
 
+#include "by_pass.hpp"
 #include "frontier.hpp"
 #include "team.hpp"
 #include "trace.hpp"
@@ -54,6 +55,11 @@ constexpr unsigned kShareEntries = 1024;
 // the next share.
 IG_DEV unsigned team_share(int size) { return size == 1 ? kSoloEntries : static_cast<unsigned>(kSmallCap); }
 
+struct BfsBase {
+  int level;
+  unsigned last_m;
+};
+
 struct BfsControl {
   GridBarrier bar;
   TeamSlots team;
@@ -63,9 +69,9 @@ struct BfsControl {
   int bottom_up_levels;
   int small_levels;
   int status;
-  int level_base;   // level at which the grid resumes after a team phase
-  unsigned last_m;  // degree sum of the level before it
-  int pad[26];
+  // where the grid resumes after a team phase: level, degree sum of the level before it
+  ByPass<BfsBase> base;
+  int pad[24];
   LevelTrace trace;
 };
 
@@ -331,8 +337,8 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
           return;
         }
         if (tm.rank == 0 && threadIdx.x == 0) {
-          st_relaxed(&ctl->level_base, L2);
-          st_relaxed(&ctl->last_m, last);
+          st_relaxed(&ctl->base.of(R).level, L2);
+          st_relaxed(&ctl->base.of(R).last_m, last);
           ctl->small_levels += L2 - L;
         }
       }
@@ -340,12 +346,12 @@ __global__ __launch_bounds__(kBfsBlock) __attribute__((amdgpu_waves_per_eu(6, 8)
         if (tid == 0) ctl->status = 1;
         return;
       }
-      const int L2 = ld_relaxed(&ctl->level_base);
+      const int L2 = ld_relaxed(&ctl->base.of(R).level);
       if (L2 == L) {  // an uneven frontier: this level goes to the grid
         declined = L;
         continue;
       }
-      prev = ld_relaxed(&ctl->last_m);
+      prev = ld_relaxed(&ctl->base.of(R).last_m);
       L = L2;
       R++;
       continue;

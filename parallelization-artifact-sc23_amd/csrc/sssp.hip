@@ -36,6 +36,7 @@
 // delta defaults to a sampled mean weight x 32 / mean degree (at least 1).
 #include "sssp.hpp"
 
+#include "by_pass.hpp"
 #include "far_piles.hpp"
 #include "frontier.hpp"
 #include "team.hpp"
@@ -54,6 +55,11 @@ constexpr int kFarCap = 2048;
 constexpr unsigned kSoloEntries = 1024;
 constexpr unsigned kShareEntries = 512;
 
+struct SsspBase {
+  int it, split, epoch;
+  unsigned last_m;
+};
+
 struct SsspControl {
   GridBarrier bar;
   TeamSlots team;
@@ -67,11 +73,8 @@ struct SsspControl {
   int small_iters;  // iterations (near and split) run by teams
   // where the grid resumes after a team phase: iteration (stamp) count, split
   // T, far-pile epoch, degree sum of the frontier before the one handed over
-  int it_base;
-  int split_base;
-  int epoch_base;
-  unsigned last_m;
-  int pad[23];
+  ByPass<SsspBase> base;
+  int pad[19];
   LevelTrace trace;
 };
 
@@ -488,10 +491,10 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
         // to the whole workgroup; a return here spilled 42 registers instead of 15)
         const bool ok = team_near(a, it2, n, tm, T2, epoch2, delta, in, out, oc, ctl, deadline, &last, s_lds.small);
         if (ok && tm.rank == 0 && threadIdx.x == 0) {
-          st_relaxed(&ctl->it_base, it2);
-          st_relaxed(&ctl->split_base, T2);
-          st_relaxed(&ctl->epoch_base, epoch2);
-          st_relaxed(&ctl->last_m, last);
+          st_relaxed(&ctl->base.of(R).it, it2);
+          st_relaxed(&ctl->base.of(R).split, T2);
+          st_relaxed(&ctl->base.of(R).epoch, epoch2);
+          st_relaxed(&ctl->base.of(R).last_m, last);
           ctl->small_iters += it2 - it;
         }
       }
@@ -499,15 +502,15 @@ __global__ __launch_bounds__(kSsspBlock) __attribute__((amdgpu_waves_per_eu(6, 8
         if (tid == 0) ctl->status = 1;
         return;
       }
-      const int it2 = ld_relaxed(&ctl->it_base);
+      const int it2 = ld_relaxed(&ctl->base.of(R).it);
       if (it2 == it) {  // an uneven frontier: this pass goes to the grid
         declined = it;
         continue;
       }
       it = it2;
-      T = ld_relaxed(&ctl->split_base);
-      epoch = ld_relaxed(&ctl->epoch_base);
-      prev = ld_relaxed(&ctl->last_m);
+      T = ld_relaxed(&ctl->base.of(R).split);
+      epoch = ld_relaxed(&ctl->base.of(R).epoch);
+      prev = ld_relaxed(&ctl->base.of(R).last_m);
       R++;
       continue;
     }
