@@ -14,8 +14,8 @@
 // that would finish last take them (widen_gangs).  The cap depends on how much
 // work a barrier separates: 256 for the dense sweeps of PR, CC and MIS, 128 for
 // BFS, 64 for SSSP's many short rounds (256 of idle workgroups), and 16 for BFS
-// on deep sparse graphs (average degree below 6), whose thousands of levels are
-// bound by barrier latency.  A free workgroup joins the first task in queue
+// on sparse graphs (average degree below 6), which may have thousands of
+// levels, each bound by barrier latency.  A free workgroup joins the first task in queue
 // order that still has a free slot (one atomic on the task's `joined`
 // counter); the gang starts when all k members have arrived.  Because every
 // workgroup is resident and gangs are filled strictly in queue order, a gang
@@ -47,11 +47,15 @@
 //         vertex queues it.  Otherwise it pulls: every vertex with sources
 //         still missing ORs its neighbours' frontier masks.  A second phase
 //         turns the next masks into the new frontier and writes the level
-//         into the slab rows of the new bits.  Deep graphs (grids, roads)
-//         cost their edge work plus two barriers per level.
+//         into the slab rows of the new bits.  A level costs its edge work plus
+//         two barriers: the gang's, or the workgroup's for levels of at most kNarrow
+//         entries, which member 0 runs alone.
 //   SSSP: Bellman-Ford driven by a queue of active vertices over vertex-major
-//         rows of distances; relaxations by atomicMin, a vertex is queued for
-//         the next round when its distance for some source drops.
+//         rows of distances, with a mask of the sources that are active at a vertex;
+//         lists are taken in blocks of 64 entries, whose (entry, source) pairs are
+//         relaxed by atomicMin, and a vertex is queued for the next round when its
+//         distance for some source drops.  Sources go through in passes where
+//         their rows do not fit the memory.  Narrow rounds are member 0's, too.
 //   CC  : union-find hooking the larger root under the smaller (labels =
 //         component minima), then flattening; graphs of average degree 8 or
 //         more link in Afforest order and skip the giant component's lists.
@@ -371,7 +375,7 @@ IG_DEV void item_neighbours(int eb, int ee, const BatchTask& T, F&& f)
 IG_DEV void write_rows(const BatchTask& T, unsigned long long m, int v, int level)
 {
   // ... and few sources per vertex each lane its own: a path's frontier of 128 vertices for
-  // 64 64 sources cost a BFS 64 turns of the wave a level (10.5 -> 7.8 us).
+  // 64 sources cost a BFS 64 turns of the wave a level (10.5 -> 7.8 us).
   unsigned long long rows = wave_or(m);
   const int bits = wave_bcast(wave_inclusive_scan(__popcll(m)), kWave - 1);
   if (4 * bits >= kWave * __popcll(rows)) {
@@ -1363,7 +1367,8 @@ namespace {
 int gang_for(int alg, int nodes, int edges, int grid) { return std::min(batch_gang(alg, nodes, edges), std::max(1, grid)); }
 
 // Estimated nanoseconds of one query on one workgroup, fitted to batches of
-// one query on graphs of 2^10 to 2^18 entries.
+// one query on graphs of 2^10 to 2^18 entries (and not again since BFS, SSSP, PR and,
+// most of all, MIS became faster).
 double query_cost(const indigo_query& Q, const indigo_graph_ref& G)
 {
   const double entries = static_cast<double>(G.edges) + G.nodes;
@@ -1397,8 +1402,8 @@ long long widen_floor(const indigo_query& Q, const indigo_graph_ref& G)
 // With gangs of 2^18 entries per member alone, a batch was as long as its
 // largest task on a workgroup or two (SSSP of 16 sources on 10^5 vertices: 20
 // to 30 ms) while most of the grid idled.  Batches of 24, 12, 6 and 2 graphs of
-// 2^10 to 2^17 vertices, five algorithms each: 52.6, 69.5, 27.6 and 22.9 ->
-// 15.2, 11.8, 10.8 and 5.0 ms; floors of 1024 and 2048 entries per member
+// 2^10 to 2^17 vertices, five algorithms each (at the time of that step): 52.6, 69.5,
+// 27.6 and 22.9 -> 15.2, 11.8, 10.8 and 5.0 ms; floors of 1024 and 2048 entries per member
 // measured the same within 12%, 16384 up to 23% slower.
 void widen_gangs(std::vector<int>& gang, const indigo_graph_ref* graphs, const indigo_query* queries, int grid)
 {

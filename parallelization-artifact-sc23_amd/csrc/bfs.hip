@@ -15,7 +15,7 @@
 // Each level is either
 //   * top-down: the degree-binned frontier of frontier.hpp (small lists by
 //     64-lane waves with the in-wave balancer, mid lists one wave each, huge
-//     lists in 2048-entry chunks over all workgroups); a neighbour is claimed
+//     lists in 512-entry items of one wave each); a neighbour is claimed
 //     with one CAS INT_MAX -> L+1, so each vertex joins the next frontier
 //     exactly once; or
 //   * bottom-up: every unvisited vertex looks for a parent with dist == L and

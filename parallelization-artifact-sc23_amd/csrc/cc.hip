@@ -21,7 +21,7 @@
 //                binned into mid / huge queues, appends aggregated per
 //                workgroup); vertices in c's tree skip their lists;
 //   6. heavy:    mid lists one wave each, huge lists in kHugeChunk-entry
-//                items, one workgroup each;
+//                items, one wave each;
 //   7. flatten:  label[v] = root(v).
 // Graphs with an average degree below kAfforestDeg skip steps 2-4 and link
 // every undirected edge once, from its larger endpoint.

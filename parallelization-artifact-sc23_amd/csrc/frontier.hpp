@@ -19,8 +19,8 @@
 // of up to 4095 entries on one wave (and longer ones in 2048-entry workgroup
 // items), the longest list set an iteration: SSSP on R-MAT 22, 20, 18 and 16
 // took 4.95, 2.11, 0.91 and 0.66 ms, now 4.09, 1.43, 0.76 and 0.50.
-// Appends are wave-aggregated (ballot + mbcnt prefix, one atomic per wave and
-// queue).  Counters are triple-buffered across levels so that the set written
+// Appends are aggregated by wave (ballot + mbcnt prefix, one atomic per wave and
+// queue) or, in the passes of the whole grid, by workgroup (emit.hpp).  Counters are triple-buffered across levels so that the set written
 // in level L, read in L+1 and cleared in L+2 never has two roles at once.
 //
 // The same machinery bins a static vertex set: collect_heavy() appends every

@@ -7,13 +7,13 @@
 // L1 change of the iteration is > 1e-4 and fewer than 100 iterations ran.
 //
 // Design: one persistent kernel; per iteration
-//   vertices with short lists (< kPrWaveDeg entries) are taken 64 to a wave in
-//   vertex order (coalesced score / contrib / index traffic), one lane or one
+//   vertices with short lists (< kPrWaveDeg entries) are taken 64 to a wave (fewer
+//   on graphs that would leave waves idle) in vertex order (coalesced score / contrib / index traffic), one lane or one
 //   group of lanes to a list;
 //   longer lists, collected once into a static list, one wave each; lists of
 //   kPrHugeDeg or more in kPrHugeChunk-entry items, one wave each, whose
 //   partial sums go to a per-item slot; the wave that finishes a huge
-//   vertex's last item (a counter per vertex) combines its item partials in
+//   vertex's last item (a counter per vertex, and per 32 items) combines its item partials in
 //   item order, so no second barrier is needed;
 // then one barrier and the stop test.  Per-vertex sums are FP32 with Neumaier
 // compensation (the improved Kahan-Babuska sum: a running error term added
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
       if (lane == 0) d += finish_vertex(a, v, old, acc.value(), base, cout);
     }
     trace_level(&ctl->trace, tl + 2, static_cast<unsigned>(it), 0ull, 2);
-    // phase A: short lists, 64 vertices a wave, vertex order
+    // phase A: short lists, `per` vertices a wave, vertex order
     for (int c0 = 0, at = wave; c0 < chunks; c0 += nwaves, at = next_turn(at)) {
       const int c = c0 + at;
       const int v = c * per + lane;

@@ -10,11 +10,10 @@
 // the queue takes the slot alone (its kernels are ordinary launches), and so
 // does a BFS or SSSP request on a deep, sparse graph (average degree below
 // 6, at least 65536 vertices: grids, road networks), on the single-query
-// kernels: their team phase runs the thousands of narrow levels at
-// workgroup-barrier cost (the batched engine's gangs pay a device barrier
-// per level: 82 ms against about 45 for a 2048^2 grid's BFS), and the
-// batched Bellman-Ford rounds re-relax such graphs many times over, while
-// near-far settles them in distance order.  The
+// kernels: their team phase runs thousands of levels at the cost of one exchange
+// each (the batched engine's gangs pay device barriers for levels that are
+// not narrow), and the batched Bellman-Ford rounds re-relax such graphs many
+// times over, while near-far settles them in distance order.  The
 // other slots keep running, so requests that arrive while the GPU is busy
 // are admitted as soon as a slot and memory are free, and their work
 // overlaps on the device.  Completion is polled with events; results are
@@ -183,7 +182,7 @@ struct Server {
   // SSSP 3000, CC 50000, MIS 10000, PageRank 1600, TC 2000).  BFS and SSSP
   // on deep sparse graphs run alone on the single-query kernels and are
   // costed by their level count instead (about 2 sqrt(V) levels from a
-  // random source at 10 and 20 us per level).
+  // random source at 10 and 20 us per level, above what they take on the whole GPU).
   double est_us(const indigo_request& r) const
   {
     const indigo_graph_ref& G = graphs[r.graph];

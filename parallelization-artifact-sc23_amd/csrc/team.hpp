@@ -10,7 +10,7 @@
 // round) and the queue reads.  Shares drift apart (on a 2048^2 road one of 32
 // grew to 1929 of 6860 entries within 800 levels, and the level's time with it,
 // 3.4 to 11.5 us), so the members deal the frontier out again when the largest
-// share passes twice the average.
+// share passes half as much again as the average and 64 entries (share_uneven).
 // A team of one is a workgroup alone: its exchange is free.
 #pragma once
 

@@ -21,8 +21,8 @@ analysis_median.ipynb, cell 1, and the file names under codes/cuda/*):
                        the data-driven SSSP worklist
   Thread / Warp / Block
                        the gang size of a batched task (workgroups per task)
-                       and INDIGO_HINT_SMALL_FRONTIER (levels run by one
-                       workgroup while the frontier is small)
+                       and INDIGO_HINT_SMALL_FRONTIER (narrow levels run by
+                       one workgroup or a team of them)
   ThreadsPerBlock      INDIGO_HINT_BLOCK_SIZE: 256, 512 or 1024 threads per
                        workgroup of the edge-centric kernels (the suite's
                        ThreadsPerBlock, include/pr_cuda.h:44)
