@@ -92,7 +92,8 @@ struct PrArgs {
   unsigned* hdone;       // per huge vertex: items (of more than kPrGroupItems, groups of them) finished this sweep
   PaddedU32* gdone;      // per group of items: those finished this sweep
   int ngroups;
-  double* hres;          // per huge vertex: |s' - s| of this sweep
+  double* hres[2];       // per huge vertex: |s' - s| of a sweep, by its parity: whoever
+                         // is late to add them up may see the next sweep's items done
   double* partial;       // [2][2 * kPrMaxGrid] per-workgroup residuals (phase A, phase B)
   int* exit_it;     // [kPrMaxGrid] iteration at which each workgroup left
   double* exit_total;
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
         }
         tot = wave_merge(tot);
         if (lane == 0) {
-          st_relaxed(&a.hres[item.j], finish_vertex(a, v, a.scores[v], tot.value(), base, cout));
+          st_relaxed(&a.hres[it & 1][item.j], finish_vertex(a, v, a.scores[v], tot.value(), base, cout));
           st_relaxed(&a.hdone[item.j], 0u);  // every item of this sweep has counted
         }
       }
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(kPrBlock) void pr_kernel(PrArgs a)
     double part = 0.0;
     for (int b = threadIdx.x; b < static_cast<int>(gridDim.x); b += kPrBlock) part += slots[2 * b];
     double hpart_sum = 0.0;
-    for (int j = threadIdx.x; j < static_cast<int>(nh); j += kPrBlock) hpart_sum += ld_relaxed(&a.hres[j]);
+    for (int j = threadIdx.x; j < static_cast<int>(nh); j += kPrBlock) hpart_sum += ld_relaxed(&a.hres[it & 1][j]);
     const double total = block_sum_f64(part, s_red) + block_sum_f64(hpart_sum, s_red);
     if (!(total > a.eps && it < a.max_iter)) {
       if (tid == 0) {
@@ -451,7 +452,7 @@ size_t pr_workspace_bytes(int nodes, int edges)
   for (int c = 0; c < kPrClasses; c++) mid += Carver::round(pr_class_cap(edges, c) * 4);
   return Carver::round(sizeof(PrControl)) + mid + 5 * Carver::round(v * 4) + Carver::round(pr_max_chunks(edges) * 16) +
          Carver::round(pr_max_chunks(edges) * 8) +
-         Carver::round((static_cast<size_t>(edges) / kPrHugeDeg + 1) * 12) + 256 +
+         Carver::round((static_cast<size_t>(edges) / kPrHugeDeg + 1) * 20) + 512 +
          Carver::round(pr_max_groups(edges) * sizeof(PaddedU32)) +
          Carver::round(4 * kPrMaxGrid * 8) + Carver::round(kPrMaxGrid * 4) + Carver::round(kPrMaxGrid * 8) + 4096;
 }
@@ -481,7 +482,7 @@ int pr_run(indigo_ctx* ctx, int nodes, int edges, const int* nindex, const int* 
   a.hdone = cv.take<unsigned>(static_cast<size_t>(a.hcap));
   a.ngroups = static_cast<int>(pr_max_groups(edges));
   a.gdone = cv.take<PaddedU32>(static_cast<size_t>(a.ngroups));
-  a.hres = cv.take<double>(static_cast<size_t>(a.hcap));
+  for (double*& hres : a.hres) hres = cv.take<double>(static_cast<size_t>(a.hcap));
   a.partial = cv.take<double>(4 * kPrMaxGrid);
   a.exit_it = cv.take<int>(kPrMaxGrid);
   a.exit_total = cv.take<double>(kPrMaxGrid);
